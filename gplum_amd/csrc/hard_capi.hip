@@ -16,8 +16,9 @@ namespace gplum {
 namespace {
 
 struct HardCtx {
-    hipStream_t st = nullptr, st2 = nullptr;
-    hipEvent_t e0 = nullptr, e1 = nullptr, fork = nullptr, join = nullptr;
+    hipStream_t st = nullptr;
+    HardStreams hs;
+    hipEvent_t e0 = nullptr, e1 = nullptr;
     HardBuffers hb;
     DArray<int32_t> off, order;
     // uploaded state kept for graph replays (each replay restores it first)
@@ -36,9 +37,6 @@ struct HardCtx {
         GPLUM_HIP(hipGetDeviceProperties(&prop, dev));
         n_cu = prop.multiProcessorCount;
         GPLUM_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-        GPLUM_HIP(hipStreamCreateWithFlags(&st2, hipStreamNonBlocking));
-        GPLUM_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
-        GPLUM_HIP(hipEventCreateWithFlags(&join, hipEventDisableTiming));
         GPLUM_HIP(hipEventCreate(&e0));
         GPLUM_HIP(hipEventCreate(&e1));
         return GPLUM_OK;
@@ -127,7 +125,7 @@ int hard_upload(HardCtx &c, const gplum_params *p, const gplum_particle *pp, int
     GPLUM_ENSURE(c.order, n_cluster);
     if ((rc = upload(c.off, offs, c.st))) return rc;
     if ((rc = upload(c.order, pl.order, c.st))) return rc;
-    GPLUM_ENSURE(hb.next, 3);
+    GPLUM_ENSURE(hb.next, HERMITE_CLASSES);
     GPLUM_ENSURE(hb.edisp, n_cluster);
     GPLUM_ENSURE(hb.ncol, n_cluster);
     GPLUM_ENSURE(hb.nblock, n_cluster);
@@ -239,7 +237,7 @@ extern "C" int gplum_hard_integrate(const gplum_params *p, gplum_particle *pp, i
         // mode bit 3: clusters of 2 to 4 bodies on the one-lane-per-particle path too
         const int giant_min = (mode & 4) ? HARD_SEQ_MAX : GIANT_MIN_DEFAULT;
         const int terms_max = (mode & 8) ? 0 : TERMS_MAX;
-        if ((rc = hard_launch(*p, c.hb, n_cluster, c.off.p, c.order.p, true, c.n_cu, c.st, c.st2, c.fork, c.join, 8,
+        if ((rc = hard_launch(*p, c.hb, n_cluster, c.off.p, c.order.p, true, c.n_cu, c.st, c.hs, 8,
                               HERMITE_LDS, giant_min, terms_max)))
             return rc;
     } else {
@@ -284,7 +282,8 @@ extern "C" int gplum_hard_integrate_graph(const gplum_params *p, gplum_particle 
     for (const Pair &s : state)
         GPLUM_HIP(hipMemcpyAsync(s.src, s.dst, s.bytes, hipMemcpyDeviceToDevice, c.st));
     GPLUM_HIP(hipStreamSynchronize(c.st));
-    // capture: restore the state, reset the queue, the size-class kernels on two streams
+    // capture: restore the state, reset the queue, the size-class kernels on their streams
+    if ((rc = c.hs.ensure())) return rc;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     GPLUM_HIP(hipStreamBeginCapture(c.st, hipStreamCaptureModeThreadLocal));
@@ -293,7 +292,7 @@ extern "C" int gplum_hard_integrate_graph(const gplum_params *p, gplum_particle 
             rc = fail(GPLUM_E_HIP, "hipMemcpyAsync failed during graph capture");
     // (the whole-GPU path for giant clusters is host-driven and cannot be captured)
     if (!rc)
-        rc = hard_launch(*p, hb, n_cluster, c.off.p, c.order.p, true, c.n_cu, c.st, c.st2, c.fork, c.join, 8,
+        rc = hard_launch(*p, hb, n_cluster, c.off.p, c.order.p, true, c.n_cu, c.st, c.hs, 8,
                          HERMITE_LDS, GIANT_OFF);
     const hipError_t ec = hipStreamEndCapture(c.st, &graph);
     if (rc) { if (graph) (void)hipGraphDestroy(graph); return rc; }

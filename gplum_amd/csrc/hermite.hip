@@ -6,10 +6,10 @@
 // time+dt, predicts every particle, checks collisions (perfect merging), corrects
 // the active particles with two P(EC) iterations and updates their block steps.
 // The active particles of one block step are independent (each reads only the
-// predicted positions of the others), so they are corrected in parallel with one
-// barrier per block step.  The j-data of the cluster (predicted position/velocity,
-// mass, 1/r_out, id) lives in LDS for clusters of up to HERMITE_LDS particles.
-// The kernel is persistent: workgroups pull clusters (costliest first: estimated block
+// predicted positions of the others), so they are corrected in parallel.  Clusters of 2 to
+// 4 bodies hold their state in registers (integrate_terms), those of up to HERMITE_LDS in
+// LDS (hermite_lds.hpp), larger ones in global memory.
+// The kernels are persistent: workgroups pull clusters (costliest first: estimated block
 // steps times size) from an atomic queue until it is empty.
 #include <algorithm>
 #include <cfloat>
@@ -162,6 +162,55 @@ __device__ inline double dt_block(const HP &P, double time, double dt, double ac
     return dt_next;
 }
 
+// Whether d is a power of two (normal, 2^-999 to 2^999): then 1/d, and products with it, are
+// exact.  Every block step is one (dt_tree halved some times).
+__device__ inline bool is_pow2(double d) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(d);
+    const unsigned hi = (unsigned)(b >> 32);
+    return ((unsigned)b | (hi & 0xFFFFFu)) == 0u && hi - (24u << 20) <= (1998u << 20);
+}
+__device__ inline double pow2_inverse(double d) {
+    return __longlong_as_double(0x7FE0000000000000ll - __double_as_longlong(d));
+}
+// recip_block without its frexp and ldexp
+__device__ inline double recip_step(double d) {
+    if (is_pow2(d)) return pow2_inverse(d);
+    return recip_block(d);
+}
+
+// The first part of dt_block: dt_max halved until it divides time (cap: it never did).
+__device__ inline double dt_candidate(double time, double dt_max, bool &cap) {
+    double d = dt_max;
+    if (is_pow2(d) && time >= 0.) {
+        double q = time * pow2_inverse(d);          // exact, so q is whole iff d divides time
+        int it = 0;
+        for (; q != floor(q) && it < HALVE_CAP; it++) { q *= 2.; d *= 0.5; }
+        cap = it == HALVE_CAP;
+    } else {
+        double rem = fmod_block(time, d);
+        for (int it = 0; rem != 0.0 && it < HALVE_CAP; it++) { d *= 0.5; rem = fmod_block(time, d); }
+        cap = rem != 0.0;
+    }
+    return d;
+}
+// Its last part: dt_0 halved while it exceeds both dt_1 and dt / 2 (twice at most when dt_0
+// <= 2 dt).
+__device__ inline double dt_reduce(double dt_0, double dt_1, double dt) {
+    double d = dt_0;
+    if (dt_0 <= 2. * dt) {
+        for (int it = 0; it < 2; it++) d = (dt_1 < d && 0.5 * dt < d) ? 0.5 * d : d;
+    } else {
+        for (int it = 0; dt_1 < d && 0.5 * dt < d && it < HALVE_CAP; it++) d *= 0.5;
+    }
+    return d;
+}
+// clear_of_grid for a power of two d from t's mantissa bits (a slightly narrower range)
+__device__ inline bool clear_of_steps(double t, double d) {
+    if (!is_pow2(d)) return clear_of_grid(t, d);
+    const unsigned hi = (unsigned)((unsigned long long)__double_as_longlong(t) >> 32);
+    return (hi & 0xFFFFFu) - 1025u < 0x100000u - 2049u - 1025u && hi - (24u << 20) <= (1998u << 20);
+}
+
 // ------------------------------------------------------------- hard pair
 
 // gravity_hard.h:219-255: the summands of acc_d, jerk_d (and phi_d) of i from j,
@@ -205,9 +254,20 @@ struct HardView {          // SoA arrays of the gathered cluster particles
     int32_t *flags, *twin_of, *act;     // act: active in the current block step
     // collision records (COLREC doubles each, see perfect_merge), when the caller keeps a
     // collision log: crec null otherwise
-    double *crec = nullptr;
-    unsigned *ccount = nullptr;
-    unsigned ccap = 0;
+    double *crec;
+    unsigned *ccount;
+    unsigned ccap;
+    int base;              // index of the arrays' first element among all clusters' particles
+};
+
+// The clusters of one launch: offsets, processing order (or null), queue and outcomes.
+struct ClusterArgs {
+    const int32_t *off, *order;
+    int ncl, persistent;
+    int *next;
+    double *edisp;
+    int *ncol;
+    long long *nblock, *npair;
 };
 
 __device__ inline void ld3(const double *a, int i, double v[3]) {
@@ -315,33 +375,6 @@ __device__ inline void gravity_loop_lane(const HP &P, const JData &J, int n, int
     }
 }
 
-// Partner j's predicted state (position, velocity, mass, 1/r_out), held in registers
-// for the three force evaluations of a block step.
-struct JReg {
-    double x[3], v[3], m, ri;
-};
-__device__ inline void load_jreg(const JData &J, int j, JReg &r) {
-    for (int d = 0; d < 3; d++) { r.x[d] = J.x[3 * j + d]; r.v[d] = J.v[3 * j + d]; }
-    r.m = J.m[j];
-    r.ri = J.ri[j];
-}
-
-// force_lane_fixed<M> on partner data in registers.
-template <int M>
-__device__ inline void force_jreg(const HP &P, const JReg (&pj)[M], const double xi[3], const double vi[3],
-                                  double rinv_i, double as[3], double js[3], double ad[3], double jd[3]) {
-    double ta[M][3], tj[M][3];
-#pragma unroll
-    for (int k = 0; k < M; k++)
-        pair_term(P, xi, vi, rinv_i, pj[k].x[0], pj[k].x[1], pj[k].x[2], pj[k].v[0], pj[k].v[1], pj[k].v[2],
-                  pj[k].m, pj[k].ri, ta[k], tj[k], nullptr);
-    star_acc_jerk(P, xi, vi, as, js, nullptr);
-    for (int d = 0; d < 3; d++) { ad[d] = 0.; jd[d] = 0.; }
-#pragma unroll
-    for (int k = 0; k < M; k++)
-        for (int d = 0; d < 3; d++) { ad[d] += ta[k][d]; jd[d] += tj[k][d]; }
-}
-
 // calcGravity (full, with phi_d and Sun phi), gravity_hard.h:203-256, current pos/vel.
 __device__ void gravity_full(const HP &P, HardView &H, int b, int n, int i) {
     double x[3], v[3], as[3], js[3], ad[3], jd[3], phs, phd = 0.;
@@ -375,52 +408,6 @@ __device__ inline void predict(HardView &H, int g, double Dt) {
     }
 }
 
-// FPHard::correct, src/particle.h:1208-1274 (position term with ALPHA = 7/6000, as written).
-__device__ inline void correct(HardView &H, int g, double Dt) {
-    const double Dt2 = Dt * Dt;
-    const double Dt_inv = recip_block(Dt);
-    const double Dt_inv2 = Dt_inv * Dt_inv;
-    const double Dt_inv3 = Dt_inv2 * Dt_inv;
-    for (int k = 0; k < 3; k++) {
-        const int q = 3 * g + k;
-        const double Am_s = H.acc_s[q] - H.a0_s[q];
-        const double J0_s = Dt * H.j0_s[q];
-        const double J1_s = Dt * H.jerk_s[q];
-        const double A2_s = 3. * Am_s - (J1_s + 2. * J0_s);
-        const double A3_s = -2. * Am_s + (J1_s + J0_s);
-        H.a2_s[q] = 2. * Dt_inv2 * (A2_s + 3. * A3_s);
-        H.a3_s[q] = 6. * Dt_inv3 * A3_s;
-        const double Am_d = H.acc_d[q] - H.a0_d[q];
-        const double J0_d = H.j0_d[q] * Dt;
-        const double J1_d = H.jerk_d[q] * Dt;
-        const double A2_d = 3. * Am_d - (J1_d + 2. * J0_d);
-        const double A3_d = -2. * Am_d + (J1_d + J0_d);
-        H.a2_d[q] = 2. * (A2_d + 3. * A3_d) * Dt_inv2;
-        H.a3_d[q] = 6. * A3_d * Dt_inv3;
-        const double A2_sd = A2_s + A2_d;
-        const double A3_sd = A3_s + A3_d;
-        H.pos[q] = H.xp[q] + ONE_SIXTIETH * Dt2 * (5. * A2_sd + 3. * ALPHA_POS * A3_sd);
-        H.vel[q] = H.vp[q] + ONE_TWELFTH * Dt * (4. * A2_sd + 3. * A3_sd);
-    }
-}
-
-// Register-resident twins of predict() and correct() (same operation order), for the
-// one-particle-per-lane path of clusters that fit one wave.
-__device__ inline void predict_regs(double Dt, const double pos[3], const double vel[3], const double as[3],
-                                    const double js[3], const double ad[3], const double jd[3], double a0s[3],
-                                    double j0s[3], double a0d[3], double j0d[3], double xp[3], double vp[3]) {
-    for (int k = 0; k < 3; k++) {
-        a0s[k] = as[k];
-        j0s[k] = js[k];
-        j0d[k] = jd[k];
-        a0d[k] = ad[k];
-        const double acc_sd = as[k] + ad[k];
-        const double jerk_sd = js[k] + jd[k];
-        xp[k] = pos[k] + Dt * (vel[k] + Dt * (SECONDORDER * acc_sd + THIRDORDER * Dt * jerk_sd));
-        vp[k] = vel[k] + Dt * (acc_sd + Dt * SECONDORDER * jerk_sd);
-    }
-}
-
 __device__ inline void correct_regs(double Dt, const double xp[3], const double vp[3], const double as[3],
                                     const double a0s[3], const double j0s[3], const double js[3], const double ad[3],
                                     const double a0d[3], const double j0d[3], const double jd[3], double pos[3],
@@ -449,20 +436,6 @@ __device__ inline void correct_regs(double Dt, const double xp[3], const double 
         pos[k] = xp[k] + ONE_SIXTIETH * Dt2 * (5. * A2_sd + 3. * ALPHA_POS * A3_sd);
         vel[k] = vp[k] + ONE_TWELFTH * Dt * (4. * A2_sd + 3. * A3_sd);
     }
-}
-
-// gravity_p / gravity_c of particle g (cluster-local i) against the predicted j-data.
-__device__ inline void gravity_pc(const HP &P, HardView &H, const JData &J, int n, int g,
-                                  bool corrected) {
-    double x[3], v[3], as[3], js[3], ad[3], jd[3];
-    if (corrected) { ld3(H.pos, g, x); ld3(H.vel, g, v); }
-    else { ld3(H.xp, g, x); ld3(H.vp, g, v); }
-    star_acc_jerk(P, x, v, as, js, nullptr);
-    gravity_loop(P, J, n, H.id[g], x, v, H.rinv[g], ad, jd, nullptr);
-    st3(H.acc_s, g, as);
-    st3(H.jerk_s, g, js);
-    st3(H.acc_d, g, ad);
-    st3(H.jerk_d, g, jd);
 }
 
 // Hard force on one particle with all 64 lanes of the (one-wave) workgroup: lane l
@@ -592,7 +565,7 @@ __device__ double perfect_merge(const HP &P, HardView &H, int b, int n, int ic, 
                          dot3(pos_new[0], pos_new[1], pos_new[2], pos_new[0], pos_new[1], pos_new[2]));
             r[18] = sqrt(dot3(dv[0], dv[1], dv[2], dv[0], dv[1], dv[2]) /
                          dot3(vel_g[0], vel_g[1], vel_g[2], vel_g[0], vel_g[1], vel_g[2]));
-            r[COLREC - 1] = (double)b;
+            r[COLREC - 1] = (double)(H.base + b);
         }
     }
     const double mass_rem = mass_imp + mass_tar;
@@ -654,48 +627,6 @@ __device__ double perfect_merge(const HP &P, HardView &H, int b, int n, int ic, 
 
 // --------------------------------------------------------------- kernel
 
-struct Reduce {              // block-level reductions through LDS
-    double d[HERMITE_BIG_BLOCK];
-    int i[HERMITE_BIG_BLOCK];
-    int j[HERMITE_BIG_BLOCK];
-};
-
-__device__ inline double block_min(Reduce &R, double v) {
-    const int t = threadIdx.x;
-    __syncthreads();
-    R.d[t] = v;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if (t < w && R.d[t + w] < R.d[t]) R.d[t] = R.d[t + w];
-        __syncthreads();
-    }
-    const double r = R.d[0];
-    __syncthreads();
-    return r;
-}
-
-// argmin of (R, i) lexicographic, j carried along; returns R, sets *bi, *bj
-__device__ inline double block_argmin(Reduce &R, double v, int i, int j, int *bi, int *bj) {
-    const int t = threadIdx.x;
-    __syncthreads();
-    R.d[t] = v; R.i[t] = i; R.j[t] = j;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if (t < w) {
-            const double a = R.d[t], c = R.d[t + w];
-            if (c < a || (c == a && R.i[t + w] < R.i[t])) {
-                R.d[t] = c; R.i[t] = R.i[t + w]; R.j[t] = R.j[t + w];
-            }
-        }
-        __syncthreads();
-    }
-    const double r = R.d[0];
-    *bi = R.i[0];
-    *bj = R.j[0];
-    __syncthreads();
-    return r;
-}
-
 // Minimum over the 64 lanes of the wave (every lane active; values not NaN): four DPP
 // steps inside each row of 16 lanes, then the four row minima read as scalars.  Far
 // shorter latency than a shuffle butterfly through the LDS crossbar.
@@ -706,23 +637,13 @@ __device__ inline double wave_min(double v) {
     v = dmin(v, dpp_f64<DPP_ROW_MIRROR>(v));
     return dmin(dmin(readlane_f64(v, 0), readlane_f64(v, 16)), dmin(readlane_f64(v, 32), readlane_f64(v, 48)));
 }
-// two minima at once (independent chains)
-__device__ inline void wave_min2(double &u, double &v) {
-    u = dmin(u, dpp_f64<DPP_QUAD_1032>(u)); v = dmin(v, dpp_f64<DPP_QUAD_1032>(v));
-    u = dmin(u, dpp_f64<DPP_QUAD_2301>(u)); v = dmin(v, dpp_f64<DPP_QUAD_2301>(v));
-    u = dmin(u, dpp_f64<DPP_ROW_HALF_MIRROR>(u)); v = dmin(v, dpp_f64<DPP_ROW_HALF_MIRROR>(v));
-    u = dmin(u, dpp_f64<DPP_ROW_MIRROR>(u)); v = dmin(v, dpp_f64<DPP_ROW_MIRROR>(v));
-    u = dmin(dmin(readlane_f64(u, 0), readlane_f64(u, 16)), dmin(readlane_f64(u, 32), readlane_f64(u, 48)));
-    v = dmin(dmin(readlane_f64(v, 0), readlane_f64(v, 16)), dmin(readlane_f64(v, 32), readlane_f64(v, 48)));
+// the minimum over each row of 16 lanes, in every lane of the row
+__device__ inline double row_min(double v) {
+    v = __builtin_fmin(v, dpp_f64<DPP_QUAD_1032>(v));
+    v = __builtin_fmin(v, dpp_f64<DPP_QUAD_2301>(v));
+    v = __builtin_fmin(v, dpp_f64<DPP_ROW_HALF_MIRROR>(v));
+    return __builtin_fmin(v, dpp_f64<DPP_ROW_MIRROR>(v));
 }
-__device__ inline void wave_argmin(double &v, int &i, int &j) {
-    for (int d = 32; d > 0; d >>= 1) {
-        const double ov = __shfl_xor(v, d);
-        const int oi = __shfl_xor(i, d), oj = __shfl_xor(j, d);
-        if (ov < v || (ov == v && oi < i)) { v = ov; i = oi; j = oj; }
-    }
-}
-
 // Orders the wave's own global-memory writes before its later reads (lane 0 writes
 // state that all lanes read back): the wave's memory operations are complete at the
 // fence, and the barrier keeps the compiler from moving accesses across it.
@@ -840,30 +761,14 @@ __device__ void coop_correct_active(const HP &P, HardView &H, const JData &J, in
     }
 }
 
-// ---------------------------- multi-wave kernels: lane groups and wave-level reductions
+// ------------------------------------- multi-wave kernel: workgroup-level reductions
 
-// Per-workgroup scratch of the multi-wave kernels' block steps: one slot per wave for
-// each reduction (separate slots, so that a reduction needs no barrier before its
-// writes), and the list of the block step's active particles.
+// One slot per wave for each reduction (separate slots, so that a reduction needs no
+// barrier before its writes).
 struct WaveSlots {
     double ts[8], sys[8], rm[8];
     int lo[8], hi[8];
-    int na, nm;                // active particles without twins (listed in act), merged targets
-    int act[HERMITE_LDS];
-    int32_t tw[HERMITE_LDS];   // the cluster's twin_of, copied at each block step's prediction
-    // merged targets of the block step, their twins (concatenated, ascending index per
-    // target) and the lane-group layout of the bodies to integrate: slot k holds body
-    // ent[k] (-1: empty), the first slot of its family efam[k] and the family's size
-    // efn[k] (FAM_MERGED set for a merged family; 1 for a body without twins)
-    int mt[HERMITE_LDS];
-    int twl[HERMITE_LDS];
-    int twn[HERMITE_LDS];
-    int ent[2 * HERMITE_LDS], efam[2 * HERMITE_LDS], efn[2 * HERMITE_LDS];
-    int nslot, gs, nfam;       // slots in use, log2 of the lanes per slot, families placed
 };
-constexpr int FAM_MERGED = 1 << 16;
-constexpr int FAM_MAX = 8;     // largest family integrated in the lane groups (64 / 8 lanes)
-constexpr int FAM_GROUPS = 16; // families per block step in the lane groups (slot capacity)
 
 // Minimum over the workgroup (every lane active, values not NaN): the wave's minimum by
 // DPP, the waves' minima through slot[] and one barrier.  Exact, hence the value of
@@ -895,197 +800,6 @@ __device__ inline void block_argmin_waves(double &v, int &lo, int &hi, WaveSlots
     v = W.rm[0]; lo = W.lo[0]; hi = W.hi[0];
     for (int w = 1; w < (int)(blockDim.x >> 6); w++)
         if (rlh_less(W.rm[w], W.lo[w], W.hi[w], v, lo, hi)) { v = W.rm[w]; lo = W.lo[w]; hi = W.hi[w]; }
-}
-
-// Subtree sums of coop_pair_sum's butterfly.  With all 64 lanes on one particle, lane l
-// holds the partial P_l (pairs j = l, l + 64, ... in ascending j) and the xor butterfly
-// 32, 16, ..., 1 adds them: after the level of distance 2^k every lane holds V_k(l mod
-// 2^k), the sum of the partials m = l (mod 2^k), where V_k(r) = V_(k+1)(r) + V_(k+1)(r +
-// 2^k).  A group of S = 2^s lanes holding one particle computes the same sums: lane r of
-// the group builds V_s(r) from its 64/S partials m = r + S bitrev(q), q = 0, 1, ... (the
-// leaves of that subtree from left to right, so that a binary counter over q adds two
-// sibling subtrees as soon as the second one is complete), then the group runs the
-// butterfly's last s levels.  The same additions of the same values as coop_pair_sum,
-// hence the same force bit for bit.  K = ceil(n / 64) pairs per partial, evaluated side
-// by side (partials with fewer pairs evaluate a clamped j and drop it).  Every lane of
-// the wave calls it (groups of invalid particles compute a stand-in); 3 <= s <= 6.
-template <int K>
-__device__ inline void group_pair_sum(const HP &P, const JData &J, int n, int s, int r, int64_t idi,
-                                      const double xi[3], const double vi[3], double rinv_i, double acc[3],
-                                      double jerk[3]) {
-    const int depth = 6 - s;                      // levels of the lane's own subtree
-    const int nq = 1 << depth;
-    double st[3][6];
-    double c[6];
-    for (int q = 0; q < nq; q++) {
-        const int m = r + ((depth ? (int)(__builtin_bitreverse32((unsigned)q) >> (32 - depth)) : 0) << s);
-        for (int d = 0; d < 6; d++) c[d] = 0.;
-#pragma unroll
-        for (int u0 = 0; u0 < K; u0 += 2) {
-            constexpr int L = 2;
-            double ta[L][3], tj[L][3];
-            int jj[L];
-#pragma unroll
-            for (int u = 0; u < L; u++) {
-                jj[u] = min(m + 64 * (u0 + u), n - 1);
-                if (u0 + u < K) pair_term_j(P, J, jj[u], xi, vi, rinv_i, ta[u], tj[u], nullptr);
-            }
-#pragma unroll
-            for (int u = 0; u < L; u++) {
-                if (u0 + u >= K) continue;
-                const bool use = m + 64 * (u0 + u) < n && J.id[jj[u]] != idi;
-                for (int d = 0; d < 3; d++) {
-                    c[d] = use ? c[d] + ta[u][d] : c[d];
-                    c[3 + d] = use ? c[3 + d] + tj[u][d] : c[3 + d];
-                }
-            }
-        }
-        // binary counter: level k holds the left subtree of 2^k leaves until its sibling
-        // is complete
-        bool stored = false;
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            if (stored || k >= depth) continue;
-            if (q & (1 << k)) {
-                for (int d = 0; d < 6; d++) c[d] = st[k][d] + c[d];
-            } else {
-                for (int d = 0; d < 6; d++) st[k][d] = c[d];
-                stored = true;
-            }
-        }
-    }
-    // the last s levels of the butterfly, inside the group (as in coop_pair_sum)
-    if (s == 6)
-        for (int d = 0; d < 6; d++) c[d] += __shfl_xor(c[d], 32);
-    if (s >= 5)
-        for (int d = 0; d < 6; d++) c[d] += __shfl_xor(c[d], 16);
-    if (s >= 4)
-        for (int d = 0; d < 6; d++) c[d] += dpp_f64<DPP_ROW_ROR8>(c[d]);
-    for (int d = 0; d < 6; d++) c[d] += dpp_f64<DPP_QUAD_3210>(dpp_f64<DPP_ROW_HALF_MIRROR>(c[d]));
-    for (int d = 0; d < 6; d++) c[d] += dpp_f64<DPP_QUAD_2301>(c[d]);
-    for (int d = 0; d < 6; d++) c[d] += dpp_f64<DPP_QUAD_1032>(c[d]);
-    for (int d = 0; d < 3; d++) { acc[d] = c[d]; jerk[d] = c[3 + d]; }
-}
-
-// The active-particle correction of integrate_from (hermite.h:300-375) in lane groups,
-// for clusters with j-data in LDS.  The bodies to integrate are laid out in slots
-// (WaveSlots::ent): the active particles without twins, and merged targets with their
-// twins as families of consecutive slots inside one wave (a merged target integrates its
-// twins alongside, each with its own position and cut-off radius, and mergeAccJerk
-// averages their hard forces by mass).  A slot gets S = 2^s lanes (W.gs); each group
-// evaluates its body's hard force by group_pair_sum, and the members of a family add
-// their forces by shuffles in the order of coop_correct_active (target first, then the
-// twins in ascending index).  The steps and their order are those of
-// coop_correct_active, so the results are too.  Every thread of the workgroup calls it
-// (no barrier inside).
-template <int K>
-__device__ void group_correct_active(const HP &P, HardView &H, const JData &J, int b, int n, double t_s,
-                                     int flag_col, long long &pairs, const WaveSlots &W,
-                                     const double *__restrict__ a0_lds) {
-    const int t = threadIdx.x;
-    const int B = blockDim.x;
-    const int s = W.gs, E = 64 >> s;
-    const int r = t & ((1 << s) - 1);
-    const int nslot = W.nslot;
-    const bool fams = W.nfam > 0;
-    const int per_round = B >> s;
-    const int wave_first = (t & ~63) >> s;     // the wave's first slot in a round
-    for (int a0 = 0; a0 < nslot; a0 += per_round) {
-        if (a0 + wave_first >= nslot) continue;   // no body for this wave (wave-uniform)
-        const int slot = a0 + (t >> s);
-        const int e = slot < nslot ? W.ent[slot] : -1;
-        const bool valid = e >= 0;
-        const int g = b + (valid ? e : 0);      // empty slots compute a stand-in
-        int fn = 1, ff = slot;
-        bool mfam = false;
-        if (fams && slot < nslot) {
-            fn = W.efn[slot] & (FAM_MERGED - 1);
-            mfam = (W.efn[slot] & FAM_MERGED) != 0;
-            ff = W.efam[slot];
-        }
-        const bool twin = ff != slot;
-        const int gt = twin ? b + W.ent[ff] : g;  // the family's target
-        const int ffw = ff - (a0 + wave_first);   // its slot within the wave
-        const bool wave_fam = fams && __ballot(mfam) != 0ull;
-        const bool lead = valid && r == 0;
-        const double mass_e = H.mass[g];
-        double as[3], js[3], ad[3], jd[3], x[3], v[3];
-        // mergeAccJerk over the family (hermite.h:36-74), from the members' lanes
-        auto merge = [&]() __attribute__((always_inline)) {
-            if (!wave_fam) return;
-            double sa[6] = {0., 0., 0., 0., 0., 0.}, msum = 0.;
-            for (int k = 0; k < E; k++) {
-                const int src = ((ffw + k) << s) + r;
-                const double mk = __shfl(mass_e, src);
-                double ak[6];
-                for (int d = 0; d < 3; d++) { ak[d] = __shfl(ad[d], src); ak[3 + d] = __shfl(jd[d], src); }
-                if (k < fn) {
-                    if (k == 0) {
-                        for (int d = 0; d < 6; d++) sa[d] = mk * ak[d];
-                        msum = mk;
-                    } else {
-                        for (int d = 0; d < 6; d++) sa[d] += mk * ak[d];
-                        msum += mk;
-                    }
-                }
-            }
-            if (mfam) {
-                const double minv = 1. / msum;
-                for (int d = 0; d < 3; d++) { ad[d] = sa[d] * minv; jd[d] = sa[3 + d] * minv; }
-            }
-        };
-        // Registers are scarce here (the pair sums keep a subtree stack per lane): the
-        // body's predicted state and its acc/jerk at the start of the block step are
-        // reread from LDS (the j-data and a0) for each correction instead of being held
-        // across the pair sums, and the correction's a2/a3 terms go through H.
-        const int el = valid ? e : 0;
-        const double rinv = H.rinv[g];
-        const int64_t id = H.id[g];
-        {
-            double xp[3], vp[3];
-            ld3(J.x, el, xp); ld3(J.v, el, vp);
-            group_pair_sum<K>(P, J, n, s, r, id, xp, vp, rinv, ad, jd);
-            star_acc_jerk(P, xp, vp, as, js, nullptr);
-        }
-        merge();
-        const double t_c = t_s - H.time[gt];    // twins carry their target's time
-        for (int ite = 0; ite < 2; ite++) {
-            {
-                double xp[3], vp[3], a0s[3], j0s[3], a0d[3], j0d[3], a2s[3], a3s[3], a2d[3], a3d[3];
-                ld3(J.x, el, xp); ld3(J.v, el, vp);
-                const double *q = a0_lds + 12 * el;
-                for (int k = 0; k < 3; k++) {
-                    a0s[k] = q[k]; j0s[k] = q[3 + k]; a0d[k] = q[6 + k]; j0d[k] = q[9 + k];
-                }
-                correct_regs(t_c, xp, vp, as, a0s, j0s, js, ad, a0d, j0d, jd, x, v, a2s, a3s, a2d, a3d);
-                if (ite == 1 && lead && !twin) {
-                    st3(H.a2_s, g, a2s); st3(H.a3_s, g, a3s); st3(H.a2_d, g, a2d); st3(H.a3_d, g, a3d);
-                }
-            }
-            star_acc_jerk(P, x, v, as, js, nullptr);
-            group_pair_sum<K>(P, J, n, s, r, id, x, v, rinv, ad, jd);
-            merge();
-        }
-        wave_sync();     // the leader's a2/a3 before the group reads them back
-        const double time = H.time[g] + t_c;
-        double dt = H.dt[g];
-        if (!flag_col) {
-            double a2s[3], a3s[3], a2d[3], a3d[3];
-            ld3(H.a2_s, g, a2s); ld3(H.a3_s, g, a3s); ld3(H.a2_d, g, a2d); ld3(H.a3_d, g, a3d);
-            dt = dt_block(P, time, dt, H.acc0[g], ad, jd, a2d, a3d, as, js, a2s, a3s);
-        }
-        if (wave_fam) {                           // twins take their target's step
-            const double dtt = __shfl(dt, (ffw << s) + r);
-            if (twin) dt = dtt;
-        }
-        if (lead) {
-            pairs += 3 * (long long)(n - 1);
-            st3(H.pos, g, x); st3(H.vel, g, v);
-            st3(H.acc_s, g, as); st3(H.jerk_s, g, js); st3(H.acc_d, g, ad); st3(H.jerk_d, g, jd);
-            H.time[g] = time;
-            if (!flag_col) H.dt[g] = dt;
-        }
-    }
 }
 
 // After the collision test found the pair (ic, jc) in a block step and the active
@@ -1122,16 +836,11 @@ __device__ void collision_tail(const HP &P, HardView &H, int b, int n, int ic, i
     __syncthreads();
 }
 
-// Block steps of one cluster from (sys_time, loop) to the end of the soft step on the
-// global-memory state H (j-data through J), then the final calcGravity.  Every
-// thread of the workgroup calls it; collisions and twins handled here.  COOP: the
-// cluster has more than HARD_SEQ_MAX particles (the other correction path is left out
-// of the instantiation, which keeps its register use down).
-template <bool LDSJ, bool COOP>
-__device__ void integrate_from(const HP &P, HardView &H, const JData &J, Reduce &R, double *s_x, double *s_v,
-                               int64_t *s_id, double *s_fr, int b, int n, double &sys_time, long long &loop,
-                               double &ed, int &n_col, long long &pairs, WaveSlots *W = nullptr,
-                               double *s_a0 = nullptr) {
+// Block steps of a cluster too large for the LDS, from the start of the soft step to its
+// end on the global-memory state H (j-data through J), then the final calcGravity.  Every
+// thread of the workgroup calls it; collisions and twins handled here.
+__device__ void integrate_global(const HP &P, HardView &H, const JData &J, int b, int n, double &sys_time,
+                                 long long &loop, double &ed, int &n_col, long long &pairs, WaveSlots &W) {
     const int t = threadIdx.x;
     const int B = blockDim.x;
     const double time_end = P.dt_tree;
@@ -1140,135 +849,31 @@ __device__ void integrate_from(const HP &P, HardView &H, const JData &J, Reduce 
         double tl = 1.e10;
         for (int i = t; i < n; i += B)
             if (!(H.flags[b + i] & GPLUM_FLAG_DEAD)) tl = dmin(tl, H.time[b + i] + H.dt[b + i]);
-        const double t_s = COOP ? block_min_waves(tl, W->ts) : block_min(R, tl);
+        const double t_s = block_min_waves(tl, W.ts);
         // predict all (hermite.h:277-283)
-        for (int i = t; i < n; i += B) {
-            predict(H, b + i, t_s - H.time[b + i]);
-            if (LDSJ) {
-                for (int k = 0; k < 3; k++) {
-                    s_x[3 * i + k] = H.xp[3 * (b + i) + k];
-                    s_v[3 * i + k] = H.vp[3 * (b + i) + k];
-                }
-                s_id[i] = H.id[b + i];
-                // f R of the live particles for the collision test (-1: dead)
-                s_fr[i] = (H.flags[b + i] & GPLUM_FLAG_DEAD) ? -1. : H.f[b + i] * H.r_planet[b + i];
-                if (COOP) {
-                    W->tw[i] = H.twin_of[b + i];
-                    // acc/jerk at the start of the block step (predict's a0), for the lane groups
-                    for (int k = 0; k < 3; k++) {
-                        s_a0[12 * i + k] = H.a0_s[3 * (b + i) + k];
-                        s_a0[12 * i + 3 + k] = H.j0_s[3 * (b + i) + k];
-                        s_a0[12 * i + 6 + k] = H.a0_d[3 * (b + i) + k];
-                        s_a0[12 * i + 9 + k] = H.j0_d[3 * (b + i) + k];
-                    }
-                }
-            }
-        }
+        for (int i = t; i < n; i += B) predict(H, b + i, t_s - H.time[b + i]);
         __threadfence_block();
         __syncthreads();
         // collisionDetermination (hermite.h:98-196)
         int flag_col = 0, ic = -1, jc = -1;
         if (P.collision) {
-            double rmin = 1.;
-            int bi = 0x7fffffff, bj = COOP ? 0x7fffffff : -1;
-            if (LDSJ && COOP) {
-                // the unordered pairs {a, c} over all threads: c = (a + d) mod n for d = 1 ..
-                // (n - 1) / 2 and every a, and for even n d = n / 2 with a < n / 2.  R is
-                // symmetric bit for bit (squared differences, a commutative sum of f R),
-                // so the (R, lower, higher index) minimum is the (R, i, first j) minimum
-                // of the ordered loop below.
-                // Thread t takes particle a = t mod n and the r-th of R = B / n runs of
-                // the distances d (a difference of signs leaves d2 unchanged).
-                const int R = max(1, B / n);
-                if (t < n * R) {
-                    const int a = t % n, r = t / n;
-                    const int h = (n - 1) >> 1;
-                    const int dlen = (h + R - 1) / R;
-                    const int d0 = 1 + r * dlen, d1 = min(h, d0 + dlen - 1);
-                    const double fra = s_fr[a];
-                    const double xa = s_x[3 * a], ya = s_x[3 * a + 1], za = s_x[3 * a + 2];
-                    auto pair = [&](int c) {
-                        const double frc = s_fr[c];
-                        if (frc < 0.) return;
-                        const double dx = xa - s_x[3 * c];
-                        const double dy = ya - s_x[3 * c + 1];
-                        const double dz = za - s_x[3 * c + 2];
-                        const double d2 = dot3(dx, dy, dz, dx, dy, dz);
-                        const double r2 = fra + frc;
-                        if (!(d2 < COL_FILTER * r2 * r2)) return;
-                        const double Rr = sqrt(d2) / r2;
-                        const int lo = min(a, c), hi = max(a, c);
-                        if (Rr < 1. && rlh_less(Rr, lo, hi, rmin, bi, bj)) { rmin = Rr; bi = lo; bj = hi; }
-                    };
-                    if (fra >= 0.) {
-                        // four distances at a time (their LDS reads overlap); the minimum
-                        // does not depend on the order in which pairs are met
-                        int d = d0;
-                        for (; d + 3 <= d1; d += 4) {
-                            double frc[4], ddx[4], ddy[4], ddz[4];
-                            int cc[4];
-#pragma unroll
-                            for (int u = 0; u < 4; u++) {
-                                cc[u] = a + d + u < n ? a + d + u : a + d + u - n;
-                                frc[u] = s_fr[cc[u]];
-                                ddx[u] = xa - s_x[3 * cc[u]];
-                                ddy[u] = ya - s_x[3 * cc[u] + 1];
-                                ddz[u] = za - s_x[3 * cc[u] + 2];
-                            }
-#pragma unroll
-                            for (int u = 0; u < 4; u++) {
-                                if (frc[u] < 0.) continue;
-                                const double d2 = dot3(ddx[u], ddy[u], ddz[u], ddx[u], ddy[u], ddz[u]);
-                                const double r2 = fra + frc[u];
-                                if (!(d2 < COL_FILTER * r2 * r2)) continue;
-                                const double Rr = sqrt(d2) / r2;
-                                const int lo = min(a, cc[u]), hi = max(a, cc[u]);
-                                if (Rr < 1. && rlh_less(Rr, lo, hi, rmin, bi, bj)) { rmin = Rr; bi = lo; bj = hi; }
-                            }
-                        }
-                        for (; d <= d1; d++) pair(a + d < n ? a + d : a + d - n);
-                        // even n: the pairs at distance n / 2, once each (a < n / 2)
-                        if (!(n & 1) && r == R - 1 && a < (n >> 1)) pair(a + (n >> 1));
-                    }
-                }
-            } else
+            double rm = 1.;
+            int gi = 0x7fffffff, gj = 0x7fffffff;
             for (int i = t; i < n; i += B) {
-                if (LDSJ) {
-                    // predicted positions and f R from LDS
-                    const double fri = s_fr[i];
-                    if (fri < 0.) continue;
-                    const double xi = s_x[3 * i], yi = s_x[3 * i + 1], zi = s_x[3 * i + 2];
-                    for (int j = 0; j < n; j++) {
-                        const double frj = s_fr[j];
-                        if (i == j || frj < 0.) continue;
-                        const double dx = xi - s_x[3 * j];
-                        const double dy = yi - s_x[3 * j + 1];
-                        const double dz = zi - s_x[3 * j + 2];
-                        const double d2 = dot3(dx, dy, dz, dx, dy, dz);
-                        const double r2 = fri + frj;
-                        if (!(d2 < COL_FILTER * r2 * r2)) continue;
-                        const double Rr = sqrt(d2) / r2;
-                        if (Rr < rmin) { rmin = Rr; bi = i; bj = j; }
-                    }
-                } else {
-                    if (H.flags[b + i] & GPLUM_FLAG_DEAD) continue;
-                    for (int j = 0; j < n; j++) {
-                        if (i == j || (H.flags[b + j] & GPLUM_FLAG_DEAD)) continue;
-                        const double dx = H.xp[3 * (b + i)] - H.xp[3 * (b + j)];
-                        const double dy = H.xp[3 * (b + i) + 1] - H.xp[3 * (b + j) + 1];
-                        const double dz = H.xp[3 * (b + i) + 2] - H.xp[3 * (b + j) + 2];
-                        const double d2 = dot3(dx, dy, dz, dx, dy, dz);
-                        const double r2 = H.f[b + i] * H.r_planet[b + i] + H.f[b + j] * H.r_planet[b + j];
-                        if (!(d2 < COL_FILTER * r2 * r2)) continue;
-                        const double Rr = sqrt(d2) / r2;
-                        if (Rr < rmin) { rmin = Rr; bi = i; bj = j; }
-                    }
+                if (H.flags[b + i] & GPLUM_FLAG_DEAD) continue;
+                for (int j = 0; j < n; j++) {
+                    if (i == j || (H.flags[b + j] & GPLUM_FLAG_DEAD)) continue;
+                    const double dx = H.xp[3 * (b + i)] - H.xp[3 * (b + j)];
+                    const double dy = H.xp[3 * (b + i) + 1] - H.xp[3 * (b + j) + 1];
+                    const double dz = H.xp[3 * (b + i) + 2] - H.xp[3 * (b + j) + 2];
+                    const double d2 = dot3(dx, dy, dz, dx, dy, dz);
+                    const double r2 = H.f[b + i] * H.r_planet[b + i] + H.f[b + j] * H.r_planet[b + j];
+                    if (!(d2 < COL_FILTER * r2 * r2)) continue;
+                    const double Rr = sqrt(d2) / r2;
+                    if (Rr < rm) { rm = Rr; gi = i; gj = j; }
                 }
             }
-            int gi = bi, gj = bj;
-            double rm = rmin;
-            if (COOP) block_argmin_waves(rm, gi, gj, *W);
-            else rm = block_argmin(R, rmin, bi, bj, &gi, &gj);
+            block_argmin_waves(rm, gi, gj, W);
             if (rm < 1.) {
                 flag_col = 1;
                 if (H.mass[b + gi] < H.mass[b + gj]) { ic = gi; jc = gj; } else { ic = gj; jc = gi; }
@@ -1279,142 +884,12 @@ __device__ void integrate_from(const HP &P, HardView &H, const JData &J, Reduce 
             __syncthreads();
         }
         // correct the active particles (hermite.h:300-375)
-        if (COOP && LDSJ) {
-            // The bodies of the block step, laid out by the first wave for the lane groups
-            // (group_correct_active): the merged targets with their twins as families of
-            // consecutive slots that stay inside one wave (at most FAM_MAX members and
-            // FAM_GROUPS families; larger or further ones are flagged in H.act for
-            // coop_correct_active), then the active particles without twins in ascending
-            // index.  The two paths write disjoint particles and read only the predicted
-            // j-data.
-            if (t < 64) {
-                const unsigned long long below = (1ull << t) - 1ull;
-                int base = 0, nm = 0;
-                for (int i0 = 0; i0 < n; i0 += 64) {
-                    const int i = i0 + t;
-                    int a = 0, m = 0;
-                    if (i < n) {
-                        const int f = H.flags[b + i];
-                        a = !(f & GPLUM_FLAG_DEAD) && (flag_col || H.time[b + i] + H.dt[b + i] == t_s);
-                        m = a && (f & GPLUM_FLAG_MERGED);
-                        H.act[b + i] = 0;
-                        a = a && !m;
-                    }
-                    const unsigned long long ma = __ballot(a), mm = __ballot(m);
-                    if (a) W->act[base + __popcll(ma & below)] = i;
-                    if (m) W->mt[nm + __popcll(mm & below)] = i;
-                    base += __popcll(ma);
-                    nm += __popcll(mm);
-                }
-                // each merged target's twins in ascending index
-                int ntw = 0, nfam = 0, nbig = 0, fmem = 0, fmax = 1;
-                for (int k = 0; k < nm; k++) {
-                    const int tg = W->mt[k];
-                    int c = 0;
-                    for (int i0 = 0; i0 < n; i0 += 64) {
-                        const int i = i0 + t;
-                        const bool q = i < n && W->tw[i] == tg;
-                        const unsigned long long qm = __ballot(q);
-                        if (q) W->twl[ntw + c + __popcll(qm & below)] = i;
-                        c += __popcll(qm);
-                    }
-                    if (1 + c > FAM_MAX || nfam >= FAM_GROUPS) {
-                        if (t == 0) H.act[b + tg] = 1;     // coop_correct_active
-                        c = -1;
-                        nbig++;
-                    } else {
-                        ntw += c;
-                        nfam++;
-                        fmem += 1 + c;
-                        fmax = max(fmax, 1 + c);
-                    }
-                    if (t == 0) W->twn[k] = c;
-                }
-                // lanes per slot: the most that hold every body at once (at least 8, and
-                // few enough that a wave holds the largest family)
-                const int ne = base + fmem;
-                int sg = 6;
-                while (sg > 3 && (ne * (1 << sg) > B || (64 >> sg) < fmax)) sg--;
-                const int E = 64 >> sg;
-                int pos = 0;
-                if (t == 0) {
-                    int tw0 = 0;
-                    for (int k = 0; k < nm; k++) {
-                        const int c = W->twn[k];
-                        if (c < 0) continue;
-                        const int fsz = 1 + c;
-                        if ((pos % E) + fsz > E)
-                            while (pos % E) { W->ent[pos] = -1; W->efam[pos] = pos; W->efn[pos] = 1; pos++; }
-                        W->ent[pos] = W->mt[k];
-                        for (int q = 0; q < c; q++) W->ent[pos + 1 + q] = W->twl[tw0 + q];
-                        for (int q = 0; q < fsz; q++) { W->efam[pos + q] = pos; W->efn[pos + q] = fsz | FAM_MERGED; }
-                        tw0 += c;
-                        pos += fsz;
-                    }
-                }
-                pos = __shfl(pos, 0);
-                for (int k = t; k < base; k += 64) {
-                    W->ent[pos + k] = W->act[k];
-                    W->efam[pos + k] = pos + k;
-                    W->efn[pos + k] = 1;
-                }
-                if (t == 0) { W->nslot = pos + base; W->gs = sg; W->nfam = nfam; W->na = base; W->nm = nbig; }
-            }
-            __threadfence_block();
-            __syncthreads();
-            const int K = (n + 63) >> 6;
-            if (K <= 2) group_correct_active<2>(P, H, J, b, n, t_s, flag_col, pairs, *W, s_a0);
-            else if (K == 3) group_correct_active<3>(P, H, J, b, n, t_s, flag_col, pairs, *W, s_a0);
-            else group_correct_active<4>(P, H, J, b, n, t_s, flag_col, pairs, *W, s_a0);
-            if (W->nm > 0)
-                coop_correct_active(P, H, J, b, n, t_s, flag_col, pairs, (int)(threadIdx.x >> 6), B >> 6, W->tw);
-        } else if (COOP) {
-            for (int i = t; i < n; i += B)
-                H.act[b + i] = !(H.flags[b + i] & GPLUM_FLAG_DEAD) &&
-                               (flag_col || H.time[b + i] + H.dt[b + i] == t_s);
-            __threadfence_block();
-            __syncthreads();
-            coop_correct_active(P, H, J, b, n, t_s, flag_col, pairs, (int)(threadIdx.x >> 6), B >> 6,
-                                H.twin_of + b);
-        } else
-        for (int i = t; i < n; i += B) {
-            const int g = b + i;
-            if (H.flags[g] & GPLUM_FLAG_DEAD) continue;
-            if (!flag_col && H.time[g] + H.dt[g] != t_s) continue;
-            // a merged target integrates its dead twins alongside (hermite.h:300-375): each
-            // twin feels the hard force with its own r_out (cut-off), and mergeAccJerk
-            // averages target and twins by mass
-            const bool merged = (H.flags[g] & GPLUM_FLAG_MERGED) != 0;
-            pairs += 3 * (long long)(n - 1);
-            gravity_pc(P, H, J, n, g, false);
-            if (merged) {
-                for (int j = 0; j < n; j++)
-                    if (H.twin_of[b + j] == i) { gravity_pc(P, H, J, n, b + j, false); pairs += 3 * (long long)(n - 1); }
-                merge_acc_jerk(H, b, n, i);
-            }
-            const double t_c = t_s - H.time[g];
-            for (int ite = 0; ite < 2; ite++) {
-                correct(H, g, t_c);
-                if (merged)
-                    for (int j = 0; j < n; j++) if (H.twin_of[b + j] == i) correct(H, b + j, t_c);
-                gravity_pc(P, H, J, n, g, true);
-                if (merged) {
-                    for (int j = 0; j < n; j++) if (H.twin_of[b + j] == i) gravity_pc(P, H, J, n, b + j, true);
-                    merge_acc_jerk(H, b, n, i);
-                }
-            }
-            H.time[g] += t_c;
-            if (merged)
-                for (int j = 0; j < n; j++) if (H.twin_of[b + j] == i) H.time[b + j] += t_c;
-            if (!flag_col) {
-                double ad[3], jd[3], a2d[3], a3d[3], as[3], js[3], a2s[3], a3s[3];
-                ld3(H.acc_d, g, ad); ld3(H.jerk_d, g, jd); ld3(H.a2_d, g, a2d); ld3(H.a3_d, g, a3d);
-                ld3(H.acc_s, g, as); ld3(H.jerk_s, g, js); ld3(H.a2_s, g, a2s); ld3(H.a3_s, g, a3s);
-                H.dt[g] = dt_block(P, H.time[g], H.dt[g], H.acc0[g], ad, jd, a2d, a3d, as, js, a2s, a3s);
-                if (merged)
-                    for (int j = 0; j < n; j++) if (H.twin_of[b + j] == i) H.dt[b + j] = H.dt[g];
-            }
-        }
+        for (int i = t; i < n; i += B)
+            H.act[b + i] = !(H.flags[b + i] & GPLUM_FLAG_DEAD) &&
+                           (flag_col || H.time[b + i] + H.dt[b + i] == t_s);
+        __threadfence_block();
+        __syncthreads();
+        coop_correct_active(P, H, J, b, n, t_s, flag_col, pairs, (int)(threadIdx.x >> 6), B >> 6, H.twin_of + b);
         __threadfence_block();
         __syncthreads();
         if (flag_col) {
@@ -1425,7 +900,7 @@ __device__ void integrate_from(const HP &P, HardView &H, const JData &J, Reduce 
         double tm = 1.e10;
         for (int i = t; i < n; i += B)
             if (!(H.flags[b + i] & GPLUM_FLAG_DEAD)) tm = dmin(tm, H.time[b + i]);
-        sys_time = COOP ? block_min_waves(tm, W->sys) : block_min(R, tm);
+        sys_time = block_min_waves(tm, W.sys);
         loop++;
     }
     for (int i = t; i < n; i += B) { gravity_full(P, H, b, n, i); pairs += n - 1; }
@@ -1436,43 +911,6 @@ __device__ void integrate_from(const HP &P, HardView &H, const JData &J, Reduce 
             if (H.flags[b + i] & GPLUM_FLAG_MERGED) merge_acc_jerk(H, b, n, i);
     }
     __syncthreads();
-}
-
-// Pairs side by side for clusters of 3 to 8 particles (n (n - 1) <= 64): particle p
-// is held by the m = n - 1 lanes p m .. p m + m - 1, each keeping the particle's whole
-// state (computed alike), and lane p m + k evaluates p's pair with its k-th partner
-// j = k + (k >= p).  One pair_term latency covers all pairs of a block step; every lane
-// of the group then adds the group's m summands from the LDS, from zero in ascending j
-// (the sum of gravity_loop_lane).  Called by the lanes of active particles only.
-__device__ inline void side_force(const HP &P, int t, int base, int m, const double xo[3], const double vo[3],
-                                  double rinv, const double xj[3], const double vj[3], double mj, double rinv_j,
-                                  double *s_tm, double as[3], double js[3], double ad[3], double jd[3]) {
-    double ta[3], tj[3];
-    pair_term(P, xo, vo, rinv, xj[0], xj[1], xj[2], vj[0], vj[1], vj[2], mj, rinv_j, ta, tj, nullptr);
-    for (int d = 0; d < 3; d++) { s_tm[6 * t + d] = ta[d]; s_tm[6 * t + 3 + d] = tj[d]; }
-    star_acc_jerk(P, xo, vo, as, js, nullptr);
-    wave_sync();
-    for (int d = 0; d < 3; d++) { ad[d] = 0.; jd[d] = 0.; }
-    for (int k = 0; k < m; k++) {
-        const int L = base + k;
-        for (int d = 0; d < 3; d++) { ad[d] += s_tm[6 * L + d]; jd[d] += s_tm[6 * L + 3 + d]; }
-    }
-    wave_sync();   // summands read before the next evaluation writes them
-}
-
-// wave_min2 over the particles' values when the lanes p m (p < n) hold them and the
-// other lanes hold copies or 1e10 (m, n wave-uniform): up to four particles read
-// their lanes directly.
-__device__ inline void wave_min2_lead(double &u, double &v, int n, int m) {
-    if (n <= 2) {
-        u = dmin(readlane_f64(u, 0), readlane_f64(u, m));
-        v = dmin(readlane_f64(v, 0), readlane_f64(v, m));
-    } else if (n <= 4) {
-        u = dmin(dmin(readlane_f64(u, 0), readlane_f64(u, m)), dmin(readlane_f64(u, 2 * m), readlane_f64(u, 3 * m)));
-        v = dmin(dmin(readlane_f64(v, 0), readlane_f64(v, m)), dmin(readlane_f64(v, 2 * m), readlane_f64(v, 3 * m)));
-    } else {
-        wave_min2(u, v);
-    }
 }
 
 // ------------------------------------------- clusters of 2 to 4 bodies: lane per term
@@ -1862,325 +1300,168 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
     return true;
 }
 
-// Clusters that fit one wave: each particle's whole state stays in registers (one
-// lane per particle, or a group of lanes for 3 to 8 particles, see side_force) and
-// only the predicted j-data (and f r_planet) goes through LDS, so a block step costs a
-// few LDS round trips and wave shuffles instead of global-memory round trips.  Same
-// operations in the same order as integrate_from.  At the first block step with a
-// collision the state is written back to H and integrate_from takes over from the
-// start of that block step (it predicts the same positions and finds the same pair),
-// so merging and twins need no register path.
-__device__ void integrate_regs(const HP &P, HardView &H, const JData &J, Reduce &R, double *s_x, double *s_v,
-                               double *s_m, double *s_ri, int64_t *s_id, double *s_fr, double *s_tm, int b,
-                               int n, double &sys_time, long long &loop, double &ed, int &n_col,
-                               long long &pairs) {
-    n = __builtin_amdgcn_readfirstlane(n);   // wave-uniform: scalar branches on the size
-    const int t = threadIdx.x;
-    const bool side = n >= 3 && n * (n - 1) <= 64;
-    const int m = side ? n - 1 : 1;            // lanes per particle
-    const int p = t / m;                       // this lane's particle
-    const bool own = p < n;
-    const bool lead = own && t == p * m;       // the lane that writes p's shared state
-    const int g = b + p;
-    double x[3] = {0., 0., 0.}, v[3] = {0., 0., 0.}, as[3], js[3], ad[3], jd[3];
-    double time = 0., dt = 0., acc0 = 0., rinv = 0., fr = 0.;
-    int64_t id = -1;
-    if (own) {
-        ld3(H.pos, g, x);
-        ld3(H.vel, g, v);
-        time = H.time[g];
-        dt = H.dt[g];
-        acc0 = H.acc0[g];
-        rinv = H.rinv[g];
-        id = H.id[g];
-        fr = H.f[g] * H.r_planet[g];
-        if (lead) {
-            s_m[p] = H.mass[g];
-            s_ri[p] = rinv;
-            s_id[p] = id;
-            s_fr[p] = fr;
-            st3(s_x, p, x);
-            st3(s_v, p, v);
-        }
-    }
-    __syncthreads();
-    // The clusters the reference forms have distinct ids, and the partner loops below
-    // leave the id test out; a cluster with a repeated id takes the global-memory path
-    // from the start (the non-register kernels' preamble, then integrate_from).
-    // (One call site of integrate_from serves both hand-overs: a second inlined copy
-    // would double the kernel's register allocation.)
-    bool rep = false;
-    if (own)
-        for (int j = 0; j < n; j++) rep = rep || (j != p && s_id[j] == id);
-    const bool from_start = __ballot(rep) != 0;
-    // 2 to 4 bodies: the lane-per-term path (a collision hands over to integrate_from below)
-    const bool terms = !from_start && n <= P.terms_max;
-    bool terms_handover = false;
-    if (terms) {
-        const bool done =
-            (n == 2) ? integrate_terms<2>(P, H, J, s_x, s_v, s_m, s_ri, s_id, s_fr, s_tm, b, sys_time, loop, pairs)
-            : (n == 3) ? integrate_terms<3>(P, H, J, s_x, s_v, s_m, s_ri, s_id, s_fr, s_tm, b, sys_time, loop, pairs)
-                       : integrate_terms<4>(P, H, J, s_x, s_v, s_m, s_ri, s_id, s_fr, s_tm, b, sys_time, loop, pairs);
-        if (done) return;
-        terms_handover = true;
-    }
-    // side_force: this lane's partner and its constants
-    int jp = 0;
-    double m_jp = 0., ri_jp = 0.;
-    if (side && own) {
-        const int k = t - p * m;
-        jp = k + (k >= p ? 1 : 0);
-        m_jp = s_m[jp];
-        ri_jp = s_ri[jp];
-    }
-    if (from_start) {
-        if (lead) {
-            gravity_full(P, H, b, n, p);
-            H.flags[g] &= ~(GPLUM_FLAG_DEAD | GPLUM_FLAG_MERGED);
-            H.twin_of[g] = -1;
-        }
-    } else if (own && !terms) {
-        // initial calcGravity (hermite.h:259-270)
-        star_acc_jerk(P, x, v, as, js, nullptr);
-        gravity_loop_lane<false>(P, J, n, p, id, x, v, rinv, ad, jd, nullptr);
-    }
-    const double time_end = P.dt_tree;
-    double a0s[3], j0s[3], a0d[3], j0d[3], xp[3], vp[3], a2s[3], a3s[3], a2d[3], a3d[3];
-    // t_s: the next block time, min(time + dt) (makeActiveList); computed together with
-    // the system time at the end of each step
-    double t_s = wave_min(own ? time + dt : 1.e10);
-    bool handover = false;
-    while (!from_start && !terms && sys_time < time_end && loop < BLOCK_STEP_CAP) {
-        __syncthreads();   // the previous step's j-data reads are done
-        if (own) {
-            predict_regs(t_s - time, x, v, as, js, ad, jd, a0s, j0s, a0d, j0d, xp, vp);
-            if (lead) {
-                st3(s_x, p, xp);
-                st3(s_v, p, vp);
-            }
-        }
-        __syncthreads();
-        if (P.collision) {
-            double rmin = 1.;
-            int bi = 0x7fffffff, bj = -1;
-            if (own) {
-                for (int k = 0; k < n - 1; k++) {
-                    const int j = k + (k >= p ? 1 : 0);   // the partners, ascending
-                    const double dx = xp[0] - s_x[3 * j];
-                    const double dy = xp[1] - s_x[3 * j + 1];
-                    const double dz = xp[2] - s_x[3 * j + 2];
-                    const double d2 = dot3(dx, dy, dz, dx, dy, dz);
-                    const double r2 = fr + s_fr[j];
-                    if (!(d2 < COL_FILTER * r2 * r2)) continue;   // R >= 1: never the minimum
-                    const double Rr = sqrt(d2) / r2;
-                    if (Rr < rmin) { rmin = Rr; bi = p; bj = j; }
-                }
-            }
-            // the argmin only when some pair is below 1 (rare)
-            if (__ballot(rmin < 1.)) wave_argmin(rmin, bi, bj);
-            if (__ballot(rmin < 1.)) { handover = true; break; }
-        }
-        if (own && time + dt == t_s) {
-            if (lead) pairs += 3 * (long long)(n - 1);
-            const double t_c = t_s - time;
-            if (side) {
-                // the partner's predicted state, once for the three evaluations
-                double xj[3], vj[3];
-                ld3(s_x, jp, xj);
-                ld3(s_v, jp, vj);
-                side_force(P, t, p * m, m, xp, vp, rinv, xj, vj, m_jp, ri_jp, s_tm, as, js, ad, jd);
-                for (int ite = 0; ite < 2; ite++) {
-                    correct_regs(t_c, xp, vp, as, a0s, j0s, js, ad, a0d, j0d, jd, x, v, a2s, a3s, a2d, a3d);
-                    side_force(P, t, p * m, m, x, v, rinv, xj, vj, m_jp, ri_jp, s_tm, as, js, ad, jd);
-                }
-            } else if (n == 2) {
-                // the partner's predicted state is read once for the three evaluations
-                JReg pj[1];
-                load_jreg(J, p == 0 ? 1 : 0, pj[0]);
-                force_jreg<1>(P, pj, xp, vp, rinv, as, js, ad, jd);
-                for (int ite = 0; ite < 2; ite++) {
-                    correct_regs(t_c, xp, vp, as, a0s, j0s, js, ad, a0d, j0d, jd, x, v, a2s, a3s, a2d, a3d);
-                    force_jreg<1>(P, pj, x, v, rinv, as, js, ad, jd);
-                }
-            } else {
-                star_acc_jerk(P, xp, vp, as, js, nullptr);
-                gravity_loop_lane<false>(P, J, n, p, id, xp, vp, rinv, ad, jd, nullptr);
-                for (int ite = 0; ite < 2; ite++) {
-                    correct_regs(t_c, xp, vp, as, a0s, j0s, js, ad, a0d, j0d, jd, x, v, a2s, a3s, a2d, a3d);
-                    star_acc_jerk(P, x, v, as, js, nullptr);
-                    gravity_loop_lane<false>(P, J, n, p, id, x, v, rinv, ad, jd, nullptr);
-                }
-            }
-            time += t_c;
-            dt = dt_block(P, time, dt, acc0, ad, jd, a2d, a3d, as, js, a2s, a3s);
-        }
-        sys_time = own ? time : 1.e10;
-        t_s = own ? time + dt : 1.e10;
-        wave_min2_lead(sys_time, t_s, n, m);
-        loop++;
-    }
-    if (handover || from_start || terms_handover) {
-        // a collision in this block step: hand the cluster to the global-memory path
-        // at the start of the step (kept out of the loop, which then holds less state)
-        if (handover && lead) {
-            st3(H.pos, g, x); st3(H.vel, g, v);
-            st3(H.acc_s, g, as); st3(H.jerk_s, g, js);
-            st3(H.acc_d, g, ad); st3(H.jerk_d, g, jd);
-            H.time[g] = time;
-            H.dt[g] = dt;
-            H.flags[g] &= ~(GPLUM_FLAG_DEAD | GPLUM_FLAG_MERGED);
-            H.twin_of[g] = -1;
-        }
-        __threadfence_block();
-        __syncthreads();
-        integrate_from<true, false>(P, H, J, R, s_x, s_v, s_id, s_fr, b, n, sys_time, loop, ed, n_col, pairs);
-        return;
-    }
-    // final calcGravity with potentials (hermite.h:466-470), current positions
-    __syncthreads();
-    if (lead) {
-        st3(s_x, p, x);
-        st3(s_v, p, v);
-    }
-    __syncthreads();
-    if (own) {
-        double phs = 0., phd = 0.;
-        star_acc_jerk(P, x, v, as, js, &phs);
-        gravity_loop_lane<false>(P, J, n, p, id, x, v, rinv, ad, jd, &phd);
-        if (lead) {
-            pairs += n - 1;
-            st3(H.pos, g, x); st3(H.vel, g, v);
-            st3(H.acc_s, g, as); st3(H.jerk_s, g, js);
-            st3(H.acc_d, g, ad); st3(H.jerk_d, g, jd);
-            H.time[g] = time;
-            H.dt[g] = dt;
-            H.phi_s[g] = phs;
-            H.phi_d[g] = phd;
-            H.flags[g] &= ~(GPLUM_FLAG_DEAD | GPLUM_FLAG_MERGED);
-            H.twin_of[g] = -1;
-        }
-    }
-    __syncthreads();
-}
+}  // namespace gplum
 
-// Three instantiations, one per cluster-size class (each skips the others):
-// REG: n <= HARD_SEQ_MAX, particle state in registers (integrate_regs);
-// LDSJ && !REG: HARD_SEQ_MAX < n <= HERMITE_LDS, j-data in LDS (integrate_from);
-// !LDSJ: n > HERMITE_LDS, j-data in global memory.
-// The REG kernel runs one wave per workgroup; the other two run HERMITE_BIG_BLOCK
-// threads, whose waves share the active particles of a block step.
-// Separate kernels keep the register-heavy small-cluster path from lowering the
-// occupancy of the others.
-template <bool LDSJ, bool REG>
-__device__ __forceinline__ void hermite_clusters(HP P_arg, HardView H,
-                                                           const int32_t *__restrict__ cl_off,
-                                                           const int32_t *__restrict__ order, int ncl,
-                                                           int *__restrict__ next, double *__restrict__ edisp,
-                                                           int *__restrict__ ncol, long long *__restrict__ nblock,
-                                                           long long *__restrict__ npair, int persistent,
-                                                           int lds_max, int giant_min) {
-    __shared__ double s_x[3 * HERMITE_LDS], s_v[3 * HERMITE_LDS], s_m[HERMITE_LDS], s_ri[HERMITE_LDS];
-    __shared__ int64_t s_id[HERMITE_LDS];
-    __shared__ double s_fr[HERMITE_LDS];
-    __shared__ Reduce R;
+#include "hermite_lds.hpp"
+
+namespace gplum {
+
+// The clusters of a launch, pulled from a queue (persistent) or one per workgroup: calls
+// run(c, b, n, sys_time, loop, ed, n_col, pairs) for those of lo < n <= hi members and
+// records the outcome.  Every thread of the workgroup calls it.
+template <class F>
+__device__ __forceinline__ void cluster_queue(const HP &P, const ClusterArgs &A, int lo, int hi, F run) {
     __shared__ int s_cl;
     __shared__ unsigned long long s_pairs;
-    // the register path reads the physics constants from LDS: as kernel arguments they
-    // would occupy scalar registers for the whole kernel (and be spilled and reloaded
-    // in its loop); the other paths keep them as arguments
-    __shared__ HP s_P;
-    // register path, 3 to 8 particles: pair summands (side_force)
-    __shared__ double s_tm[REG ? 6 * 64 : 1];
-    // multi-wave kernels: reduction slots and the active list, and each particle's
-    // acc/jerk at the start of the block step (12 per particle) for the lane groups
-    __shared__ __align__(8) unsigned char s_ws[REG ? 8 : sizeof(WaveSlots)];
-    __shared__ double s_a0[(REG || !LDSJ) ? 1 : 12 * HERMITE_LDS];
     const int t = threadIdx.x;
     const int B = blockDim.x;
-    if (REG) {
-        if (t == 0) s_P = P_arg;
-        __syncthreads();
-    }
-    const HP &P = REG ? s_P : P_arg;
     for (int iter = 0;; iter++) {
-        if (persistent) {
-            if (t == 0) s_cl = atomicAdd(next, 1);
-            __syncthreads();
-        } else {
-            if (t == 0) s_cl = (iter == 0) ? (int)blockIdx.x : ncl;
-            __syncthreads();
-        }
+        if (t == 0) s_cl = A.persistent ? atomicAdd(A.next, 1) : ((iter == 0) ? (int)blockIdx.x : A.ncl);
+        __syncthreads();
         const int q = s_cl;
         __syncthreads();
-        if (q >= ncl) break;
-        const int c = order ? order[q] : q;
-        const int b = cl_off[c];
-        const int n = cl_off[c + 1] - b;
-        if (REG && n > HARD_SEQ_MAX) continue;
-        if (LDSJ && !REG && (n <= HARD_SEQ_MAX || n > lds_max || n > giant_min)) continue;
-        if (!LDSJ && (n <= lds_max || n > giant_min)) continue;
-        JData J;
-        if (LDSJ) {
-            J = JData{s_x, s_v, s_m, s_ri, s_id, 3};
-            for (int i = t; i < n; i += B) { s_m[i] = H.mass[b + i]; s_ri[i] = H.rinv[b + i]; }
-        } else {
-            J = JData{H.xp + 3 * b, H.vp + 3 * b, H.mass + b, H.rinv + b, H.id + b, 3};
-        }
-        // pair evaluations of this cluster (hard_pair calls), for the roofline
-        long long pairs = (long long)(n > 0 ? n - 1 : 0) * ((t < n) ? (n - 1 - t) / B + 1 : 0);
+        if (q >= A.ncl) break;
+        const int c = A.order ? A.order[q] : q;
+        const int b = __builtin_amdgcn_readfirstlane(A.off[c]);
+        const int n = __builtin_amdgcn_readfirstlane(A.off[c + 1]) - b;
+        if (n <= lo || n > hi) continue;
+        // pair evaluations of this cluster (hard_pair calls), for the roofline: those of the
+        // initial calcGravity first
+        long long pairs = (long long)(n - 1) * ((t < n) ? (n - 1 - t) / B + 1 : 0);
         if (t == 0) s_pairs = 0ull;
         double ed = 0.;
         int n_col = 0;
         long long loop = 0;
         double sys_time = 0.;
-        if (REG) {
-            integrate_regs(P, H, J, R, s_x, s_v, s_m, s_ri, s_id, s_fr, s_tm, b, n, sys_time, loop, ed, n_col,
-                           pairs);
-        } else {
-            // initial calcGravity for all, flags cleared (hermite.h:259-270)
-            for (int i = t; i < n; i += B) {
-                gravity_full(P, H, b, n, i);
-                H.flags[b + i] &= ~(GPLUM_FLAG_DEAD | GPLUM_FLAG_MERGED);
-                H.twin_of[b + i] = -1;
-            }
-            __syncthreads();
-            integrate_from<LDSJ, true>(P, H, J, R, s_x, s_v, s_id, s_fr, b, n, sys_time, loop, ed, n_col, pairs,
-                                       reinterpret_cast<WaveSlots *>(s_ws), s_a0);
-        }
+        run(b, n, sys_time, loop, ed, n_col, pairs);
+        __syncthreads();
         atomicAdd(&s_pairs, (unsigned long long)pairs);
         __syncthreads();
-        const double time_end = P.dt_tree;
         if (t == 0) {
-            edisp[c] = ed;
-            ncol[c] = n_col;
-            nblock[c] = (sys_time < time_end) ? -1 : loop;   // -1: block-step cap reached
-            npair[c] = (long long)s_pairs;
+            A.edisp[c] = ed;
+            A.ncol[c] = n_col;
+            A.nblock[c] = (sys_time < P.dt_tree) ? -1 : loop;   // -1: block-step cap reached
+            A.npair[c] = (long long)s_pairs;
         }
         __syncthreads();
     }
 }
 
-// The register path: one wave per workgroup, all the registers a lane may have.
-template <bool LDSJ, bool REG>
-__global__ __launch_bounds__(HERMITE_BLOCK) void k_hermite(HP P, HardView H, const int32_t *__restrict__ cl_off,
-                                                           const int32_t *__restrict__ order, int ncl,
-                                                           int *__restrict__ next, double *__restrict__ edisp,
-                                                           int *__restrict__ ncol, long long *__restrict__ nblock,
-                                                           long long *__restrict__ npair, int persistent, int lds_max,
-                                                           int giant_min) {
-    hermite_clusters<LDSJ, REG>(P, H, cl_off, order, ncl, next, edisp, ncol, nblock, npair, persistent, lds_max,
-                                giant_min);
+// Clusters of up to HERMITE_SMALL members, one wave each: 2 to terms_max bodies with a lane
+// per term (a collision hands over to the LDS path in the middle of the soft step), the
+// others on the LDS path.  The arguments are read from LDS: in scalar registers they would
+// be spilled and reloaded in the block-step loop.
+__global__ __launch_bounds__(HERMITE_BLOCK) void k_hermite_small(HP P_arg, HardView H_arg, ClusterArgs A_arg, int lo,
+                                                                 int hi) {
+    __shared__ HP P;
+    __shared__ HardView H;
+    __shared__ ClusterArgs A;
+    __shared__ ClusterLds<HERMITE_SMALL> C;
+    constexpr int TP = lds_terms(HERMITE_BLOCK, 1, HERMITE_SMALL);
+    __shared__ double2 s_term[3 * TP];
+    const int t = threadIdx.x;
+    if (t == 0) {
+        P = P_arg;
+        H = H_arg;
+        A = A_arg;
+    }
+    __syncthreads();
+    cluster_queue(P, A, lo, hi, [&](int b, int n, double &sys_time, long long &loop, double &ed, int &n_col,
+                                    long long &pairs) {
+        bool fresh = true;
+        if (n >= 2 && n <= P.terms_max) {
+            if (t < n) {
+                C.mass[t] = H.mass[b + t];
+                C.rinv[t] = H.rinv[b + t];
+                C.id[t] = H.id[b + t];
+                C.fr[t] = H.f[b + t] * H.r_planet[b + t];
+            }
+            __syncthreads();
+            // the clusters the reference forms have distinct ids, and the lane-per-term path
+            // leaves the id test out
+            bool rep = false;
+            if (t < n)
+                for (int j = 0; j < n; j++) rep = rep || (j != t && C.id[j] == C.id[t]);
+            if (__ballot(rep) == 0) {
+                const JData J{C.xp, C.vp, C.mass, C.rinv, C.id, 3};
+                double *tm = reinterpret_cast<double *>(s_term);
+                const bool done =
+                    (n == 2)   ? integrate_terms<2>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b, sys_time, loop, pairs)
+                    : (n == 3) ? integrate_terms<3>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b, sys_time, loop, pairs)
+                               : integrate_terms<4>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b, sys_time, loop, pairs);
+                if (done) return;
+                fresh = false;
+                __threadfence_block();
+                __syncthreads();
+            }
+        }
+        run_cluster_lds<HERMITE_SMALL, HERMITE_BLOCK>(P, H, C, b, n, fresh, n_col, pairs, [&](HardView &V) {
+            integrate_seq<HERMITE_SMALL, HERMITE_BLOCK, TP>(P, C, V, s_term, n, sys_time, loop, ed, n_col, pairs);
+        });
+    });
 }
 
-// The larger clusters' kernels: HERMITE_BIG_BLOCK threads, two waves per SIMD (256
-// registers per lane).
-template <bool LDSJ>
-__global__ __launch_bounds__(HERMITE_BIG_BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void k_hermite_multi(
-    HP P, HardView H, const int32_t *__restrict__ cl_off, const int32_t *__restrict__ order, int ncl,
-    int *__restrict__ next, double *__restrict__ edisp, int *__restrict__ ncol, long long *__restrict__ nblock,
-    long long *__restrict__ npair, int persistent, int lds_max, int giant_min) {
-    hermite_clusters<LDSJ, false>(P, H, cl_off, order, ncl, next, edisp, ncol, nblock, npair, persistent, lds_max,
-                                  giant_min);
+// Clusters of NMIN to NMAX <= HARD_SEQ_MAX members on T threads.
+// (two waves per SIMD: two to four clusters of a large batch share a CU)
+template <int NMIN, int NMAX, int T>
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(2))) void k_hermite_mid(HP P, HardView H_arg, ClusterArgs A_arg, int lo, int hi) {
+    __shared__ HardView H;
+    __shared__ ClusterArgs A;
+    __shared__ ClusterLds<NMAX> C;
+    constexpr int TP = lds_terms(T, NMIN, NMAX);
+    __shared__ double2 s_term[3 * TP];
+    if (threadIdx.x == 0) {
+        H = H_arg;
+        A = A_arg;
+    }
+    __syncthreads();
+    cluster_queue(P, A, lo, hi, [&](int b, int n, double &sys_time, long long &loop, double &ed, int &n_col,
+                                    long long &pairs) {
+        run_cluster_lds<NMAX, T>(P, H, C, b, n, true, n_col, pairs, [&](HardView &V) {
+            integrate_seq<NMAX, T, TP>(P, C, V, s_term, n, sys_time, loop, ed, n_col, pairs);
+        });
+    });
+}
+
+// Clusters of HARD_SEQ_MAX + 1 to HERMITE_LDS members.
+__global__ __launch_bounds__(HERMITE_BIG_BLOCK) void k_hermite_big(HP P, HardView H_arg, ClusterArgs A_arg, int lo,
+                                                                   int hi) {
+    __shared__ HardView H;
+    __shared__ ClusterArgs A;
+    __shared__ ClusterLds<HERMITE_LDS> C;
+    __shared__ TreeLds<HERMITE_LDS> E;
+    if (threadIdx.x == 0) {
+        H = H_arg;
+        A = A_arg;
+    }
+    __syncthreads();
+    cluster_queue(P, A, lo, hi, [&](int b, int n, double &sys_time, long long &loop, double &ed, int &n_col,
+                                    long long &pairs) {
+        run_cluster_lds<HERMITE_LDS, HERMITE_BIG_BLOCK>(P, H, C, b, n, true, n_col, pairs, [&](HardView &V) {
+            integrate_tree<HERMITE_LDS, HERMITE_BIG_BLOCK>(P, C, E, V, n, sys_time, loop, ed, n_col, pairs);
+        });
+    });
+}
+
+// Larger clusters on the global-memory state: eight waves, two per SIMD (256 registers per
+// lane).
+__global__ __launch_bounds__(HERMITE_GLOBAL_BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void k_hermite_global(
+    HP P, HardView H, ClusterArgs A, int lo, int hi) {
+    __shared__ WaveSlots W;
+    const int t = threadIdx.x;
+    cluster_queue(P, A, lo, hi, [&](int b, int n, double &sys_time, long long &loop, double &ed, int &n_col,
+                                    long long &pairs) {
+        const JData J{H.xp + 3 * b, H.vp + 3 * b, H.mass + b, H.rinv + b, H.id + b, 3};
+        // initial calcGravity for all, flags cleared (hermite.h:259-270)
+        for (int i = t; i < n; i += HERMITE_GLOBAL_BLOCK) {
+            gravity_full(P, H, b, n, i);
+            H.flags[b + i] &= ~(GPLUM_FLAG_DEAD | GPLUM_FLAG_MERGED);
+            H.twin_of[b + i] = -1;
+        }
+        __threadfence_block();
+        __syncthreads();
+        integrate_global(P, H, J, b, n, sys_time, loop, ed, n_col, pairs, W);
+    });
 }
 
 // ------------------------------------------------------------- isolated
@@ -2737,35 +2018,54 @@ static int hard_giants(const HP &P, HardView &H, HardBuffers &hb, const std::vec
     return GPLUM_OK;
 }
 
-// zeroes the three cluster-queue counters (a kernel, not a memset, so that the launch
+// The size classes of the batched launch and their kernels; each class has a queue counter
+// of its own.  A class of T threads evaluates T / n bodies' pair terms per round, and most
+// block steps correct fewer bodies than that.  The lines (us per block step of one cluster):
+// 16 members on one wave 5.9-7.2, on 256 threads 5.2-5.4, but four clusters per CU instead of
+// one or two, which decides for batches; 32 on 256 threads 6.1-7.4, on 128 6.7-9.6; 64 on 512
+// threads 8.8-9.4, on 256 10.2-10.9.
+static int class_hi(int cls, int lds_max) {
+    return cls == 0 ? HERMITE_SMALL : cls == 1 ? HERMITE_MID : cls == 2 ? HARD_SEQ_MAX : cls == 3 ? lds_max : 0x7fffffff;
+}
+static int class_lo(int cls, int lds_max) { return cls == 0 ? 0 : class_hi(cls - 1, lds_max); }
+static void launch_class(int cls, const HP &P, const HardView &H, const ClusterArgs &A, int grid, int lo, int hi,
+                         hipStream_t st) {
+    switch (cls) {
+    case 0: hipLaunchKernelGGL(k_hermite_small, dim3(grid), dim3(HERMITE_BLOCK), 0, st, P, H, A, lo, hi); break;
+    case 1: hipLaunchKernelGGL((k_hermite_mid<HERMITE_SMALL + 1, HERMITE_MID, 256>), dim3(grid), dim3(256), 0, st, P, H, A, lo, hi); break;
+    case 2: hipLaunchKernelGGL((k_hermite_mid<HERMITE_MID + 1, HARD_SEQ_MAX, 512>), dim3(grid), dim3(512), 0, st, P, H, A, lo, hi); break;
+    case 3: hipLaunchKernelGGL(k_hermite_big, dim3(grid), dim3(HERMITE_BIG_BLOCK), 0, st, P, H, A, lo, hi); break;
+    default:
+        hipLaunchKernelGGL(k_hermite_global, dim3(grid), dim3(HERMITE_GLOBAL_BLOCK), 0, st, P, H, A, lo, hi);
+    }
+}
+
+// zeroes the cluster-queue counters (a kernel, not a memset, so that the launch
 // sequence can be captured into a graph and replayed)
 __global__ void k_reset_queue(int *next) {
-    if (threadIdx.x < 3) next[threadIdx.x] = 0;
+    if (threadIdx.x < HERMITE_CLASSES) next[threadIdx.x] = 0;
 }
 
 int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *d_off,
-                const int32_t *d_order, bool persistent, int n_cu, hipStream_t st, hipStream_t st2,
-                hipEvent_t ev_fork, hipEvent_t ev_join, int wg_per_cu, int lds_max, int giant_min, int terms_max) {
+                const int32_t *d_order, bool persistent, int n_cu, hipStream_t st, HardStreams &hs,
+                int wg_per_cu, int lds_max, int giant_min, int terms_max) {
     if (ncl <= 0) return GPLUM_OK;
     HP P = make_hp(p);
     P.terms_max = std::max(0, std::min(TERMS_MAX, terms_max));
     HardView H = hard_view(hb);
-    GPLUM_ENSURE(hb.next, 3);
+    GPLUM_ENSURE(hb.next, HERMITE_CLASSES);
     GPLUM_ENSURE(hb.edisp, ncl);
     GPLUM_ENSURE(hb.ncol, ncl);
     GPLUM_ENSURE(hb.nblock, ncl);
     GPLUM_ENSURE(hb.npair, ncl);
     hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, st, hb.next.p);
-    const int pers = persistent ? 1 : 0;
     lds_max = std::min(HERMITE_LDS, std::max(HARD_SEQ_MAX, lds_max));
     const int grid = persistent ? std::min(ncl, std::max(1, n_cu) * std::max(1, wg_per_cu)) : ncl;
-    // clusters above HARD_SEQ_MAX on a second stream (when given), concurrently with
-    // the register-path kernel
-    const bool big = hb.max_size > HARD_SEQ_MAX;
-    hipStream_t sb = (st2 && big) ? st2 : st;
-    if (sb != st) {
-        GPLUM_HIP(hipEventRecord(ev_fork, st));
-        GPLUM_HIP(hipStreamWaitEvent(sb, ev_fork, 0));
+    const bool big = hb.max_size > HERMITE_SMALL;
+    if (big) {
+        int rc = hs.ensure();
+        if (rc) return rc;
+        GPLUM_HIP(hipEventRecord(hs.fork, st));
     }
     giant_min = std::max(HARD_SEQ_MAX, giant_min);
     // giant clusters start right after the gather: their stream pool waits on this event
@@ -2775,16 +2075,18 @@ int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *
         if (rc) return rc;
         GPLUM_HIP(hipEventRecord(gpool.fork, st));
     }
-    if (hb.max_size > lds_max)
-        hipLaunchKernelGGL((k_hermite_multi<false>), dim3(grid), dim3(HERMITE_BIG_BLOCK), 0, sb, P, H, d_off, d_order,
-                           ncl, hb.next.p + 2, hb.edisp.p, hb.ncol.p, hb.nblock.p, hb.npair.p, pers, lds_max,
-                           giant_min);
-    if (big)
-        hipLaunchKernelGGL((k_hermite_multi<true>), dim3(grid), dim3(HERMITE_BIG_BLOCK), 0, sb, P, H, d_off, d_order,
-                           ncl, hb.next.p + 1, hb.edisp.p, hb.ncol.p, hb.nblock.p, hb.npair.p, pers, lds_max,
-                           giant_min);
-    hipLaunchKernelGGL((k_hermite<true, true>), dim3(grid), dim3(HERMITE_BLOCK), 0, st, P, H, d_off, d_order, ncl,
-                       hb.next.p, hb.edisp.p, hb.ncol.p, hb.nblock.p, hb.npair.p, pers, lds_max, giant_min);
+    ClusterArgs A{d_off, d_order, ncl, persistent ? 1 : 0, hb.next.p, hb.edisp.p, hb.ncol.p, hb.nblock.p, hb.npair.p};
+    bool launched[HERMITE_CLASSES] = {};
+    for (int k = 0; k < HERMITE_CLASSES; k++) {
+        const int cls = HERMITE_CLASSES - 1 - k;               // the longest chains first
+        const int lo = class_lo(cls, lds_max), hi = std::min(class_hi(cls, lds_max), giant_min);
+        if (cls > 0 && (hb.max_size <= lo || hi <= lo)) continue;
+        A.next = hb.next.p + cls;
+        if (cls > 0) GPLUM_HIP(hipStreamWaitEvent(hs.s[cls - 1], hs.fork, 0));
+        launch_class(cls, P, H, A, grid, lo, hi, cls > 0 ? hs.s[cls - 1] : st);
+        if (cls > 0) GPLUM_HIP(hipEventRecord(hs.join[cls - 1], hs.s[cls - 1]));
+        launched[cls] = true;
+    }
     if (hb.max_size > giant_min) {
         // giant clusters: several at a time over the whole GPU on a stream pool (the
         // size-class kernels above run meanwhile)
@@ -2800,10 +2102,8 @@ int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *
         int rc = hard_giants(P, H, hb, giants, off, st, gpool);
         if (rc) return rc;
     }
-    if (sb != st) {
-        GPLUM_HIP(hipEventRecord(ev_join, sb));
-        GPLUM_HIP(hipStreamWaitEvent(st, ev_join, 0));
-    }
+    for (int cls = 1; cls < HERMITE_CLASSES; cls++)
+        if (launched[cls]) GPLUM_HIP(hipStreamWaitEvent(st, hs.join[cls - 1], 0));
     GPLUM_HIP(hipGetLastError());
     return GPLUM_OK;
 }
@@ -2842,15 +2142,10 @@ int hard_launch_single(const gplum_params &p, HardBuffers &hb, int c, int n_c, c
     // one launch integrating cluster c (n_c particles) only: the per-cluster-launch comparator
     HP P = make_hp(p);
     HardView H = hard_view(hb);
-    if (n_c <= HARD_SEQ_MAX)
-        hipLaunchKernelGGL((k_hermite<true, true>), dim3(1), dim3(HERMITE_BLOCK), 0, st, P, H, d_off + c, nullptr, 1,
-                           hb.next.p, hb.edisp.p + c, hb.ncol.p + c, hb.nblock.p + c, hb.npair.p + c, 0, HERMITE_LDS, 0x7fffffff);
-    else if (n_c <= HERMITE_LDS)
-        hipLaunchKernelGGL((k_hermite_multi<true>), dim3(1), dim3(HERMITE_BIG_BLOCK), 0, st, P, H, d_off + c, nullptr, 1,
-                           hb.next.p, hb.edisp.p + c, hb.ncol.p + c, hb.nblock.p + c, hb.npair.p + c, 0, HERMITE_LDS, 0x7fffffff);
-    else
-        hipLaunchKernelGGL((k_hermite_multi<false>), dim3(1), dim3(HERMITE_BIG_BLOCK), 0, st, P, H, d_off + c, nullptr,
-                           1, hb.next.p, hb.edisp.p + c, hb.ncol.p + c, hb.nblock.p + c, hb.npair.p + c, 0, HERMITE_LDS, 0x7fffffff);
+    const ClusterArgs A{d_off + c, nullptr, 1, 0, hb.next.p, hb.edisp.p + c, hb.ncol.p + c, hb.nblock.p + c, hb.npair.p + c};
+    int cls = 0;
+    while (n_c > class_hi(cls, HERMITE_LDS)) cls++;
+    launch_class(cls, P, H, A, 1, 0, 0x7fffffff, st);
     GPLUM_HIP(hipGetLastError());
     return GPLUM_OK;
 }

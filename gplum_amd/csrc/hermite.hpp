@@ -4,10 +4,15 @@
 
 namespace gplum {
 
-constexpr int HERMITE_BLOCK = 64;      // threads per workgroup, clusters up to HARD_SEQ_MAX
-// threads per workgroup (8 waves, two per SIMD) of the larger clusters' kernels
+constexpr int HERMITE_BLOCK = 64;      // threads per workgroup, clusters up to HERMITE_SMALL
+constexpr int HERMITE_SMALL = 16;      // members of the largest cluster one wave integrates
+constexpr int HERMITE_MID = 32;        // members of the largest cluster of the 256-thread kernel
+// threads per workgroup (8 waves, two per SIMD) of the clusters above HARD_SEQ_MAX in LDS and
+// of those in global memory
 constexpr int HERMITE_BIG_BLOCK = 512;
-constexpr int HERMITE_LDS = 256;     // clusters up to this size keep j-data in LDS
+constexpr int HERMITE_GLOBAL_BLOCK = 512;
+constexpr int HERMITE_CLASSES = 5;     // size classes of a batched launch
+constexpr int HERMITE_LDS = 256;       // clusters up to this size are integrated in LDS
 // Clusters up to HARD_SEQ_MAX particles sum each particle's hard force sequentially in
 // j (one lane per particle); larger ones with 64 lane-strided partial sums and a
 // butterfly (all lanes on one particle), an order the oracle reproduces.
@@ -52,6 +57,31 @@ struct HardBuffers {
     }
 };
 
+// Streams of the size classes above the one-wave kernel, so that the classes' longest chains
+// run side by side: fork after the gather on the caller's stream, which waits for the joins.
+struct HardStreams {
+    hipStream_t s[HERMITE_CLASSES - 1] = {};
+    hipEvent_t fork = nullptr, join[HERMITE_CLASSES - 1] = {};
+    HardStreams() = default;
+    HardStreams(const HardStreams &) = delete;
+    HardStreams &operator=(const HardStreams &) = delete;
+    ~HardStreams() {
+        for (hipStream_t q : s)
+            if (q) (void)hipStreamDestroy(q);
+        for (hipEvent_t e : join)
+            if (e) (void)hipEventDestroy(e);
+        if (fork) (void)hipEventDestroy(fork);
+    }
+    // created when first needed (never inside a graph capture: the caller ensures them before)
+    int ensure() {
+        if (fork) return GPLUM_OK;
+        for (hipStream_t &q : s) GPLUM_HIP(hipStreamCreateWithFlags(&q, hipStreamNonBlocking));
+        for (hipEvent_t &e : join) GPLUM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        GPLUM_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
+        return GPLUM_OK;
+    }
+};
+
 struct IsoArgs {
     double *pos, *vel, *acc_d, *jerk_d, *acc_s, *jerk_s, *phi_d, *phi_s, *time, *dt, *acc0;
     const int32_t *number;
@@ -62,19 +92,16 @@ struct IsoArgs {
 // d_off[0..ncl] (local time 0 -> dt_tree; caller sets time = 0).  d_order (optional)
 // gives the processing order (largest first).  persistent: one grid pulling
 // clusters from an atomic queue; otherwise one workgroup per cluster.
-// st2/ev_fork/ev_join (optional): clusters above HARD_SEQ_MAX run on st2 concurrently
-// with the small-cluster kernel on st, and st waits for st2.  wg_per_cu: persistent
-// workgroups per CU; lds_max (<= HERMITE_LDS): the largest cluster whose j-data is
-// staged in LDS (larger ones read it from global memory); clusters above giant_min run
+// hs: streams for the size classes above the one-wave kernel, which st waits for.
+// wg_per_cu: persistent workgroups per CU; lds_max (<= HERMITE_LDS): the largest cluster
+// integrated in LDS (larger ones on the global-memory state); clusters above giant_min run
 // over the whole GPU, several at a time on a stream pool, host-driven (not capturable in
 // a graph).  terms_max: clusters of 2 .. terms_max bodies take the lane-per-term path
-// (0: every cluster up to HARD_SEQ_MAX takes the one-lane-per-particle path).  None of
-// these changes results.
+// (0: every cluster up to HERMITE_SMALL takes the LDS path).  None of these changes results.
 constexpr int GIANT_MIN_DEFAULT = 1024;
 constexpr int GIANT_OFF = 0x7fffffff;
 int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *d_off,
-                const int32_t *d_order, bool persistent, int n_cu, hipStream_t st, hipStream_t st2 = nullptr,
-                hipEvent_t ev_fork = nullptr, hipEvent_t ev_join = nullptr, int wg_per_cu = 8,
+                const int32_t *d_order, bool persistent, int n_cu, hipStream_t st, HardStreams &hs, int wg_per_cu = 8,
                 int lds_max = HERMITE_LDS, int giant_min = GIANT_MIN_DEFAULT, int terms_max = TERMS_MAX);
 // Sun + hard acc/jerk and the initial block step of every cluster particle (as the
 // initial force correction leaves them), for callers that bring bare clusters.

@@ -228,7 +228,6 @@ System::~System() {
     if (log_rem) std::fclose(log_rem);
     if (log_col) std::fclose(log_col);
     if (st) (void)hipStreamDestroy(st);
-    if (st2) (void)hipStreamDestroy(st2);
     if (st_fc) (void)hipStreamSynchronize(st_fc);
     if (st_fc) (void)hipStreamDestroy(st_fc);
     if (st_iso) (void)hipStreamSynchronize(st_iso);
@@ -237,8 +236,6 @@ System::~System() {
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : {ev_fc_ready, ev_fc_done})
         if (e) (void)hipEventDestroy(e);
-    if (ev_fork) (void)hipEventDestroy(ev_fork);
-    if (ev_join) (void)hipEventDestroy(ev_join);
     for (auto &e : ev) if (e) (void)hipEventDestroy(e);
     for (auto &e : evd) if (e) (void)hipEventDestroy(e);
     for (const TimedPair &q : tpend) {
@@ -259,15 +256,12 @@ int System::init_device() {
     GPLUM_HIP(hipGetDeviceProperties(&prop, dev));
     n_cu = prop.multiProcessorCount;
     GPLUM_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    GPLUM_HIP(hipStreamCreateWithFlags(&st2, hipStreamNonBlocking));
     GPLUM_HIP(hipStreamCreateWithFlags(&st_fc, hipStreamNonBlocking));
     GPLUM_HIP(hipStreamCreateWithFlags(&st_iso, hipStreamNonBlocking));
     GPLUM_HIP(hipEventCreateWithFlags(&ev_iso_fork, hipEventDisableTiming));
     GPLUM_HIP(hipEventCreateWithFlags(&ev_iso_join, hipEventDisableTiming));
     GPLUM_HIP(hipEventCreateWithFlags(&ev_fc_ready, hipEventDisableTiming));
     GPLUM_HIP(hipEventCreateWithFlags(&ev_fc_done, hipEventDisableTiming));
-    GPLUM_HIP(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
-    GPLUM_HIP(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
     for (auto &e : ev) GPLUM_HIP(hipEventCreate(&e));
     return GPLUM_OK;
 }
@@ -817,13 +811,12 @@ int System::hard_part(bool persistent) {
         }
         if (persistent) {
             tick(EV_HK0);
-            if ((rc = hard_launch(p, hb, ncl, cl.off.p, cl.order.p, true, n_cu, st, st2, ev_fork, ev_join,
-                                  hard_wg_per_cu, hard_lds_max, hard_giant_min, hard_terms_max)))
+            if ((rc = hard_launch(p, hb, ncl, cl.off.p, cl.order.p, true, n_cu, st, hs, hard_wg_per_cu, hard_lds_max, hard_giant_min, hard_terms_max)))
                 return rc;
             tick(EV_HK1);
         } else {
             // the comparator: one launch per cluster
-            GPLUM_ENSURE(hb.next, 3);
+            GPLUM_ENSURE(hb.next, HERMITE_CLASSES);
             GPLUM_ENSURE(hb.edisp, ncl);
             GPLUM_ENSURE(hb.ncol, ncl);
             GPLUM_ENSURE(hb.nblock, ncl);
@@ -1189,7 +1182,7 @@ int System::hard_trial(int wg_per_cu, int lds_max, double *ms) {
     PartPtrs P = ptrs(A);
     hipLaunchKernelGGL(k_hard_gather, dim3(ceil_div(m, 256)), dim3(256), 0, st, m, cl.index.p, H, P, time_c.p);
     tick(EV_HARD0);
-    if ((rc = hard_launch(p, hb, ncl, cl.off.p, cl.order.p, true, n_cu, st, st2, ev_fork, ev_join, wg_per_cu,
+    if ((rc = hard_launch(p, hb, ncl, cl.off.p, cl.order.p, true, n_cu, st, hs, wg_per_cu,
                           lds_max, hard_giant_min, hard_terms_max)))
         return rc;
     tick(EV_HARD1);

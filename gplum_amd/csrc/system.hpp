@@ -56,8 +56,8 @@ struct Removed {
 
 struct System {
     gplum_params p;
-    hipStream_t st = nullptr, st2 = nullptr;   // st2: large clusters of the hard part
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    hipStream_t st = nullptr;
+    HardStreams hs;                     // the larger clusters of the hard part
     // the forecaster's training runs on st_fc, overlapping the next step's hard part;
     // the next soft force (which rewrites its inputs and reads the network) waits for it
     hipStream_t st_fc = nullptr;

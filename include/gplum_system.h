@@ -151,13 +151,13 @@ typedef struct gplum_tuning {
     int32_t n_group_limit;   /* i-group size of the tree walk                        */
     int32_t soft_tile;       /* j-particles per LDS pass of the FP32 soft kernel      */
     int32_t hard_wg_per_cu;  /* persistent Hermite workgroups per CU                  */
-    int32_t hard_lds_max;    /* clusters up to this size stage their j-data in LDS    */
+    int32_t hard_lds_max;    /* clusters up to this size are integrated in LDS        */
     int32_t hard_giant_min;  /* larger clusters run over the whole GPU (not tuned)    */
     int32_t tree_coop_min;   /* tree nodes of at least this many particles split with a
                                 workgroup-wide search (not tuned; 0 = 65536)          */
     int32_t hard_terms_max;  /* clusters of 2 .. this many (<= 4) bodies spread a block
                                 step over one lane per particle, term and component;
-                                0: one lane per particle (not tuned; same results)   */
+                                0: the larger clusters' path (not tuned; same results) */
     int32_t pad_;
     double soft_ms, hard_ms; /* best measured soft stage / Hermite kernels, ms        */
 } gplum_tuning;
@@ -192,8 +192,8 @@ int gplum_system_put_forecast(gplum_system *s, const float *theta, const float *
  * mode bit 0 set: one persistent batched launch (largest cluster first); clear: one
  * launch per cluster (plain comparator).  mode bit 2 (with bit 0): every cluster above
  * 64 particles runs on the whole-GPU path meant for giant clusters (normally above 1024;
- * same results).  mode bit 3 (with bit 0): clusters of 2 to 4 bodies run one lane per
- * particle instead of one lane per particle, term and component (same results).
+ * same results).  mode bit 3 (with bit 0): clusters of 2 to 4 bodies run the larger clusters'
+ * path in LDS instead of one lane per particle, term and component (same results).
  * mode bit 1 set: the clusters are bare
  * (pos, vel, mass, r_out_inv, acc0, dt only): Sun and hard acc/jerk and the first
  * block step are computed on the device first, as the initial force correction
@@ -268,7 +268,7 @@ int gplum_system_restart_write(gplum_system *s, const char *path, int32_t id_nex
  * `replays` times (no counterpart in the reference; same clusters, results and
  * outputs as mode 1, for callers that replay a fixed batch).  The graph restores the
  * uploaded state, resets the cluster queue with a kernel and launches the size-class
- * kernels on two streams; every replay therefore integrates the same step.  prepare
+ * kernels on a stream each; every replay therefore integrates the same step.  prepare
  * as mode bit 1.  Outputs (each may be null): ms_per_replay (HIP events around each
  * replay, mean), mismatches (replays whose outputs differ bit for bit from the first
  * replay's: 0 expected).  pp receives the first replay's result. */
