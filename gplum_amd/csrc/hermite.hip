@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "hermite.hpp"
@@ -41,14 +42,77 @@ __device__ inline double dmin(double a, double b) { return (b < a) ? b : a; }
 // pair are unchanged.
 constexpr double COL_FILTER = 1.0 + 1e-10;
 
+// ------------------------------------------- square roots and reciprocals together
+//
+// A force term needs sqrt(s) and 1 / sqrt(s), or 1 / s and its square root, each correctly
+// rounded.  One hardware estimate of 1 / sqrt(s) serves both: a Goldschmidt step gives g ~
+// sqrt(s) and h ~ 1 / (2 sqrt(s)) to about 2^-45, and two residual corrections (the residual
+// exact by FMA, the second one the rounding step) give the correctly rounded root, and two
+// Newton steps the correctly rounded reciprocal (Markstein, IBM J. Res. Dev. 34, 1990).  The
+// library's sqrt takes the same corrections after scaling, its division starts over from the
+// estimate of 1 / b; in range there is nothing to scale, and a wave with a value out of range
+// calls the library.  gplum_hermite_dt_selfcheck compares the results with sqrt and 1 / x bit for
+// bit.  sqrt and division in sequence took 92 + 70 cycles of latency (dependent FP64
+// operations 7 cycles, the estimate 18); here 18 + 14 operations.
+
+// s in [2^-400, 2^401): roots and reciprocals are normal and nothing is scaled
+__device__ inline bool root_range(double s) {
+    const unsigned hi = (unsigned)((unsigned long long)__double_as_longlong(s) >> 32);
+    return hi - (623u << 20) < (801u << 20);
+}
+// rcp_fix rounds correctly unless b's mantissa is all ones: a low word of ones (one value in
+// 2^32) goes to the library too
+__device__ inline bool rcp_exception(double b) { return (int)__double_as_longlong(b) == -1; }
+__device__ inline void root_seed(double s, double &g, double &h) {
+    const double y = __builtin_amdgcn_rsq(s);
+    g = s * y;
+    h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(g, r, g);
+}
+// sqrt(x) from g ~ sqrt(x) and h ~ 1 / (2 sqrt(x))
+__device__ inline double root_fix(double x, double g, double h) {
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+// 1 / b from y ~ 1 / b
+__device__ inline double rcp_fix(double b, double y) {
+    y = __builtin_fma(__builtin_fma(-b, y, 1.), y, y);
+    return __builtin_fma(__builtin_fma(-b, y, 1.), y, y);
+}
+// r = sqrt(s) and rinv = 1 / r (need: the values are used; otherwise anything may come back)
+__device__ inline void root_and_inverse(double s, bool need, double &r, double &rinv) {
+    double g, h;
+    root_seed(s, g, h);
+    r = root_fix(s, g, h);
+    rinv = rcp_fix(r, 2. * h);
+    if (__ballot(need && (!root_range(s) || rcp_exception(r)))) {
+        r = sqrt(s);
+        rinv = 1. / r;
+    }
+}
+// sinv = 1 / s and rinv = sqrt(sinv)
+__device__ inline void inverse_and_root(double s, double &sinv, double &rinv) {
+    double g, h;
+    root_seed(s, g, h);
+    const double y = 2. * h;
+    sinv = rcp_fix(s, y * y);
+    rinv = root_fix(sinv, y, 0.5 * g);
+    if (__ballot(!root_range(s) || rcp_exception(s))) {
+        sinv = 1. / s;
+        rinv = sqrt(sinv);
+    }
+}
+
 // ---------------------------------------------------------- Sun gravity
 
 __device__ inline void star_acc_jerk(const HP &P, const double x[3], const double v[3],
                                      double acc[3], double jerk[3], double *phi) {
     const double dr[3] = {-x[0], -x[1], -x[2]};
     const double dv[3] = {-v[0], -v[1], -v[2]};
-    const double r2inv = 1. / (dot3(dr[0], dr[1], dr[2], dr[0], dr[1], dr[2]) + P.eps2_sun);
-    const double rinv = sqrt(r2inv);
+    double r2inv, rinv;
+    inverse_and_root(dot3(dr[0], dr[1], dr[2], dr[0], dr[1], dr[2]) + P.eps2_sun, r2inv, rinv);
     const double r3inv = rinv * r2inv;
     const double mj = P.m_sun * r3inv;
     const double alpha = dot3(dr[0], dr[1], dr[2], dv[0], dv[1], dv[2]) * r2inv;
@@ -164,8 +228,9 @@ __device__ inline double dt_block(const HP &P, double time, double dt, double ac
 
 // Whether d is a power of two (normal, 2^-999 to 2^999): then 1/d, and products with it, are
 // exact.  Every block step is one (dt_tree halved some times).
-__device__ inline bool is_pow2(double d) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(d);
+__host__ __device__ inline bool is_pow2(double d) {
+    unsigned long long b;
+    __builtin_memcpy(&b, &d, sizeof b);
     const unsigned hi = (unsigned)(b >> 32);
     return ((unsigned)b | (hi & 0xFFFFFu)) == 0u && hi - (24u << 20) <= (1998u << 20);
 }
@@ -213,25 +278,42 @@ __device__ inline bool clear_of_steps(double t, double d) {
 
 // ------------------------------------------------------------- hard pair
 
+// K(x) and dK/dr of cutfunc.h with selects (the polynomial evaluated everywhere).
+__device__ inline double cutoff_K_sel(const Cutoff &c, double rij, double r_out_inv) {
+    const double x = (c.gamma - rij * r_out_inv) * c.g_1_inv;
+    const double x2 = x * x;
+    const double p = (((-20. * x + 70.) * x - 84.) * x + 35.) * x2 * x2;
+    return (x < 0.) ? 0. : ((x >= 1.) ? 1. : p);
+}
+__device__ inline double cutoff_dKdt_sel(const Cutoff &c, double rij, double r_out_inv, double alpha) {
+    const double x = (c.gamma - rij * r_out_inv) * c.g_1_inv;
+    const double x_1 = x - 1.;
+    const double d = 140. * x * x * x * x_1 * x_1 * x_1 * r_out_inv * c.g_1_inv;
+    const double dKdr = (x < 0. || x >= 1.) ? 0. : d;
+    return alpha * rij * dKdr;
+}
+
 // gravity_hard.h:219-255: the summands of acc_d, jerk_d (and phi_d) of i from j,
 // returned separately so that several j can be evaluated side by side and added in
-// ascending j afterwards (the sums stay those of a sequential loop).
+// ascending j afterwards (the sums stay those of a sequential loop).  need: the summands are
+// used (the pair of a particle with itself, at distance 0, is evaluated and dropped).
 __device__ inline void pair_term(const HP &P, const double xi[3], const double vi[3], double rinv_i,
                                  double xj0, double xj1, double xj2, double vj0, double vj1, double vj2,
-                                 double mj, double rinv_j, double ta[3], double tj[3], double *tphi) {
+                                 double mj, double rinv_j, double ta[3], double tj[3], double *tphi,
+                                 bool need = true) {
     const double dr[3] = {xj0 - xi[0], xj1 - xi[1], xj2 - xi[2]};
     double dr2 = dot3(dr[0], dr[1], dr[2], dr[0], dr[1], dr[2]);
     dr2 += P.eps2;
     const double dv[3] = {vj0 - vi[0], vj1 - vi[1], vj2 - vi[2]};
-    const double rij = sqrt(dr2);
-    const double rinv = 1. / rij;
+    double rij, rinv;
+    root_and_inverse(dr2, need, rij, rinv);
     const double r2inv = rinv * rinv;
     const double r3inv = r2inv * rinv;
     const double r_out_inv = dmin(rinv_i, rinv_j);
     const double mj_rij3 = mj * r3inv;
     const double alpha = dot3(dr[0], dr[1], dr[2], dv[0], dv[1], dv[2]) * r2inv;
-    const double _K = 1. - cutoff_K(P.cut, rij, r_out_inv);
-    const double dKdt = cutoff_dKdt(P.cut, rij, r_out_inv, alpha);
+    const double _K = 1. - cutoff_K_sel(P.cut, rij, r_out_inv);
+    const double dKdt = cutoff_dKdt_sel(P.cut, rij, r_out_inv, alpha);
     const double alpha_c = alpha * _K;
     if (tphi) {
         const double _W = 1. - cutoff_W(P.cut, rij, r_out_inv);
@@ -289,9 +371,9 @@ struct JData {
 constexpr int HARD_ILP = 4;
 
 __device__ inline void pair_term_j(const HP &P, const JData &J, int j, const double xi[3], const double vi[3],
-                                   double rinv_i, double ta[3], double tj[3], double *tphi) {
+                                   double rinv_i, double ta[3], double tj[3], double *tphi, bool need = true) {
     pair_term(P, xi, vi, rinv_i, J.x[3 * j], J.x[3 * j + 1], J.x[3 * j + 2], J.v[3 * j], J.v[3 * j + 1],
-              J.v[3 * j + 2], J.m[j], J.ri[j], ta, tj, tphi);
+              J.v[3 * j + 2], J.m[j], J.ri[j], ta, tj, tphi, need);
 }
 
 // Sum over j = j0, j0 + s, j0 + 2s, ... < n (j != i by id) in ascending j, ILP pairs
@@ -304,11 +386,15 @@ __device__ inline void pair_sum_strided(const HP &P, const JData &J, int j0, int
     int j = j0;
     for (; j + (ILP - 1) * s < n; j += ILP * s) {
         double ta[ILP][3], tj[ILP][3], tp[ILP];
-#pragma unroll
-        for (int u = 0; u < ILP; u++) pair_term_j(P, J, j + u * s, xi, vi, rinv_i, ta[u], tj[u], phi ? &tp[u] : nullptr);
+        bool use[ILP];
 #pragma unroll
         for (int u = 0; u < ILP; u++) {
-            if (J.id[j + u * s] == idi) continue;
+            use[u] = J.id[j + u * s] != idi;
+            pair_term_j(P, J, j + u * s, xi, vi, rinv_i, ta[u], tj[u], phi ? &tp[u] : nullptr, use[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < ILP; u++) {
+            if (!use[u]) continue;
             for (int k = 0; k < 3; k++) { acc[k] += ta[u][k]; jerk[k] += tj[u][k]; }
             if (phi) *phi -= tp[u];
         }
@@ -977,43 +1063,63 @@ __device__ inline void rows_of(double x, double (&r)[4]) {
     }
 }
 
-// K(x) and dK/dr of cutfunc.h with selects (the polynomial evaluated everywhere).
-__device__ inline double cutoff_K_sel(const Cutoff &c, double rij, double r_out_inv) {
-    const double x = (c.gamma - rij * r_out_inv) * c.g_1_inv;
-    const double x2 = x * x;
-    const double p = (((-20. * x + 70.) * x - 84.) * x + 35.) * x2 * x2;
-    return (x < 0.) ? 0. : ((x >= 1.) ? 1. : p);
-}
-__device__ inline double cutoff_dKdt_sel(const Cutoff &c, double rij, double r_out_inv, double alpha) {
-    const double x = (c.gamma - rij * r_out_inv) * c.g_1_inv;
-    const double x_1 = x - 1.;
-    const double d = 140. * x * x * x * x_1 * x_1 * x_1 * r_out_inv * c.g_1_inv;
-    const double dKdr = (x < 0. || x >= 1.) ? 0. : d;
-    return alpha * rij * dKdr;
-}
+// Constants of the lane-per-term path.  They are kept in vector registers (the kernel has
+// plenty and this path uses few): as scalars the compiler spills and reloads some of them in
+// every block step.
+struct TermConsts {
+    double gamma, g_1_inv, c140, c70, c84, c35, half_tree, dt_min, alpha2;
+    __device__ explicit TermConsts(const HP &P)
+        : gamma(P.cut.gamma), g_1_inv(P.cut.g_1_inv), c140(140.), c70(70.), c84(84.), c35(35.),
+          half_tree(0.5 * P.dt_tree), dt_min(P.dt_min), alpha2(P.alpha2) {
+        asm("" : "+v"(gamma), "+v"(g_1_inv), "+v"(c140), "+v"(c70), "+v"(c84));
+        asm("" : "+v"(c35), "+v"(half_tree), "+v"(dt_min), "+v"(alpha2));
+    }
+};
 
 // The lane's term of a hard force evaluation, in one instruction stream for the Sun row
 // (star_acc_jerk: xj = vj = -0, so that xj - x = -x exactly; mT = m_sun, eps2T =
 // eps2_sun) and the partner rows (pair_term with r_out_inv = min of the two 1/r_out):
 // the Sun's (1/s, then sqrt) and the pair's (sqrt, then 1/r) sequences are both
-// evaluated and the row's own one selected; the Sun row takes K = 1 and dK/dt = -0,
-// exact identities (1 K = K, alpha 1 = alpha, 3 alpha + (-0) = 3 alpha) that leave
-// star_acc_jerk's acc = mj dr and jerk = mj (dv - 3 alpha dr).
-__device__ inline void term_eval(const Cutoff &cut, bool sun, bool pad, double xi, double vi, double xj, double vj,
-                                 double mT, double eps2T, double r_out_inv, double &ta, double &tj) {
+// evaluated from one estimate and the row's own one selected.  The Sun row's r_out_inv =
+// SUN_R_OUT_INV puts it below the changeover (x < 0), so K = 1 and dK/dt is a zero of
+// alpha's sign: exact identities (1 K = K, alpha 1 = alpha, 3 alpha + 0 = 3 alpha) that leave
+// star_acc_jerk's acc = mj dr and jerk = mj (dv - 3 alpha dr).  need: the lane's term is used.
+constexpr double SUN_R_OUT_INV = -1e300;
+__device__ inline void term_eval(const TermConsts &C, bool sun, bool pad, bool need, double xi, double vi, double xj,
+                                 double vj, double mT, double eps2T, double r_out_inv, double &ta, double &tj) {
     const double dr = xj - xi;
     const double dv = vj - vi;
     const double s = quad_sq(dr) + eps2T;
-    const double a = 1. / s, b = sqrt(s);
-    const double y1 = sun ? a : b;                 // Sun: 1/r^2; pair: r
-    const double c = sqrt(y1), d = 1. / y1;
-    const double rinv = sun ? c : d;
-    const double r2inv = sun ? y1 : d * d;
+    // y1: the Sun's 1/r^2, the pair's r
+    double y1, rinv, r2inv;
+    {
+        double g, h;
+        root_seed(s, g, h);
+        const double y = 2. * h;
+        const double a = rcp_fix(s, y * y), b = root_fix(s, g, h);
+        const double c = root_fix(a, y, 0.5 * g), d = rcp_fix(b, y);
+        y1 = sun ? a : b;
+        rinv = sun ? c : d;
+        r2inv = sun ? a : d * d;
+    }
+    if (__ballot(need && (!root_range(s) || rcp_exception(sun ? s : y1)))) {
+        const double a = 1. / s, b = sqrt(s);
+        y1 = sun ? a : b;
+        const double c = sqrt(y1), d = 1. / y1;
+        rinv = sun ? c : d;
+        r2inv = sun ? y1 : d * d;
+    }
     const double r3inv = r2inv * rinv;
     const double mj_r3 = mT * r3inv;
     const double alpha = quad_dot(dr, dv, pad) * r2inv;
-    const double K = sun ? 1. : 1. - cutoff_K_sel(cut, y1, r_out_inv);
-    const double dKdt = sun ? -0. : cutoff_dKdt_sel(cut, y1, r_out_inv, alpha);
+    // cutoff_K_sel and cutoff_dKdt_sel
+    const double x = (C.gamma - y1 * r_out_inv) * C.g_1_inv;
+    const double x2 = x * x, x_1 = x - 1.;
+    const double poly = (((-20. * x + C.c70) * x - C.c84) * x + C.c35) * x2 * x2;
+    const double slope = C.c140 * x * x * x * x_1 * x_1 * x_1 * r_out_inv * C.g_1_inv;
+    const bool below = x < 0., above = x >= 1.;
+    const double K = 1. - (below ? 0. : (above ? 1. : poly));
+    const double dKdt = alpha * y1 * ((below || above) ? 0. : slope);
     const double alpha_c = alpha * K;
     const double c2 = 3. * alpha_c + dKdt;
     ta = mj_r3 * K * dr;
@@ -1070,7 +1176,8 @@ __device__ inline void correct_one(double Dt, double Dt2, double Dt_inv2, double
     vel = vp + ONE_TWELFTH * Dt * (4. * A2_sd + 3. * A3_sd);
 }
 
-// calc_dt4_fast and calc_dt4 of the lane's term (the row's vectors, dots over the quad).
+// calc_dt4_fast and calc_dt4 of the lane's term (the row's vectors, dots over the quad).  The
+// fast one gives NaN whenever a product is not normal.
 __device__ inline double dt4_fast_quad(double eta, double alpha2, double acc0, double a, double j, double s,
                                        double c) {
     const double Acc2 = quad_sq(a) + alpha2 * acc0 * acc0;
@@ -1078,11 +1185,10 @@ __device__ inline double dt4_fast_quad(double eta, double alpha2, double acc0, d
     const double Snap2 = quad_sq(s);
     const double Crac2 = quad_sq(c);
     const double as2 = Acc2 * Snap2, jc2 = Jerk2 * Crac2;
-    const bool ok = (as2 >= DBL_MIN || (Acc2 == 0. || Snap2 == 0.)) && (jc2 >= DBL_MIN || Crac2 == 0.);
     const double num = __builtin_amdgcn_sqrt(as2) + Jerk2;
     const double den = __builtin_amdgcn_sqrt(jc2) + Snap2;
-    const double q = ok ? eta * __builtin_amdgcn_sqrt(num * __builtin_amdgcn_rcp(den)) : __builtin_nan("");
-    return (Jerk2 > 0.) ? q : DBL_MAX;
+    const double q = eta * __builtin_amdgcn_sqrt(num * __builtin_amdgcn_rcp(den));
+    return (Jerk2 > 0.) ? (__builtin_fmin(as2, jc2) >= DBL_MIN ? q : __builtin_nan("")) : DBL_MAX;
 }
 __device__ inline double dt4_quad(double eta, double alpha2, double acc0, double a, double j, double s, double c) {
     const double Acc = sqrt(quad_sq(a) + alpha2 * acc0 * acc0);
@@ -1093,12 +1199,6 @@ __device__ inline double dt4_quad(double eta, double alpha2, double acc0, double
     const double Crac = sqrt(quad_sq(c));
     return (Jerk > 0.) ? eta * sqrt((Acc * Snap + Jerk2) / (Jerk * Crac + Snap2)) : DBL_MAX;
 }
-
-// Physics constants of the lane-per-term path, in registers (the kernel keeps HP in LDS).
-struct TermConsts {
-    Cutoff cut;
-    double dt_tree, dt_min, alpha2;
-};
 
 // the Sun row's and the first partner row's values of the lane's position
 template <int N>
@@ -1115,33 +1215,61 @@ __device__ inline void sun_planet_of(double x, double &f_sun, double &f_planet) 
 // dt_block with the Sun criterion from the Sun row and the planet criterion from the
 // partner rows (each lane evaluates its own row's, reads the other by a lane swap); the
 // exact criteria when either fast one is not finite or dt_1 lies near the step grid.
-template <int N>
+// DYADIC: the cluster's steps, dt_tree and dt_min are powers of two and its
+// times whole multiples of its steps (dyadic_steps), so the largest step that divides time is
+// min(2 dt, dt_tree / 2) or dt, the halvings end at min(that, max(the power of two at or below
+// dt_1, dt / 2)), and a step below 2 dt_min is at most dt_min.
+__device__ inline double hi_word(int hi) { return __longlong_as_double((long long)((unsigned long long)(unsigned)hi << 32)); }
+__device__ inline int hi_of(double d) { return (int)(__double_as_longlong(d) >> 32); }
+template <int N, bool DYADIC>
 __device__ inline double dt_block_rows(const TermConsts &C, double time, double dt, double etaT, double acc0T,
                                        double a, double j, double s, double c) {
-    double dt_next = dmin(2. * dt, 0.5 * C.dt_tree);
-    double rem = fmod_block(time, dt_next);
-    for (int it = 0; rem != 0.0 && it < HALVE_CAP; it++) { dt_next *= 0.5; rem = fmod_block(time, dt_next); }
+    const double dt_max = __builtin_fmin(2. * dt, C.half_tree);
+    double dt_0;
+    bool cap = false;
+    if (DYADIC) {
+        const double q = time * hi_word(0x7FE00000 - hi_of(dt_max));
+        dt_0 = (q == floor(q)) ? dt_max : dt;
+    } else {
+        dt_0 = dt_candidate(time, dt_max, cap);
+    }
     double f_sun, f_planet;
     sun_planet_of<N>(dt4_fast_quad(etaT, C.alpha2, acc0T, a, j, s, c), f_sun, f_planet);
     double dt_1 = dmin(f_planet, f_sun);
-    const bool exact = !(f_planet <= DBL_MAX && f_sun <= DBL_MAX) || !clear_of_grid(dt_1, dt_next);
+    const unsigned hi = (unsigned)hi_of(dt_1);
+    bool clear = (hi & 0xFFFFFu) - 1025u < 0x100000u - 2049u - 1025u && hi - (24u << 20) <= (1998u << 20);
+    if (!DYADIC) clear = clear_of_grid(dt_1, dt_0);
+    const bool exact = !(f_planet <= DBL_MAX && f_sun <= DBL_MAX && clear);
     if (__ballot(exact)) {
         double e_sun, e_planet;
         sun_planet_of<N>(dt4_quad(etaT, C.alpha2, acc0T, a, j, s, c), e_sun, e_planet);
         if (exact) dt_1 = dmin(e_planet, e_sun);
     }
-    for (int it = 0; dt_1 < dt_next && 0.5 * dt < dt_next && it < HALVE_CAP; it++) dt_next *= 0.5;
-    if (dt_next < 2. * C.dt_min) dt_next = C.dt_min;
-    return (rem != 0.0) ? C.dt_min : dt_next;
+    if (!DYADIC) {
+        const double d = dt_reduce(dt_0, dt_1, dt);
+        return (cap || d < 2. * C.dt_min) ? C.dt_min : d;
+    }
+    const double low = __builtin_fmax(hi_word(hi_of(dt_1) & 0x7FF00000), 0.5 * dt);
+    return __builtin_fmax(__builtin_fmin(dt_0, low), C.dt_min);
 }
 
-// Block steps of a cluster of N (2 to 4) particles with distinct ids from the start of
-// the soft step (the layout above; one wave).  Returns false when a block step has a
-// collision: the state of the start of that block step is then in H (flags and twins
-// cleared) for integrate_from.  Else the final calcGravity with potentials is done and
+// Whether a particle's starting state keeps to dt_block_rows' dyadic rule, dt_tree and dt_min
+// being powers of two no more than 2^50 apart (dyadic_tree).
+__device__ inline bool dyadic_steps(const HP &P, double time, double dt) {
+    const double q = time * pow2_inverse(dt);
+    return is_pow2(dt) && dt >= P.dt_min && time >= 0. && time <= P.dt_tree && q == floor(q);
+}
+static bool dyadic_tree(const gplum_params &p) {
+    return is_pow2(p.dt_tree) && is_pow2(p.dt_min) && p.dt_min <= 0.5 * p.dt_tree && p.dt_min >= 0x1p-50 * p.dt_tree;
+}
+
+// Block steps of a cluster of N (2 to 4) particles with distinct ids from the start of the
+// soft step (the layout above; one wave; DYADIC: all of them keep to dyadic_steps).  Returns false when a block step
+// may have a collision: the state of the start of that block step is then in H (flags and twins
+// cleared) for integrate_seq.  Else the final calcGravity with potentials is done and
 // written to H.  s_m, s_ri, s_id, s_fr hold the cluster's masses, 1/r_out, ids and
 // f r_planet; s_x, s_v and s_tm are free.
-template <int N>
+template <int N, bool DYADIC>
 __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double *s_x, double *s_v, double *s_m,
                                 double *s_ri, int64_t *s_id, double *s_fr, double *s_tm, int b, double &sys_time,
                                 long long &loop, long long &pairs) {
@@ -1159,10 +1287,10 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
     const int j = (T >= 1) ? (T - 1) + ((T - 1) >= p ? 1 : 0) : p;   // the row's partner
     const int jc = (j < N) ? j : 0, pc = own ? p : 0;
     const int g = b + pc;
-    const TermConsts C{P.cut, P.dt_tree, P.dt_min, P.alpha2};
+    const TermConsts C(P);
     const double mT = sun ? P.m_sun : s_m[jc];
     const double eps2T = sun ? P.eps2_sun : P.eps2;
-    const double r_out_inv = dmin(s_ri[pc], s_ri[jc]);
+    const double r_out_inv = sun ? SUN_R_OUT_INV : dmin(s_ri[pc], s_ri[jc]);
     const double etaT = sun ? P.eta_sun : P.eta;
     const double r2c = s_fr[pc] + s_fr[jc];
     const double col_thr = COL_FILTER * r2c * r2c;
@@ -1188,14 +1316,17 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
         if (sun) { xj = -0.; vj = -0.; }
         if (own) {
             double ta, tj;
-            term_eval(C.cut, sun, pad, x, v, xj, vj, mT, eps2T, r_out_inv, ta, tj);
+            term_eval(C, sun, pad, row, x, v, xj, vj, mT, eps2T, r_out_inv, ta, tj);
             gather_terms<N>(ta, tj, as, js, ad, jd);
         }
     }
-    double tn = own ? time + dt : 1.e10;
-    tn = dmin(tn, dpp_f64<DPP_ROW_ROR4>(tn));
-    tn = dmin(tn, dpp_f64<DPP_ROW_ROR8>(tn));
-    double t_s = readlane_f64(tn, 0);
+    // the smallest value of the particles (quads of a row; 2 bodies: quads 2, 3 are copies)
+    auto smallest = [](double u) __attribute__((always_inline)) {
+        u = __builtin_fmin(u, dpp_f64<DPP_ROW_ROR4>(u));
+        if (N > 2) u = __builtin_fmin(u, dpp_f64<DPP_ROW_ROR8>(u));
+        return readlane_f64(u, 0);
+    };
+    double t_s = smallest(own ? time + dt : 1.e10);
     bool handover = false;
     while (sys_time < time_end && loop < BLOCK_STEP_CAP) {
         const double Dt = t_s - time;
@@ -1217,43 +1348,36 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
             // collisionDetermination: a pair with R = |dx| / (f_i R_i + f_j R_j) < 1
             const double dx = xp - xj;
             const double d2 = quad_sq(dx);
-            const bool near = col_row && d2 < col_thr;
-            if (__ballot(near)) {
-                const bool hit = near && sqrt(d2) / r2c < 1.;
-                if (__ballot(hit)) { handover = true; break; }
-            }
+            if (__ballot(col_row && d2 < col_thr)) { handover = true; break; }   // R itself is left to integrate_seq
         }
         if (own && time + dt == t_s) {
             if (lead) pairs += 3 * (long long)m;
             const double Dt2 = Dt * Dt;
-            const double Dt_inv = recip_block(Dt);
+            // DYADIC: Dt = dt, a power of two
+            const double Dt_inv = DYADIC ? hi_word(0x7FE00000 - hi_of(Dt)) : recip_step(Dt);
             const double Dt_inv2 = Dt_inv * Dt_inv;
             const double Dt_inv3 = Dt_inv2 * Dt_inv;
             double ta, tj;
-            term_eval(C.cut, sun, pad, xp, vp, xj, vj, mT, eps2T, r_out_inv, ta, tj);
+            term_eval(C, sun, pad, row, xp, vp, xj, vj, mT, eps2T, r_out_inv, ta, tj);
             gather_terms<N>(ta, tj, as, js, ad, jd);
             for (int ite = 0; ite < 2; ite++) {
                 correct_one(Dt, Dt2, Dt_inv2, Dt_inv3, xp, vp, as, a0s, j0s, js, ad, a0d, j0d, jd, x, v, a2s, a3s,
                             a2d, a3d);
-                term_eval(C.cut, sun, pad, x, v, xj, vj, mT, eps2T, r_out_inv, ta, tj);
+                term_eval(C, sun, pad, row, x, v, xj, vj, mT, eps2T, r_out_inv, ta, tj);
                 gather_terms<N>(ta, tj, as, js, ad, jd);
             }
             time += Dt;
-            dt = dt_block_rows<N>(C, time, dt, etaT, acc0T, sun ? as : ad, sun ? js : jd, sun ? a2s : a2d,
+            dt = dt_block_rows<N, DYADIC>(C, time, dt, etaT, acc0T, sun ? as : ad, sun ? js : jd, sun ? a2s : a2d,
                                   sun ? a3s : a3d);
         }
-        double tm = own ? time : 1.e10;
-        tn = own ? time + dt : 1.e10;
-        tm = dmin(tm, dpp_f64<DPP_ROW_ROR4>(tm));
-        tn = dmin(tn, dpp_f64<DPP_ROW_ROR4>(tn));
-        tm = dmin(tm, dpp_f64<DPP_ROW_ROR8>(tm));
-        tn = dmin(tn, dpp_f64<DPP_ROW_ROR8>(tn));
-        sys_time = readlane_f64(tm, 0);
-        t_s = readlane_f64(tn, 0);
+        // the system time is asked for once the next block time has reached the end: before
+        // that some particle's time is below it
+        t_s = smallest(own ? time + dt : 1.e10);
+        if (!(t_s < time_end)) sys_time = smallest(own ? time : 1.e10);
         loop++;
     }
     if (handover) {
-        // the state at the start of this block step, for integrate_from
+        // the state at the start of this block step, for integrate_seq
         if (row && sun && !pad && first) {
             H.pos[3 * g + c] = x; H.vel[3 * g + c] = v;
             H.acc_s[3 * g + c] = as; H.jerk_s[3 * g + c] = js;
@@ -1350,7 +1474,9 @@ __device__ __forceinline__ void cluster_queue(const HP &P, const ClusterArgs &A,
 // Clusters of up to HERMITE_SMALL members, one wave each: 2 to terms_max bodies with a lane
 // per term (a collision hands over to the LDS path in the middle of the soft step), the
 // others on the LDS path.  The arguments are read from LDS: in scalar registers they would
-// be spilled and reloaded in the block-step loop.
+// be spilled and reloaded in the block-step loop.  DYADIC: dyadic_tree's parameters, as in
+// every ordinary run; a cluster whose own steps are not powers of two then takes the LDS path.
+template <bool DYADIC>
 __global__ __launch_bounds__(HERMITE_BLOCK) void k_hermite_small(HP P_arg, HardView H_arg, ClusterArgs A_arg, int lo,
                                                                  int hi) {
     __shared__ HP P;
@@ -1379,16 +1505,21 @@ __global__ __launch_bounds__(HERMITE_BLOCK) void k_hermite_small(HP P_arg, HardV
             __syncthreads();
             // the clusters the reference forms have distinct ids, and the lane-per-term path
             // leaves the id test out
-            bool rep = false;
-            if (t < n)
-                for (int j = 0; j < n; j++) rep = rep || (j != t && C.id[j] == C.id[t]);
-            if (__ballot(rep) == 0) {
+            bool other = false;
+            if (t < n) {
+                other = DYADIC && !dyadic_steps(P, H.time[b + t], H.dt[b + t]);
+                for (int j = 0; j < n; j++) other = other || (j != t && C.id[j] == C.id[t]);
+            }
+            if (__ballot(other) == 0) {
                 const JData J{C.xp, C.vp, C.mass, C.rinv, C.id, 3};
                 double *tm = reinterpret_cast<double *>(s_term);
-                const bool done =
-                    (n == 2)   ? integrate_terms<2>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b, sys_time, loop, pairs)
-                    : (n == 3) ? integrate_terms<3>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b, sys_time, loop, pairs)
-                               : integrate_terms<4>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b, sys_time, loop, pairs);
+                auto terms = [&](auto N) {
+                    return integrate_terms<N.value, DYADIC>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b, sys_time,
+                                                            loop, pairs);
+                };
+                const bool done = (n == 2)   ? terms(std::integral_constant<int, 2>())
+                                  : (n == 3) ? terms(std::integral_constant<int, 3>())
+                                             : terms(std::integral_constant<int, 4>());
                 if (done) return;
                 fresh = false;
                 __threadfence_block();
@@ -2028,10 +2159,13 @@ static int class_hi(int cls, int lds_max) {
     return cls == 0 ? HERMITE_SMALL : cls == 1 ? HERMITE_MID : cls == 2 ? HARD_SEQ_MAX : cls == 3 ? lds_max : 0x7fffffff;
 }
 static int class_lo(int cls, int lds_max) { return cls == 0 ? 0 : class_hi(cls - 1, lds_max); }
-static void launch_class(int cls, const HP &P, const HardView &H, const ClusterArgs &A, int grid, int lo, int hi,
+static void launch_class(int cls, bool dyadic, const HP &P, const HardView &H, const ClusterArgs &A, int grid, int lo, int hi,
                          hipStream_t st) {
     switch (cls) {
-    case 0: hipLaunchKernelGGL(k_hermite_small, dim3(grid), dim3(HERMITE_BLOCK), 0, st, P, H, A, lo, hi); break;
+    case 0:
+        if (dyadic) hipLaunchKernelGGL(k_hermite_small<true>, dim3(grid), dim3(HERMITE_BLOCK), 0, st, P, H, A, lo, hi);
+        else hipLaunchKernelGGL(k_hermite_small<false>, dim3(grid), dim3(HERMITE_BLOCK), 0, st, P, H, A, lo, hi);
+        break;
     case 1: hipLaunchKernelGGL((k_hermite_mid<HERMITE_SMALL + 1, HERMITE_MID, 256>), dim3(grid), dim3(256), 0, st, P, H, A, lo, hi); break;
     case 2: hipLaunchKernelGGL((k_hermite_mid<HERMITE_MID + 1, HARD_SEQ_MAX, 512>), dim3(grid), dim3(512), 0, st, P, H, A, lo, hi); break;
     case 3: hipLaunchKernelGGL(k_hermite_big, dim3(grid), dim3(HERMITE_BIG_BLOCK), 0, st, P, H, A, lo, hi); break;
@@ -2052,6 +2186,7 @@ int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *
     if (ncl <= 0) return GPLUM_OK;
     HP P = make_hp(p);
     P.terms_max = std::max(0, std::min(TERMS_MAX, terms_max));
+    const bool dyadic = dyadic_tree(p);
     HardView H = hard_view(hb);
     GPLUM_ENSURE(hb.next, HERMITE_CLASSES);
     GPLUM_ENSURE(hb.edisp, ncl);
@@ -2083,7 +2218,7 @@ int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *
         if (cls > 0 && (hb.max_size <= lo || hi <= lo)) continue;
         A.next = hb.next.p + cls;
         if (cls > 0) GPLUM_HIP(hipStreamWaitEvent(hs.s[cls - 1], hs.fork, 0));
-        launch_class(cls, P, H, A, grid, lo, hi, cls > 0 ? hs.s[cls - 1] : st);
+        launch_class(cls, dyadic, P, H, A, grid, lo, hi, cls > 0 ? hs.s[cls - 1] : st);
         if (cls > 0) GPLUM_HIP(hipEventRecord(hs.join[cls - 1], hs.s[cls - 1]));
         launched[cls] = true;
     }
@@ -2145,7 +2280,7 @@ int hard_launch_single(const gplum_params &p, HardBuffers &hb, int c, int n_c, c
     const ClusterArgs A{d_off + c, nullptr, 1, 0, hb.next.p, hb.edisp.p + c, hb.ncol.p + c, hb.nblock.p + c, hb.npair.p + c};
     int cls = 0;
     while (n_c > class_hi(cls, HERMITE_LDS)) cls++;
-    launch_class(cls, P, H, A, 1, 0, 0x7fffffff, st);
+    launch_class(cls, dyadic_tree(p), P, H, A, 1, 0, 0x7fffffff, st);
     GPLUM_HIP(hipGetLastError());
     return GPLUM_OK;
 }
@@ -2182,7 +2317,7 @@ __device__ inline double rnd_mag(uint64_t &st, int e0, int e1) {
 // the step's grid.  One sample in four widens every magnitude by 2^+-540, so that the
 // products of squares in the fast criterion underflow below DBL_MIN or overflow past
 // DBL_MAX.  Counts results that differ in any bit and fast values sent to the exact
-// evaluation.
+// evaluation; the pairs of roots and reciprocals are compared as well.
 __global__ void k_dt_selfcheck(HP P, long long n, uint64_t seed, unsigned long long *out) {
     unsigned long long mism = 0, fb = 0;
     for (long long s = blockIdx.x * (long long)blockDim.x + threadIdx.x; s < n; s += (long long)gridDim.x * blockDim.x) {
@@ -2204,6 +2339,23 @@ __global__ void k_dt_selfcheck(HP P, long long n, uint64_t seed, unsigned long l
         const double b = dt_block<false>(P, time + dt, dt, acc0, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]);
         mism += (__double_as_longlong(a) != __double_as_longlong(b)) ? 1 : 0;
         fb += fell;
+        // the roots and reciprocals of the force terms: random mantissas, and those next to a
+        // power of two or to a square, where a rounding is closest
+        st += 0x9E3779B97F4A7C15ULL;
+        const uint64_t u = mix64(st);
+        double x = fabs(rnd_mag(st, -420, 420));
+        const uint64_t ulps = u >> 58;
+        if ((u & 3) == 1) x = ldexp(1.0, (int)(u >> 8 & 511) - 256) * (1.0 + ((u & 4) ? 1. : -0.5) * 0x1p-52 * (double)ulps);
+        if ((u & 3) == 2) {
+            const double q = fabs(rnd_mag(st, -200, 200));
+            x = __longlong_as_double(__double_as_longlong(q * q) + (long long)ulps - 32);
+        }
+        double rt, rtinv, sinv, root;
+        root_and_inverse(x, true, rt, rtinv);
+        inverse_and_root(x, sinv, root);
+        const double r0 = sqrt(x), s0 = 1. / x;
+        mism += (__double_as_longlong(rt) != __double_as_longlong(r0)) + (__double_as_longlong(rtinv) != __double_as_longlong(1. / r0)) +
+                (__double_as_longlong(sinv) != __double_as_longlong(s0)) + (__double_as_longlong(root) != __double_as_longlong(sqrt(s0)));
     }
     atomicAdd(&out[0], mism);
     atomicAdd(&out[1], fb);

@@ -47,8 +47,8 @@ struct ClusterLds {
 // star_acc_jerk of a quad's particle, one component per lane (see quad_sum).
 __device__ inline void star_quad(const HP &P, double x, double v, bool pad, double &as, double &js) {
     const double dr = -x, dv = -v;
-    const double r2inv = 1. / (quad_sq(dr) + P.eps2_sun);
-    const double rinv = sqrt(r2inv);
+    double r2inv, rinv;
+    inverse_and_root(quad_sq(dr) + P.eps2_sun, r2inv, rinv);
     const double r3inv = rinv * r2inv;
     const double mj = P.m_sun * r3inv;
     const double alpha = quad_dot(dr, dv, pad) * r2inv;
@@ -340,7 +340,8 @@ __device__ inline void lds_pair_terms(const HP &P, const ClusterLds<NMAX> &C, do
     const double *pv = first ? C.vp + 3 * B.bd : C.bv + 3 * B.slot;
     const double xi[3] = {px[0], px[1], px[2]}, vi[3] = {pv[0], pv[1], pv[2]};
     double ta[3], tj[3];
-    pair_term(P, xi, vi, B.rinv, xj[0], xj[1], xj[2], vj[0], vj[1], vj[2], mj, rj, ta, tj, nullptr);
+    pair_term(P, xi, vi, B.rinv, xj[0], xj[1], xj[2], vj[0], vj[1], vj[2], mj, rj, ta, tj, nullptr,
+              B.tv && B.use);
     if (B.tv)
         for (int d = 0; d < 3; d++) s_term[d * TP + row] = make_double2(B.use ? ta[d] : 0., B.use ? tj[d] : 0.);
 }
@@ -622,8 +623,8 @@ __device__ void integrate_tree(const HP &P, ClusterLds<NMAX> &C, TreeLds<NMAX> &
 #pragma unroll
                     for (int u = 0; u < 2; u++) {
                         const int j = min(j0 + 64 * u + lane, n - 1);
-                        pair_term_j(P, J, j, xi, vi, rinv, ta[u], tj[u], nullptr);
                         use[u] = j0 + 64 * u + lane < n && C.id[j] != id;
+                        pair_term_j(P, J, j, xi, vi, rinv, ta[u], tj[u], nullptr, use[u]);
                     }
 #pragma unroll
                     for (int u = 0; u < 2; u++)

@@ -45,3 +45,20 @@ def test_size_classes_match_oracle(oracle_lib, sizes, merging):
     assert steps_g == steps and ed_g == ed
     assert np.allclose(got["phi_d"], ref["phi_d"], rtol=1e-13, atol=0.0)
     assert not merging or nc > 0
+
+
+@pytest.mark.parametrize("merging", [False, True])
+@pytest.mark.parametrize("dt_tree,dt_scale", [(2.0 ** -4, 1.0), (2.0 ** -4, 0.75), (3 * 2.0 ** -6, 1.0), (3 * 2.0 ** -6, 2.0 / 3)])
+def test_step_grids_match_oracle(oracle_lib, dt_tree, dt_scale, merging):
+    # steps that are powers of two and steps that are not (of a dt_tree that is none, or given)
+    kw = dict(eta=0.01, eta_sun=0.01, eta_0=0.002, eta_sun0=0.002, dt_tree=dt_tree, dt_min=dt_tree * 2.0 ** -9, gamma=0.1,
+              collision=int(merging))
+    pp, off = clusters_of((2, 3, 4, 5) * 8, 57, 1e-8 if merging else 1e-9, 100.0 if merging else 1.0)
+    oracle_lib.cluster_prepare(oracle_lib.params(**kw), pp, off)
+    pp["dt"] *= dt_scale
+    ref, got = pp.copy(), pp.copy()
+    nc, ed, steps = oracle_lib.hermite_clusters(oracle_lib.params(**kw), ref, off)
+    ed_g, steps_g, _ = gpu.hard_integrate(gpu.params(**kw), got, off)
+    print("%d block steps (oracle %d), %d collisions" % (steps_g, steps, nc))
+    assert [f for f in FIELDS if got[f].tobytes() != ref[f].tobytes()] == []
+    assert steps_g == steps and ed_g == ed
