@@ -22,7 +22,7 @@
 #include <mutex>
 #include <vector>
 
-#include "soft_kernels.hpp"
+#include "soft_direct.hpp"
 
 namespace gplum {
 namespace {
@@ -59,7 +59,7 @@ struct TagCtx {
     Pinned h_in, h_force;
     Dev d_in, d_force;
     std::vector<int> i_off;      // per walk, into the packed i array
-    int n_walk = 0, ni_total = 0;
+    int n_walk = 0, ni_total = 0, i_lanes = 0;
     bool pending = false;
 };
 
@@ -108,17 +108,24 @@ int begin_dispatch(int tag, int n_walk, const void *epi, const int *n_epi, const
     return GPLUM_OK;
 }
 
-// i-chunks of SOFT_BLOCK per walk; j and s entries of walk w start at the running totals
+// i-chunks of per_wg per walk; j and s entries of walk w start at the running totals
 std::vector<SoftGroup> walk_groups(TagCtx *c, int n_walk, const int *n_epi, const int *n_epj, const int *n_spj) {
     std::vector<SoftGroup> groups;
+    auto count = [&](int per_wg) {
+        long long n = 0;
+        for (int w = 0; w < n_walk; w++) n += ((long long)n_epi[w] + per_wg - 1) / per_wg;
+        return n;
+    };
+    direct_lanes(count, [&](auto LI) { c->i_lanes = LI.value; });
+    const int per_wg = DIRECT_IPL * c->i_lanes;
     c->i_off.assign(n_walk + 1, 0);
     long long io = 0, jo = 0, so = 0;
     for (int w = 0; w < n_walk; w++) {
         c->i_off[w] = (int)io;
-        for (int b = 0; b < n_epi[w]; b += SOFT_BLOCK) {
+        for (int b = 0; b < n_epi[w]; b += per_wg) {
             SoftGroup g{};
             g.i_begin = (int)(io + b);
-            g.ni = std::min(SOFT_BLOCK, n_epi[w] - b);
+            g.ni = std::min(per_wg, n_epi[w] - b);
             g.j_begin = (int)jo;
             g.nj = n_epj[w];
             g.jf_begin = 0;
@@ -166,9 +173,8 @@ int clear_forces(TagCtx *c, long long ni) {
 
 template <class JS, class SS, int SPMODE>
 int launch_and_return(TagCtx *c, const SoftGroup *d_groups, int ng, SrcEPI is, JS js, SS ss) {
-    SinkForce out{(gplum_force *)c->d_force.p};
-    CandBuf nocand{nullptr, nullptr, 0};
-    launch_soft_f32<SrcEPI, JS, SS, SinkForce, EP | SPMODE>(d_groups, ng, is, js, js, ss, out, g_eps2, nocand, c->st);
+    launch_direct_groups<EP | SPMODE, DirectEP<JS>, DirectSP<SS, SPMODE == SPQ>>(
+        c->i_lanes, d_groups, ng, is, js, ss, SinkForce{(gplum_force *)c->d_force.p}, g_eps2, c->st);
     GPLUM_HIP(hipGetLastError());
     GPLUM_HIP(hipMemcpyAsync(c->h_force.p, c->d_force.p, sizeof(gplum_force) * c->ni_total, hipMemcpyDeviceToHost,
                              c->st));

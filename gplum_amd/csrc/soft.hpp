@@ -147,13 +147,14 @@ struct SrcNone {
 };
 
 // ------------------------------------------------------------------ sinks
-struct SinkForce {                    // accumulate into reference ForceGrav (PIKG)
+struct SinkForce {                    // accumulate into reference ForceGrav (PIKG), rounded once
     gplum_force *f;
     __device__ void write(int i, double ax, double ay, double az, double pot, int ngb,
                           int rankf, int idmax, int idmin, bool has_ep) const {
         gplum_force &q = f[i];
-        q.acc[0] += (float)ax; q.acc[1] += (float)ay; q.acc[2] += (float)az;
-        q.phi += (float)pot;
+        q.acc[0] = (float)((double)q.acc[0] + ax); q.acc[1] = (float)((double)q.acc[1] + ay);
+        q.acc[2] = (float)((double)q.acc[2] + az);
+        q.phi = (float)((double)q.phi + pot);
         if (has_ep) {
             q.neighbor.number += ngb;
             q.neighbor.rank += rankf;

@@ -96,24 +96,10 @@ __device__ inline void emit_candidate(bool nb, int idi, int idj, const CandBuf &
     }
 }
 
-// EP-EP pair with neighbour predicate, r_out clamp and candidate emission.
-template <bool EMITC>
-__device__ inline void epep_near(const IState &I, bool valid, float4 pj, float4 aj, float4 lj, float eps2,
-                                 Acc32 &a, int &ngb, int &rankf, int &idmax, int &idmin,
-                                 const CandBuf &cand) {
+// EP-EP pair with r_out clamp; returns the neighbour predicate (up to the identity test).
+__device__ inline bool epep_pair(const IState &I, float4 pj, float4 aj, float4 lj, float eps2, Acc32 &a) {
     const float rxp = pj.x - I.xh, ryp = pj.y - I.yh, rzp = pj.z - I.zh;
     const float r2r = __builtin_fmaf(rzp, rzp, __builtin_fmaf(ryp, ryp, __builtin_fmaf(rxp, rxp, eps2)));
-    const float rs2 = fmaxf(I.rs2, aj.y);
-    const int idj = __float_as_int(aj.z), rkj = __float_as_int(aj.w);
-    const bool nb = valid && (r2r < rs2) && (I.id != idj || I.rank != rkj);
-    if (nb) {
-        ngb++;
-        const int d = I.rank - rkj;
-        rankf += d * d;
-        idmax = max(idmax, idj);
-        idmin = min(idmin, idj);
-    }
-    if (EMITC) emit_candidate(nb, I.id, idj, cand);
     const float rx = rxp + (lj.x - I.xl), ry = ryp + (lj.y - I.yl), rz = rzp + (lj.z - I.zl);
     const float r2f = __builtin_fmaf(rz, rz, __builtin_fmaf(ry, ry, __builtin_fmaf(rx, rx, eps2)));
     const float r2 = fmaxf(r2f, fmaxf(I.ro2, aj.x));
@@ -124,6 +110,35 @@ __device__ inline void epep_near(const IState &I, bool valid, float4 pj, float4 
     a.y = __builtin_fmaf(mr3, ry, a.y);
     a.z = __builtin_fmaf(mr3, rz, a.z);
     a.p -= mr;
+    return r2r < fmaxf(I.rs2, aj.y);
+}
+
+// The neighbour data of a pair within max(r_search); returns whether j is another particle.
+__device__ inline bool epep_neighbour(const IState &I, float4 aj, int &ngb, int &rankf, int &idmax, int &idmin) {
+    const int idj = __float_as_int(aj.z), rkj = __float_as_int(aj.w);
+    const bool nb = I.id != idj || I.rank != rkj;
+    if (nb) {
+        ngb++;
+        const int d = I.rank - rkj;
+        rankf += d * d;
+        idmax = max(idmax, idj);
+        idmin = min(idmin, idj);
+    }
+    return nb;
+}
+
+// The pair with candidate emission (all lanes of a wave together); most pairs of a wave have
+// no lane within r_search and skip the neighbour part.
+template <bool EMITC>
+__device__ inline void epep_near(const IState &I, bool valid, float4 pj, float4 aj, float4 lj, float eps2,
+                                 Acc32 &a, int &ngb, int &rankf, int &idmax, int &idmin,
+                                 const CandBuf &cand) {
+    const bool within = epep_pair(I, pj, aj, lj, eps2, a) && valid;
+    if (__ballot(within)) {
+        bool nb = false;
+        if (within) nb = epep_neighbour(I, aj, ngb, rankf, idmax, idmin);
+        if (EMITC) emit_candidate(nb, I.id, __float_as_int(aj.z), cand);
+    }
 }
 
 // EP-EP pair known to lie beyond 1.1 max(r_search) > r_out: no predicate, no clamp.  At
@@ -141,6 +156,15 @@ __device__ inline void epep_far(const IState &I, float4 pj, float eps2, Acc32 &a
     a.y = __builtin_fmaf(mr3, ry, a.y);
     a.z = __builtin_fmaf(mr3, rz, a.z);
     a.p -= mr;
+}
+
+// The per-SPJ hoisted terms of gravity_kernel_epsp.pikg:75-82 (FP32).
+__device__ inline void spj_terms(const double q[6], float eps2, float4 &qa, float4 &qb) {
+    const float qxx0 = (float)q[0], qyy0 = (float)q[1], qzz0 = (float)q[2];
+    const float qxy0 = (float)q[3], qxz0 = (float)q[4], qyz0 = (float)q[5];
+    const float tr = qxx0 + qyy0 + qzz0;
+    qa = make_float4(3.0f * qxx0 - tr, 3.0f * qyy0 - tr, 3.0f * qzz0 - tr, 3.0f * qxy0);
+    qb = make_float4(3.0f * qyz0, 3.0f * qxz0, -(eps2 * tr), 0.f);
 }
 
 // EP-SP pair: a node opened by neither the opening angle nor the search radius, as far
@@ -290,14 +314,7 @@ __global__ __launch_bounds__(SOFT_BLOCK) void k_soft_f32(const SoftGroup *__rest
                 double m, x, y, z, q[6];
                 ss.load(G.s_begin + base + t, m, x, y, z, q);
                 s_a[t] = make_float4((float)(x - x0), (float)(y - y0), (float)(z - z0), (float)m);
-                if (MODE & SPQ) {
-                    // per-SPJ hoisted terms of gravity_kernel_epsp.pikg:75-82 (FP32)
-                    const float qxx0 = (float)q[0], qyy0 = (float)q[1], qzz0 = (float)q[2];
-                    const float qxy0 = (float)q[3], qxz0 = (float)q[4], qyz0 = (float)q[5];
-                    const float tr = qxx0 + qyy0 + qzz0;
-                    s_b[t] = make_float4(3.0f * qxx0 - tr, 3.0f * qyy0 - tr, 3.0f * qzz0 - tr, 3.0f * qxy0);
-                    s_c[t] = make_float4(3.0f * qyz0, 3.0f * qxz0, -(eps2 * tr), 0.f);
-                }
+                if (MODE & SPQ) spj_terms(q, eps2, s_b[t], s_c[t]);
             }
             __syncthreads();
             if (S.in_split) {

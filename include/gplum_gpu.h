@@ -148,10 +148,8 @@ int gplum_calc_force_epsp_quad_f64(const gplum_epi *epi, int ni,
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc): gplum_calc_force_epep on device-resident arrays (d_epi[ni], d_epj[nj],
  * d_force[ni], accumulated as there), launched asynchronously on `stream` (a
- * hipStream_t; NULL = the default stream).  It allocates nothing: its i-chunk table
- * lives in a fixed per-device array of 4096 entries, so ni <= 1,048,576 (larger ni
- * returns GPLUM_E_ARG).  Every call on a device shares that array: calls that overlap
- * on one device (different streams or host threads) race. */
+ * hipStream_t; NULL = the default stream).  It allocates nothing and uses no memory but
+ * its arguments, so calls may overlap; ni <= 1,048,576 (larger ni returns GPLUM_E_ARG). */
 int gplum_calc_force_epep_noalloc(const gplum_epi *d_epi, int ni,
                                   const gplum_epj *d_epj, int nj,
                                   gplum_force *d_force, float eps2, void *stream);
