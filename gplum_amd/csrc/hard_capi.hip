@@ -9,6 +9,7 @@
 #include <cstring>
 #include <vector>
 
+#include "aos.hpp"
 #include "hermite.hpp"
 #include "system.hpp"
 
@@ -21,6 +22,7 @@ struct HardCtx {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     HardBuffers hb;
     DArray<int32_t> off, order;
+    DArray<gplum_particle> aos;   // the caller's particles as uploaded
     // uploaded state kept for graph replays (each replay restores it first)
     DArray<double> b_pos, b_vel, b_acc_s, b_jerk_s, b_acc_d, b_jerk_d, b_mass, b_rinv, b_time, b_dt, b_acc0,
         b_r_planet, b_f;
@@ -72,6 +74,23 @@ int check_args(const gplum_params *p, const gplum_particle *pp, int n, const int
     return GPLUM_OK;
 }
 
+// the particle words that go both ways
+AosTable aos_table(HardBuffers &hb) {
+    AosTable t;
+    AOS_SET3(t, pos, hb.pos.p); AOS_SET3(t, vel, hb.vel.p); AOS_SET3(t, acc_s, hb.acc_s.p);
+    AOS_SET3(t, jerk_s, hb.jerk_s.p); AOS_SET3(t, acc_d, hb.acc_d.p); AOS_SET3(t, jerk_d, hb.jerk_d.p);
+    AOS_SET(t, dt, hb.dt.p); AOS_SET(t, r_planet, hb.r_planet.p); AOS_SET(t, time, hb.time.p);
+    AOS_SET(t, id, hb.id.p); AOS_SET(t, flags, hb.flags.p);
+    return t;
+}
+
+__global__ void k_local_time(int n, double *__restrict__ time, int32_t *__restrict__ flags) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    time[i] = 0.;
+    flags[i] = 0;
+}
+
 // Uploads the clusters into c.hb (and the offsets / order), then, for bare clusters,
 // computes their acc/jerk and first block step on the device.
 int hard_upload(HardCtx &c, const gplum_params *p, const gplum_particle *pp, int n, const int32_t *offsets,
@@ -92,35 +111,17 @@ int hard_upload(HardCtx &c, const gplum_params *p, const gplum_particle *pp, int
     }
     std::stable_sort(pl.order.begin(), pl.order.end(), [&](int a, int b) { return pl.sizes[a] > pl.sizes[b]; });
     hb.max_size = max_size;
-    std::vector<double> v3(3 * (size_t)n), v1(n);
-    std::vector<int64_t> ids(n);
-    std::vector<int32_t> fl(n, 0), offs(offsets, offsets + n_cluster + 1);
-    auto put3 = [&](DArray<double> &d, size_t fo) {
-        for (int i = 0; i < n; i++)
-            for (int k = 0; k < 3; k++) v3[3 * i + k] = *(const double *)((const char *)&pp[i] + fo + 8 * k);
-        int r = upload(d, v3, c.st);
-        if (r) return r;
-        GPLUM_HIP(hipStreamSynchronize(c.st));   // v3 is reused
-        return (int)GPLUM_OK;
-    };
-    auto put1 = [&](DArray<double> &d, size_t fo) {
-        for (int i = 0; i < n; i++) v1[i] = *(const double *)((const char *)&pp[i] + fo);
-        int r = upload(d, v1, c.st);
-        if (r) return r;
-        GPLUM_HIP(hipStreamSynchronize(c.st));   // v1 is reused
-        return (int)GPLUM_OK;
-    };
-#define P3(dst, f) if ((rc = put3(hb.dst, offsetof(gplum_particle, f)))) return rc
-#define P1(dst, f) if ((rc = put1(hb.dst, offsetof(gplum_particle, f)))) return rc
-    P3(pos, pos); P3(vel, vel); P3(acc_s, acc_s); P3(jerk_s, jerk_s); P3(acc_d, acc_d); P3(jerk_d, jerk_d);
-    P1(mass, mass); P1(rinv, r_out_inv); P1(dt, dt); P1(acc0, acc0); P1(r_planet, r_planet); P1(f, f);
-#undef P3
-#undef P1
-    pl.tc.assign(n, 0.);
-    for (int i = 0; i < n; i++) { pl.tc[i] = pp[i].time; v1[i] = 0.; ids[i] = pp[i].id; }
-    if ((rc = upload(hb.time, v1, c.st))) return rc;
-    if ((rc = upload(hb.id, ids, c.st))) return rc;
-    if ((rc = upload(hb.flags, fl, c.st))) return rc;
+    GPLUM_ENSURE(c.aos, n);
+    GPLUM_HIP(hipMemcpyAsync(c.aos.p, pp, sizeof(gplum_particle) * (size_t)n, hipMemcpyHostToDevice, c.st));
+    AosTable t = aos_table(hb);
+    AOS_SET(t, mass, hb.mass.p); AOS_SET(t, r_out_inv, hb.rinv.p); AOS_SET(t, acc0, hb.acc0.p); AOS_SET(t, f, hb.f.p);
+    if ((rc = aos_unpack(t, 0, n, c.aos.p, c.st))) return rc;
+    if (n > 0)
+        hipLaunchKernelGGL(k_local_time, dim3(ceil_div(n, 256)), dim3(256), 0, c.st, n, hb.time.p, hb.flags.p);
+    GPLUM_HIP(hipGetLastError());
+    const std::vector<int32_t> offs(offsets, offsets + n_cluster + 1);
+    pl.tc.resize(n);
+    for (int i = 0; i < n; i++) pl.tc[i] = pp[i].time;
     GPLUM_ENSURE(c.off, n_cluster + 1);
     GPLUM_ENSURE(c.order, n_cluster);
     if ((rc = upload(c.off, offs, c.st))) return rc;
@@ -141,37 +142,16 @@ int hard_download(HardCtx &c, gplum_particle *pp, const int32_t *offsets, const 
     int rc;
     const int n = pl.n, n_cluster = pl.n_cluster;
     HardBuffers &hb = c.hb;
-    std::vector<double> v3(3 * (size_t)n), v1(n);
-    std::vector<int64_t> ids(n);
-    std::vector<int32_t> fl(n);
     std::vector<double> ed(n_cluster);
     std::vector<long long> nb(n_cluster), np(n_cluster);
     if ((rc = download(ed, hb.edisp, c.st))) return rc;
     if ((rc = download(nb, hb.nblock, c.st))) return rc;
     if ((rc = download(np, hb.npair, c.st))) return rc;
-    auto get3 = [&](DArray<double> &d, size_t fo) {
-        int r = download(v3, d, c.st);
-        if (r) return r;
-        GPLUM_HIP(hipStreamSynchronize(c.st));
-        for (int i = 0; i < n; i++)
-            for (int k = 0; k < 3; k++) *(double *)((char *)&pp[i] + fo + 8 * k) = v3[3 * i + k];
-        return (int)GPLUM_OK;
-    };
-    auto get1 = [&](DArray<double> &d, size_t fo) {
-        int r = download(v1, d, c.st);
-        if (r) return r;
-        GPLUM_HIP(hipStreamSynchronize(c.st));
-        for (int i = 0; i < n; i++) *(double *)((char *)&pp[i] + fo) = v1[i];
-        return (int)GPLUM_OK;
-    };
-#define G3(src, f) if ((rc = get3(hb.src, offsetof(gplum_particle, f)))) return rc
-#define G1(src, f) if ((rc = get1(hb.src, offsetof(gplum_particle, f)))) return rc
-    G3(pos, pos); G3(vel, vel); G3(acc_s, acc_s); G3(jerk_s, jerk_s); G3(acc_d, acc_d); G3(jerk_d, jerk_d);
-    G1(dt, dt); G1(r_planet, r_planet); G1(phi_d, phi_d); G1(phi_s, phi_s); G1(time, time); G1(mass, mass);
-#undef G3
-#undef G1
-    if ((rc = download(ids, hb.id, c.st))) return rc;
-    if ((rc = download(fl, hb.flags, c.st))) return rc;
+    // the words that the integration does not write are those uploaded
+    AosTable t = aos_table(hb);
+    AOS_SET(t, phi_d, hb.phi_d.p); AOS_SET(t, phi_s, hb.phi_s.p); AOS_SET(t, mass, hb.mass.p);
+    if ((rc = aos_pack(t, 0, n, c.aos.p, c.st))) return rc;
+    GPLUM_HIP(hipMemcpyAsync(pp, c.aos.p, sizeof(gplum_particle) * (size_t)n, hipMemcpyDeviceToHost, c.st));
     GPLUM_HIP(hipStreamSynchronize(c.st));
     double etot = 0.;
     long long btot = 0, ptot = 0;
@@ -184,8 +164,6 @@ int hard_download(HardCtx &c, gplum_particle *pp, const int32_t *offsets, const 
     for (int k = 0; k < n_cluster; k++)
         for (int i = offsets[k]; i < offsets[k + 1]; i++) {
             pp[i].time = pl.tc[i] + pp[i].time;   // resetTime
-            pp[i].id = ids[i];
-            pp[i].flags = fl[i];
             pp[i].n_cluster = pl.sizes[k];
         }
     if (edisp) *edisp = etot;

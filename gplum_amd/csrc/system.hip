@@ -19,6 +19,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include "aos.hpp"
 #include "hermite.hpp"
 #include "neighbor.hpp"
 #include "soft_kernels.hpp"
@@ -272,6 +273,26 @@ PartPtrs System::ptrs(ParticleSoA &s) {
                     s.f.p, s.phi.p, s.phi_d.p, s.phi_s.p, s.id.p, s.flags.p, s.n_cluster.p, s.number.p};
 }
 
+// Particles per transfer of set_particles and get_particles (82 MB of device memory).
+constexpr int AOS_CHUNK = 1 << 18;
+
+// every word of gplum_particle in the particle arrays
+static AosTable aos_table(ParticleSoA &s) {
+    AosTable t;
+    AOS_SET(t, id, s.id.p); AOS_SET(t, id_cluster, s.id_cluster.p);
+    AOS_SET(t, mass, s.mass.p); AOS_SET(t, r_planet, s.r_planet.p); AOS_SET(t, f, s.f.p);
+    AOS_SET3(t, pos, s.pos.p); AOS_SET3(t, vel, s.vel.p); AOS_SET3(t, acc, s.acc.p);
+    AOS_SET3(t, acc_d, s.acc_d.p); AOS_SET3(t, jerk_d, s.jerk_d.p);
+    AOS_SET3(t, acc_s, s.acc_s.p); AOS_SET3(t, jerk_s, s.jerk_s.p);
+    AOS_SET(t, phi, s.phi.p); AOS_SET(t, phi_d, s.phi_d.p); AOS_SET(t, phi_s, s.phi_s.p);
+    AOS_SET(t, r_out, s.r_out.p); AOS_SET(t, r_out_inv, s.r_out_inv.p); AOS_SET(t, r_search, s.r_search.p);
+    AOS_SET(t, v_disp, s.v_disp.p); AOS_SET(t, time, s.time.p); AOS_SET(t, dt, s.dt.p); AOS_SET(t, acc0, s.acc0.p);
+    AOS_SET(t, neighbor.number, s.number.p); AOS_SET(t, neighbor.rank, s.rank.p);
+    AOS_SET(t, neighbor.id_max, s.id_max.p); AOS_SET(t, neighbor.id_min, s.id_min.p);
+    AOS_SET(t, n_cluster, s.n_cluster.p); AOS_SET(t, flags, s.flags.p);
+    return t;
+}
+
 int System::set_particles(const gplum_particle *pp, int count, double time) {
     int rc = init_device();
     if (rc) return rc;
@@ -281,40 +302,15 @@ int System::set_particles(const gplum_particle *pp, int count, double time) {
     n = count;
     time_sys = time;
     if ((rc = A.ensure(n)) || (rc = B.ensure(n))) return rc;
-    std::vector<double> v3(3 * (size_t)n), v1(n);
-    std::vector<int64_t> i64(n);
-    std::vector<int32_t> i32(n);
-    auto put3 = [&](DArray<double> &d, size_t off) {
-        for (int i = 0; i < n; i++)
-            for (int k = 0; k < 3; k++) v3[3 * i + k] = *(const double *)((const char *)&pp[i] + off + 8 * k);
-        return hipMemcpy(d.p, v3.data(), sizeof(double) * 3 * n, hipMemcpyHostToDevice);
-    };
-    auto put1 = [&](DArray<double> &d, size_t off) {
-        for (int i = 0; i < n; i++) v1[i] = *(const double *)((const char *)&pp[i] + off);
-        return hipMemcpy(d.p, v1.data(), sizeof(double) * n, hipMemcpyHostToDevice);
-    };
-#define P3(f) GPLUM_HIP(put3(A.f, offsetof(gplum_particle, f)))
-#define P1(f) GPLUM_HIP(put1(A.f, offsetof(gplum_particle, f)))
-    P3(pos); P3(vel); P3(acc); P3(acc_d); P3(jerk_d); P3(acc_s); P3(jerk_s);
-    P1(mass); P1(r_planet); P1(f); P1(phi); P1(phi_d); P1(phi_s); P1(r_out); P1(r_out_inv); P1(r_search);
-    P1(v_disp); P1(time); P1(dt); P1(acc0);
-#undef P3
-#undef P1
-    for (int i = 0; i < n; i++) i64[i] = pp[i].id;
-    GPLUM_HIP(hipMemcpy(A.id.p, i64.data(), 8 * (size_t)n, hipMemcpyHostToDevice));
+    const AosTable t = aos_table(A);
+    for (int i0 = 0; i0 < n; i0 += AOS_CHUNK) {
+        const int c = std::min(AOS_CHUNK, n - i0);
+        GPLUM_ENSURE(aos, c);
+        GPLUM_HIP(hipMemcpyAsync(aos.p, pp + i0, sizeof(gplum_particle) * (size_t)c, hipMemcpyHostToDevice, st));
+        if ((rc = aos_unpack(t, i0, c, aos.p, st))) return rc;
+    }
+    GPLUM_HIP(hipStreamSynchronize(st));
     fc.lam_valid = false;
-    for (int i = 0; i < n; i++) i64[i] = pp[i].id_cluster;
-    GPLUM_HIP(hipMemcpy(A.id_cluster.p, i64.data(), 8 * (size_t)n, hipMemcpyHostToDevice));
-    auto puti = [&](DArray<int32_t> &d, auto getter) {
-        for (int i = 0; i < n; i++) i32[i] = getter(pp[i]);
-        return hipMemcpy(d.p, i32.data(), 4 * (size_t)n, hipMemcpyHostToDevice);
-    };
-    GPLUM_HIP(puti(A.number, [](const gplum_particle &q) { return q.neighbor.number; }));
-    GPLUM_HIP(puti(A.rank, [](const gplum_particle &q) { return q.neighbor.rank; }));
-    GPLUM_HIP(puti(A.id_max, [](const gplum_particle &q) { return q.neighbor.id_max; }));
-    GPLUM_HIP(puti(A.id_min, [](const gplum_particle &q) { return q.neighbor.id_min; }));
-    GPLUM_HIP(puti(A.n_cluster, [](const gplum_particle &q) { return q.n_cluster; }));
-    GPLUM_HIP(puti(A.flags, [](const gplum_particle &q) { return q.flags; }));
     nb.n = 0;
     nb.n_nbr = 0;
     have_nbr = false;
@@ -325,43 +321,15 @@ int System::set_particles(const gplum_particle *pp, int count, double time) {
 int System::get_particles(gplum_particle *pp, int count) {
     if (count < n) return fail(GPLUM_E_ARG, "output array too small");
     GPLUM_HIP(hipStreamSynchronize(st));
-    std::vector<double> v3(3 * (size_t)n), v1(n);
-    std::vector<int64_t> i64(n);
-    std::vector<int32_t> i32(n);
-    std::memset(pp, 0, sizeof(gplum_particle) * (size_t)n);
-    auto get3 = [&](DArray<double> &d, size_t off) {
-        hipError_t e = hipMemcpy(v3.data(), d.p, sizeof(double) * 3 * n, hipMemcpyDeviceToHost);
-        for (int i = 0; i < n; i++)
-            for (int k = 0; k < 3; k++) *(double *)((char *)&pp[i] + off + 8 * k) = v3[3 * i + k];
-        return e;
-    };
-    auto get1 = [&](DArray<double> &d, size_t off) {
-        hipError_t e = hipMemcpy(v1.data(), d.p, sizeof(double) * n, hipMemcpyDeviceToHost);
-        for (int i = 0; i < n; i++) *(double *)((char *)&pp[i] + off) = v1[i];
-        return e;
-    };
-#define G3(f) GPLUM_HIP(get3(A.f, offsetof(gplum_particle, f)))
-#define G1(f) GPLUM_HIP(get1(A.f, offsetof(gplum_particle, f)))
-    G3(pos); G3(vel); G3(acc); G3(acc_d); G3(jerk_d); G3(acc_s); G3(jerk_s);
-    G1(mass); G1(r_planet); G1(f); G1(phi); G1(phi_d); G1(phi_s); G1(r_out); G1(r_out_inv); G1(r_search);
-    G1(v_disp); G1(time); G1(dt); G1(acc0);
-#undef G3
-#undef G1
-    GPLUM_HIP(hipMemcpy(i64.data(), A.id.p, 8 * (size_t)n, hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; i++) pp[i].id = i64[i];
-    GPLUM_HIP(hipMemcpy(i64.data(), A.id_cluster.p, 8 * (size_t)n, hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; i++) pp[i].id_cluster = i64[i];
-    auto geti = [&](DArray<int32_t> &d, auto setter) {
-        hipError_t e = hipMemcpy(i32.data(), d.p, 4 * (size_t)n, hipMemcpyDeviceToHost);
-        for (int i = 0; i < n; i++) setter(pp[i], i32[i]);
-        return e;
-    };
-    GPLUM_HIP(geti(A.number, [](gplum_particle &q, int v) { q.neighbor.number = v; }));
-    GPLUM_HIP(geti(A.rank, [](gplum_particle &q, int v) { q.neighbor.rank = v; }));
-    GPLUM_HIP(geti(A.id_max, [](gplum_particle &q, int v) { q.neighbor.id_max = v; }));
-    GPLUM_HIP(geti(A.id_min, [](gplum_particle &q, int v) { q.neighbor.id_min = v; }));
-    GPLUM_HIP(geti(A.n_cluster, [](gplum_particle &q, int v) { q.n_cluster = v; }));
-    GPLUM_HIP(geti(A.flags, [](gplum_particle &q, int v) { q.flags = v; }));
+    const AosTable t = aos_table(A);
+    for (int i0 = 0; i0 < n; i0 += AOS_CHUNK) {
+        const int c = std::min(AOS_CHUNK, n - i0);
+        GPLUM_ENSURE(aos, c);
+        int rc = aos_pack(t, i0, c, aos.p, st);
+        if (rc) return rc;
+        GPLUM_HIP(hipMemcpyAsync(pp + i0, aos.p, sizeof(gplum_particle) * (size_t)c, hipMemcpyDeviceToHost, st));
+        GPLUM_HIP(hipStreamSynchronize(st));
+    }
     return GPLUM_OK;
 }
 
@@ -651,22 +619,47 @@ int System::energy(double out[5]) {
 
 // main_p3t.cpp:289-364: time, flags, r_planet/f defaults, radii, two rounds of
 // (tree force + correctForceLongInitial).
+__global__ void k_zero_one(int32_t *p) { *p = 0; }
+__global__ void k_initialize(int n, double time_sys, double increase_factor, const double *__restrict__ r_planet,
+                             double *__restrict__ time, double *__restrict__ f, int32_t *__restrict__ number,
+                             int32_t *__restrict__ n_cluster, int32_t *__restrict__ flags, int32_t *__restrict__ bare) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    time[i] = time_sys;
+    number[i] = 0;
+    n_cluster[i] = 0;
+    flags[i] = 0;
+    if (f[i] == 0.) f[i] = increase_factor;
+    if (r_planet[i] <= 0.) *bare = 1;
+}
+
 int System::initialize() {
     int rc = init_device();
     if (rc) return rc;
-    {
-        std::vector<gplum_particle> h(n);
-        if ((rc = get_particles(h.data(), n))) return rc;
-        for (auto &q : h) {
-            q.time = time_sys;
-            q.neighbor.number = 0;
-            q.n_cluster = 0;
-            q.flags = 0;
-            if (q.r_planet <= 0.) q.r_planet = std::pow(0.75 * q.mass / (3.14159265358979323846 * p.dens), 1. / 3.);
-            if (q.f == 0.) q.f = p.increase_factor;
-        }
-        if ((rc = set_particles(h.data(), n, time_sys))) return rc;
+    // the start of an integration: time, counters and, where not given, radius and enlargement
+    // (the radius on the host: its pow is the host library's)
+    GPLUM_HIP(hst.ensure(sizeof(int32_t)));
+    GPLUM_ENSURE(init_bare, 1);
+    hipLaunchKernelGGL(k_zero_one, dim3(1), dim3(1), 0, st, init_bare.p);
+    if (n > 0)
+        hipLaunchKernelGGL(k_initialize, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, time_sys, p.increase_factor, A.r_planet.p,
+                           A.time.p, A.f.p, A.number.p, A.n_cluster.p, A.flags.p, init_bare.p);
+    GPLUM_HIP(hipGetLastError());
+    GPLUM_HIP(hipMemcpyAsync(hst.p, init_bare.p, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    GPLUM_HIP(hipStreamSynchronize(st));
+    if (*hst.as<int32_t>()) {
+        std::vector<double> r(n), m(n);
+        GPLUM_HIP(hipMemcpy(r.data(), A.r_planet.p, sizeof(double) * n, hipMemcpyDeviceToHost));
+        GPLUM_HIP(hipMemcpy(m.data(), A.mass.p, sizeof(double) * n, hipMemcpyDeviceToHost));
+        for (int i = 0; i < n; i++)
+            if (r[i] <= 0.) r[i] = std::pow(0.75 * m[i] / (3.14159265358979323846 * p.dens), 1. / 3.);
+        GPLUM_HIP(hipMemcpy(A.r_planet.p, r.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     }
+    fc.lam_valid = false;
+    nb.n = 0;
+    nb.n_nbr = 0;
+    have_nbr = false;
+    istep = std::llround(time_sys / p.dt_tree);
     if ((rc = set_radii())) return rc;
     for (int r = 0; r < 2; r++)
         if ((rc = soft_force(true, plain_f64))) return rc;

@@ -91,6 +91,8 @@ struct System {
     bool tuning = false;                // inside autotune(): no training, no statistics
     bool skip_train = false;            // the force recomputed after mergers: no training
     ParticleSoA A, B;
+    DArray<gplum_particle> aos;         // the transfers of set_particles and get_particles
+    DArray<int32_t> init_bare;          // initialize(): a particle without a radius
     RadiiScratch rad;
     MergeScratch mrg;
     Tree tree;
