@@ -375,8 +375,7 @@ int fc_train(CandSizer &s, const int32_t *count_fp32, int n, hipStream_t st, boo
         hipLaunchKernelGGL(k_fc_sample, dim3(ceil_div(m, 256)), dim3(256), 0, st, m, n, stride, phase, s.x.p,
                            count_fp32, s.xs.p, s.ys.p);
         double *lp = (want_loss && k == s.train_steps - 1) ? &s.last_loss : nullptr;
-        if ((rc = s.net.loss_grad(s.xs.p, s.ys.p, m, lp, st))) return rc;
-        if ((rc = s.net.adam_step(st))) return rc;
+        if ((rc = s.net.gradient(s.xs.p, s.ys.p, m, lp, true, st))) return rc;
     }
     s.last_batch = m;
     s.trained_rounds++;

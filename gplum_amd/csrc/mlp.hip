@@ -3,11 +3,8 @@
 //
 // Parameter layout (float32, 4545 values): W1[64][4], b1[64], W2[64][64], b2[64],
 // w3[64], b3.  Loss: mean Poisson NLL  lambda - y log(lambda + 1e-6).
-// Forward/backward: one thread per sample, parameters read with wave-uniform addresses
-// (scalar loads, no per-lane traffic).  Gradient: per-sample activations and deltas are stored
-// sample-major ([n][64]); one lane per parameter sums its products over a chunk of
-// samples in FP64 (lanes of a wave read one contiguous 256-byte row per sample), and a
-// second pass adds the chunk partials in chunk order, so the gradient is deterministic.
+// Forward (k_mlp_forward): one thread per sample, parameters read with wave-uniform addresses
+// (scalar loads, no per-lane traffic).  Training: k_mlp_backward and k_mlp_update below.
 #include <vector>
 
 #include "mlp.hpp"
@@ -59,107 +56,201 @@ __global__ __launch_bounds__(256) void k_mlp_forward(const float *__restrict__ t
     lam[i] = mlp_eval(theta, xi, h1, h2, &z);
 }
 
-// per-sample backward: stores h1, h2, d1, d2 (sample-major, [n][64]) and dz[n]
-__global__ __launch_bounds__(256) void k_mlp_backward(const float *__restrict__ theta, const float *__restrict__ x,
-                                                      const float *__restrict__ y, int n, float *__restrict__ H1,
-                                                      float *__restrict__ H2, float *__restrict__ D1,
-                                                      float *__restrict__ D2, float *__restrict__ DZ,
+// --------------------------------------------------------------- training
+//
+// A training step is 0.1 GFLOP and 0.2 MB: bound by how many CUs take part and by the latency of
+// its few dependent stages.  A workgroup of 4 waves takes tiles of 32 samples (8192 samples: one
+// tile on every CU); the 64 x 64 layer runs forward and backward on the FP32 matrix
+// instruction (16 x 16 x 4: FP32 operands and sums), wave w owning hidden units 16 w ... 16 w + 15, with W2
+// as operands in registers.  The gradient is summed in FP64 (products of two FP32 values are
+// exact there): W2's on the FP64 matrix instruction, the others per lane, over the tiles of a
+// workgroup in registers; the workgroups' sums are added in a fixed order by k_mlp_update, which
+// also takes the Adam step.  One thread per sample (32 workgroups, weights by scalar loads, the
+// activations through memory to a second and third pass): 94 + 18 + 17 + 5 us per step of
+// 8192 samples.
+typedef float mlp_v4f __attribute__((ext_vector_type(4)));
+typedef double mlp_v4d __attribute__((ext_vector_type(4)));
+
+constexpr int MLP_TILE = 32;         // samples per tile
+constexpr int MLP_LD = 68;           // row stride of a tile in LDS: 16 rows x 4 columns hit 64 banks
+constexpr int MLP_MAX_WG = 256;
+
+static int mlp_grid(int n) { return std::min(ceil_div(n, MLP_TILE), MLP_MAX_WG); }
+
+__global__ __launch_bounds__(256) void k_mlp_backward(const float *__restrict__ s, const float *__restrict__ x,
+                                                      const float *__restrict__ y, int n, double *__restrict__ part,
                                                       double *__restrict__ loss_part) {
-    __shared__ double sl[256];
-    const float *__restrict__ s = theta;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double li = 0.;
-    if (i < n) {
-        float xi[MLP_NIN], h1[MLP_NH], h2[MLP_NH], z;
+    __shared__ float s_h[MLP_TILE][MLP_LD], s_d[MLP_TILE][MLP_LD], s_x[MLP_TILE][MLP_NIN];
+    __shared__ float s_z[4][MLP_TILE], s_dz[MLP_TILE];
+    const int t = (int)threadIdx.x, w = t >> 6, l = t & 63, r = l >> 4, c = l & 15;
+    // layer 1: lane t evaluates units u0 .. u0 + 7 of sample t % 32
+    const int si = t & 31, u0 = (t >> 5) * 8;
+    float w1[8][MLP_NIN], b1[8];
 #pragma unroll
-        for (int q = 0; q < MLP_NIN; q++) xi[q] = x[(size_t)q * n + i];
-        const float lam = mlp_eval(s, xi, h1, h2, &z);
-        const float yi = y[i];
-        li = (double)lam - (double)yi * log((double)lam + (double)MLP_EPS);
-        const float dz = (1.f - yi / (lam + MLP_EPS)) * sigmoid_f(z) / (float)n;
-        DZ[i] = dz;
-        float d2[MLP_NH];
+    for (int u = 0; u < 8; u++) {
+        b1[u] = s[OFF_B1 + u0 + u];
 #pragma unroll
-        for (int p = 0; p < MLP_NH; p++) {
-            d2[p] = dz * s[OFF_W3 + p] * (1.f - h2[p] * h2[p]);
-            H1[(size_t)i * MLP_NH + p] = h1[p];
-            H2[(size_t)i * MLP_NH + p] = h2[p];
-            D2[(size_t)i * MLP_NH + p] = d2[p];
-        }
-#pragma unroll
-        for (int q = 0; q < MLP_NH; q++) {
-            float a = 0.f;
-#pragma unroll
-            for (int p = 0; p < MLP_NH; p++) a = __builtin_fmaf(s[OFF_W2 + p * MLP_NH + q], d2[p], a);
-            D1[(size_t)i * MLP_NH + q] = a * (1.f - h1[q] * h1[q]);
-        }
+        for (int q = 0; q < MLP_NIN; q++) w1[u][q] = s[OFF_W1 + (u0 + u) * MLP_NIN + q];
     }
-    sl[threadIdx.x] = li;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) sl[threadIdx.x] += sl[threadIdx.x + w];
+    // W2 as right operand B[k][n] (lane: k = 4 ks + r, n = unit): forward W2[n][k], backward W2[k][n]
+    const int unit = 16 * w + c;
+    float wf[16], wb[16];
+#pragma unroll
+    for (int ks = 0; ks < 16; ks++) {
+        wf[ks] = s[OFF_W2 + unit * MLP_NH + 4 * ks + r];
+        wb[ks] = s[OFF_W2 + (4 * ks + r) * MLP_NH + unit];
+    }
+    const float b2 = s[OFF_B2 + unit], w3 = s[OFF_W3 + unit], b3 = s[OFF_B3];
+    mlp_v4d g2[4] = {};
+    double gb1 = 0., gb2 = 0., gw3 = 0., gb3 = 0., loss = 0., gw1[MLP_NIN] = {};
+    const int tiles = (n + MLP_TILE - 1) / MLP_TILE;
+    for (int tile = (int)blockIdx.x; tile < tiles; tile += (int)gridDim.x) {
+        const int i0 = MLP_TILE * tile;
+        {
+            float xi[MLP_NIN];
+#pragma unroll
+            for (int q = 0; q < MLP_NIN; q++) xi[q] = (i0 + si < n) ? x[(size_t)q * n + i0 + si] : 0.f;
+            if (t < MLP_TILE)
+#pragma unroll
+                for (int q = 0; q < MLP_NIN; q++) s_x[t][q] = xi[q];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                float a = b1[u];
+#pragma unroll
+                for (int q = 0; q < MLP_NIN; q++) a = __builtin_fmaf(w1[u][q], xi[q], a);
+                s_h[si][u0 + u] = tanhf(a);
+            }
+        }
+        __syncthreads();
+        // h2 of samples 16 h + 4 r + j, unit `unit`; the output layer's sum over the units
+        float h2[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            mlp_v4f acc = {b2, b2, b2, b2};
+#pragma unroll
+            for (int ks = 0; ks < 16; ks++)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(s_h[16 * h + c][4 * ks + r], wf[ks], acc, 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                h2[h][j] = tanhf(acc[j]);
+                float z = w3 * h2[h][j];
+#pragma unroll
+                for (int d = 1; d < 16; d <<= 1) z += __shfl_xor(z, d);
+                if (c == 0) s_z[w][16 * h + 4 * r + j] = z;
+            }
+        }
+        __syncthreads();
+        if (t < MLP_TILE) {
+            float dz = 0.f;
+            if (i0 + t < n) {
+                const float z = b3 + ((s_z[0][t] + s_z[1][t]) + (s_z[2][t] + s_z[3][t]));
+                const float lam = softplus_f(z), yi = y[i0 + t];
+                loss += (double)lam - (double)yi * log((double)lam + (double)MLP_EPS);
+                dz = (1.f - yi / (lam + MLP_EPS)) * sigmoid_f(z) / (float)n;
+            }
+            s_dz[t] = dz;
+            gb3 += (double)dz;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int row = 16 * h + 4 * r + j;
+                const float dz = s_dz[row], d2 = dz * w3 * (1.f - h2[h][j] * h2[h][j]);
+                s_d[row][unit] = d2;
+                gb2 += (double)d2;
+                gw3 += (double)dz * (double)h2[h][j];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            mlp_v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < 16; ks++)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(s_d[16 * h + c][4 * ks + r], wb[ks], acc, 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int row = 16 * h + 4 * r + j;
+                const float h1 = s_h[row][unit], d1 = acc[j] * (1.f - h1 * h1);
+                gb1 += (double)d1;
+#pragma unroll
+                for (int q = 0; q < MLP_NIN; q++) gw1[q] += (double)d1 * (double)s_x[row][q];
+            }
+        }
+        // dW2[p][q] += d2[sample][p] h1[sample][q]: rows p = 16 w + ..., columns 16 u + c
+#pragma unroll
+        for (int ks = 0; ks < MLP_TILE / 4; ks++) {
+            const double a = (double)s_d[4 * ks + r][unit];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                g2[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)s_h[4 * ks + r][16 * u + c], g2[u], 0, 0, 0);
+        }
         __syncthreads();
     }
-    if (threadIdx.x == 0) loss_part[blockIdx.x] = sl[0];
-}
-
-constexpr int MLP_CHUNK = 128;    // samples per partial sum (fixed: the sum order)
-
-// grid (ceil(NPARAM/64), nchunk), one wave per block: lane = parameter, y = sample chunk.
-// x is feature-major [4][n] (the kernels' input layout), the rest sample-major.
-__global__ __launch_bounds__(64) void k_mlp_grad_part(const float *__restrict__ x, int n,
-                                                      const float *__restrict__ H1, const float *__restrict__ H2,
-                                                      const float *__restrict__ D1, const float *__restrict__ D2,
-                                                      const float *__restrict__ DZ, double *__restrict__ part) {
-    const int k = blockIdx.x * 64 + threadIdx.x;
-    if (k >= MLP_NPARAM) return;
-    const int s0 = blockIdx.y * MLP_CHUNK, s1 = min(n, s0 + MLP_CHUNK);
-    double acc = 0.;
-    if (k < OFF_B1) {
-        const int p = k / MLP_NIN, q = k % MLP_NIN;
-#pragma unroll 4
-        for (int s = s0; s < s1; s++) acc += (double)D1[(size_t)s * MLP_NH + p] * (double)x[(size_t)q * n + s];
-    } else if (k < OFF_W2) {
-        const int p = k - OFF_B1;
-#pragma unroll 4
-        for (int s = s0; s < s1; s++) acc += (double)D1[(size_t)s * MLP_NH + p];
-    } else if (k < OFF_B2) {
-        const int p = (k - OFF_W2) / MLP_NH, q = (k - OFF_W2) % MLP_NH;
-#pragma unroll 4
-        for (int s = s0; s < s1; s++) acc += (double)D2[(size_t)s * MLP_NH + p] * (double)H1[(size_t)s * MLP_NH + q];
-    } else if (k < OFF_W3) {
-        const int p = k - OFF_B2;
-#pragma unroll 4
-        for (int s = s0; s < s1; s++) acc += (double)D2[(size_t)s * MLP_NH + p];
-    } else if (k < OFF_B3) {
-        const int p = k - OFF_W3;
-#pragma unroll 4
-        for (int s = s0; s < s1; s++) acc += (double)DZ[s] * (double)H2[(size_t)s * MLP_NH + p];
-    } else {
-#pragma unroll 4
-        for (int s = s0; s < s1; s++) acc += (double)DZ[s];
+    double *o = part + (size_t)blockIdx.x * MLP_NPARAM;
+    auto rows_sum = [](double v) {                        // over the four lanes of a unit
+        v += __shfl_xor(v, 16);
+        return v + __shfl_xor(v, 32);
+    };
+    gb1 = rows_sum(gb1);
+    gb2 = rows_sum(gb2);
+    gw3 = rows_sum(gw3);
+#pragma unroll
+    for (int q = 0; q < MLP_NIN; q++) gw1[q] = rows_sum(gw1[q]);
+    if (r == 0) {
+        o[OFF_B1 + unit] = gb1;
+        o[OFF_B2 + unit] = gb2;
+        o[OFF_W3 + unit] = gw3;
+#pragma unroll
+        for (int q = 0; q < MLP_NIN; q++) o[OFF_W1 + unit * MLP_NIN + q] = gw1[q];
     }
-    part[(size_t)blockIdx.y * MLP_NPARAM + k] = acc;
+    // the FP64 instruction's result: row 4 j + r, column c
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[OFF_W2 + (16 * w + 4 * j + r) * MLP_NH + 16 * u + c] = g2[u][j];
+    if (t < MLP_TILE) {
+#pragma unroll
+        for (int d = 1; d < MLP_TILE; d <<= 1) {
+            gb3 += __shfl_xor(gb3, d);
+            loss += __shfl_xor(loss, d);
+        }
+        if (t == 0) {
+            o[OFF_B3] = gb3;
+            loss_part[blockIdx.x] = loss;
+        }
+    }
 }
 
-__global__ void k_mlp_grad_sum(int nchunk, const double *__restrict__ part, float *__restrict__ grad) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= MLP_NPARAM) return;
+// grad = the workgroups' sums added in order (8 runs of workgroups, then the runs); adam: theta's
+// step too.  32 parameters per workgroup.
+struct AdamStep {
+    int on;
+    float lr, b1, b2, c1, c2;
+};
+__global__ __launch_bounds__(256) void k_mlp_update(int nparts, const double *__restrict__ part, float *__restrict__ grad,
+                                                    float *__restrict__ theta, float *__restrict__ m, float *__restrict__ v,
+                                                    AdamStep a) {
+    __shared__ double s_sum[8][32];
+    const int kk = (int)threadIdx.x & 31, run = (int)threadIdx.x >> 5, k = (int)blockIdx.x * 32 + kk;
+    const int per = (nparts + 7) / 8, c1 = min(nparts, (run + 1) * per);
     double acc = 0.;
-    for (int c = 0; c < nchunk; c++) acc += part[(size_t)c * MLP_NPARAM + k];
-    grad[k] = (float)acc;
-}
-
-__global__ void k_mlp_adam(float *__restrict__ theta, const float *__restrict__ grad, float *__restrict__ m,
-                           float *__restrict__ v, float lr, float b1, float b2, float c1, float c2) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= MLP_NPARAM) return;
-    const float g = grad[k];
-    const float mk = b1 * m[k] + (1.f - b1) * g;
-    const float vk = b2 * v[k] + (1.f - b2) * g * g;
+    if (k < MLP_NPARAM)
+#pragma unroll 8
+        for (int c = run * per; c < c1; c++) acc += part[(size_t)c * MLP_NPARAM + k];
+    s_sum[run][kk] = acc;
+    __syncthreads();
+    if (threadIdx.x >= 32 || k >= MLP_NPARAM) return;
+    for (int q = 1; q < 8; q++) acc += s_sum[q][kk];
+    const float g = (float)acc;
+    grad[k] = g;
+    if (!a.on) return;
+    const float mk = a.b1 * m[k] + (1.f - a.b1) * g;
+    const float vk = a.b2 * v[k] + (1.f - a.b2) * g * g;
     m[k] = mk;
     v[k] = vk;
-    theta[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + 1e-8f);
+    theta[k] -= a.lr * (mk / a.c1) / (sqrtf(vk / a.c2) + 1e-8f);
 }
 
 // ---------------------------------------------- prediction on the matrix cores
@@ -174,7 +265,6 @@ __global__ void k_mlp_adam(float *__restrict__ theta, const float *__restrict__ 
 // (D[i][n], i = 4 (l / 16) + j, n = 16 t + l % 16) start at b2, and the output layer
 // sums w3 h2 over the 16 lanes of a row.  Agrees with k_mlp_forward to bf16 precision.
 typedef short mlp_v4s __attribute__((ext_vector_type(4)));
-typedef float mlp_v4f __attribute__((ext_vector_type(4)));
 
 __device__ inline short bf16_rn(float x) {                // round to nearest even
     const unsigned u = __float_as_uint(x);
@@ -259,13 +349,8 @@ int Forecaster::ensure(int nsamp) {
     GPLUM_ENSURE(grad, MLP_NPARAM);
     GPLUM_ENSURE(m, MLP_NPARAM);
     GPLUM_ENSURE(v, MLP_NPARAM);
-    GPLUM_ENSURE(part, (size_t)MLP_NPARAM * ceil_div(nsamp, MLP_CHUNK));
-    GPLUM_ENSURE(H1, (size_t)MLP_NH * nsamp);
-    GPLUM_ENSURE(H2, (size_t)MLP_NH * nsamp);
-    GPLUM_ENSURE(D1, (size_t)MLP_NH * nsamp);
-    GPLUM_ENSURE(D2, (size_t)MLP_NH * nsamp);
-    GPLUM_ENSURE(DZ, nsamp);
-    GPLUM_ENSURE(loss_part, ceil_div(nsamp, 256) + 1);
+    GPLUM_ENSURE(part, (size_t)MLP_NPARAM * mlp_grid(nsamp));
+    GPLUM_ENSURE(loss_part, mlp_grid(nsamp));
     return GPLUM_OK;
 }
 
@@ -309,39 +394,32 @@ int Forecaster::predict(const float *d_x, int n, float *d_lam, hipStream_t st) {
     return GPLUM_OK;
 }
 
-int Forecaster::loss_grad(const float *d_x, const float *d_y, int n, double *loss, hipStream_t st) {
+int Forecaster::gradient(const float *d_x, const float *d_y, int n, double *loss, bool step, hipStream_t st) {
     int rc = ensure(n);
     if (rc) return rc;
-    const int nb = ceil_div(n, 256);
-    hipLaunchKernelGGL(k_mlp_backward, dim3(nb), dim3(256), 0, st, theta.p, d_x, d_y, n, H1.p, H2.p, D1.p, D2.p,
-                       DZ.p, loss_part.p);
-    const int nchunk = ceil_div(n, MLP_CHUNK);
-    hipLaunchKernelGGL(k_mlp_grad_part, dim3(ceil_div(MLP_NPARAM, 64), nchunk), dim3(64), 0, st, d_x, n, H1.p,
-                       H2.p, D1.p, D2.p, DZ.p, part.p);
-    hipLaunchKernelGGL(k_mlp_grad_sum, dim3(ceil_div(MLP_NPARAM, 256)), dim3(256), 0, st, nchunk, part.p, grad.p);
+    AdamStep a{0, lr, 0.9f, 0.999f, 1.f, 1.f};
+    if (step) {
+        adam_t++;
+        a.on = 1;
+        a.c1 = 1.f - std::pow(a.b1, (float)adam_t);
+        a.c2 = 1.f - std::pow(a.b2, (float)adam_t);
+    }
+    const int grid = mlp_grid(n);
+    hipLaunchKernelGGL(k_mlp_backward, dim3(grid), dim3(256), 0, st, theta.p, d_x, d_y, n, part.p, loss_part.p);
+    hipLaunchKernelGGL(k_mlp_update, dim3(ceil_div(MLP_NPARAM, 32)), dim3(256), 0, st, grid, part.p, grad.p, theta.p, m.p, v.p,
+                       a);
     GPLUM_HIP(hipGetLastError());
     if (loss) return read_loss(n, loss, st);
     return GPLUM_OK;
 }
 
 int Forecaster::read_loss(int n, double *loss, hipStream_t st) {
-    const int nb = ceil_div(n, 256);
-    std::vector<double> h(nb);
-    GPLUM_HIP(hipMemcpyAsync(h.data(), loss_part.p, sizeof(double) * nb, hipMemcpyDeviceToHost, st));
+    std::vector<double> h(mlp_grid(n));
+    GPLUM_HIP(hipMemcpyAsync(h.data(), loss_part.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
     GPLUM_HIP(hipStreamSynchronize(st));
     double s = 0.;
     for (double x : h) s += x;
     *loss = s / n;
-    return GPLUM_OK;
-}
-
-int Forecaster::adam_step(hipStream_t st) {
-    adam_t++;
-    const float b1 = 0.9f, b2 = 0.999f;
-    const float c1 = 1.f - std::pow(b1, (float)adam_t), c2 = 1.f - std::pow(b2, (float)adam_t);
-    hipLaunchKernelGGL(k_mlp_adam, dim3(ceil_div(MLP_NPARAM, 256)), dim3(256), 0, st, theta.p, grad.p, m.p, v.p, lr,
-                       b1, b2, c1, c2);
-    GPLUM_HIP(hipGetLastError());
     return GPLUM_OK;
 }
 
@@ -407,7 +485,7 @@ extern "C" int gplum_mlp_loss_grad(const float *theta, const float *x, const flo
     GPLUM_HIP(hipMemcpyAsync(c.f.theta.p, theta, sizeof(float) * gplum::MLP_NPARAM, hipMemcpyHostToDevice, c.st));
     GPLUM_HIP(hipMemcpyAsync(c.x.p, x, sizeof(float) * 4 * n, hipMemcpyHostToDevice, c.st));
     GPLUM_HIP(hipMemcpyAsync(c.y.p, y, sizeof(float) * n, hipMemcpyHostToDevice, c.st));
-    if ((rc = c.f.loss_grad(c.x.p, c.y.p, n, loss, c.st))) return rc;
+    if ((rc = c.f.gradient(c.x.p, c.y.p, n, loss, false, c.st))) return rc;
     GPLUM_HIP(hipMemcpyAsync(grad, c.f.grad.p, sizeof(float) * gplum::MLP_NPARAM, hipMemcpyDeviceToHost, c.st));
     GPLUM_HIP(hipStreamSynchronize(c.st));
     return GPLUM_OK;
@@ -420,8 +498,9 @@ extern "C" int gplum_mlp_train(float *theta, const float *x, const float *y, int
     MlpCtx &c = t_mlp;
     int rc = mlp_ctx_init(c);
     if (rc) return rc;
-    gplum::Forecaster f;   // fresh Adam state for this call
+    gplum::Forecaster &f = c.f;   // the thread's buffers, with a fresh Adam state for this call
     if ((rc = f.ensure(n))) return rc;
+    f.adam_t = 0;
     f.lr = lr;
     GPLUM_ENSURE(c.x, 4 * (size_t)n);
     GPLUM_ENSURE(c.y, (size_t)n);
@@ -432,11 +511,10 @@ extern "C" int gplum_mlp_train(float *theta, const float *x, const float *y, int
     GPLUM_HIP(hipMemcpyAsync(c.y.p, y, sizeof(float) * n, hipMemcpyHostToDevice, c.st));
     for (int s = 0; s < n_steps; s++) {
         double *lp = (s == 0) ? loss_first : nullptr;
-        if ((rc = f.loss_grad(c.x.p, c.y.p, n, lp, c.st))) return rc;
-        if ((rc = f.adam_step(c.st))) return rc;
+        if ((rc = f.gradient(c.x.p, c.y.p, n, lp, true, c.st))) return rc;
     }
     if (loss_last) {
-        if ((rc = f.loss_grad(c.x.p, c.y.p, n, loss_last, c.st))) return rc;
+        if ((rc = f.gradient(c.x.p, c.y.p, n, loss_last, false, c.st))) return rc;
     }
     GPLUM_HIP(hipMemcpyAsync(theta, f.theta.p, sizeof(float) * gplum::MLP_NPARAM, hipMemcpyDeviceToHost, c.st));
     GPLUM_HIP(hipStreamSynchronize(c.st));

@@ -11,8 +11,7 @@ constexpr int MLP_NPARAM = MLP_NH * MLP_NIN + MLP_NH + MLP_NH * MLP_NH + MLP_NH 
 
 struct Forecaster {
     DArray<float> theta, grad, m, v;        // parameters, gradient, Adam moments
-    DArray<float> H1, H2, D1, D2, DZ;       // per-sample activations / deltas, [n][64]
-    DArray<double> loss_part, part;         // loss per block, gradient per sample chunk
+    DArray<double> loss_part, part;         // loss and gradient per workgroup
     int adam_t = 0;
     float lr = 3e-3f;
     bool initialized = false;
@@ -24,11 +23,11 @@ struct Forecaster {
     // the same rates with the hidden layer on the matrix cores (bf16 operands, FP32
     // accumulation) and hardware tanh: for sizing, not for training
     int predict(const float *d_x, int n, float *d_lam, hipStream_t st);
-    // fills grad with d(mean Poisson NLL)/d theta; loss (optional) synchronises the stream
-    int loss_grad(const float *d_x, const float *d_y, int n, double *loss, hipStream_t st);
-    // the mean loss of the last loss_grad call over its n samples (synchronises st)
+    // fills grad with d(mean Poisson NLL)/d theta (step: and takes the Adam step with it);
+    // loss (optional, of the parameters before the step) synchronises the stream
+    int gradient(const float *d_x, const float *d_y, int n, double *loss, bool step, hipStream_t st);
+    // the mean loss of the last gradient call over its n samples (synchronises st)
     int read_loss(int n, double *loss, hipStream_t st);
-    int adam_step(hipStream_t st);
 };
 
 }  // namespace gplum
