@@ -1049,47 +1049,49 @@ __device__ inline void swap32(double x, double &low, double &high) {
     low = dbl_of(lo[0], hi[0]);
     high = dbl_of(lo[1], hi[1]);
 }
-// the row values r[0..N-1] of the lane's position (N = 2: rows 0 and 1 of its pair)
-template <int N>
+// the row values r[0..3] of the lane's position
 __device__ inline void rows_of(double x, double (&r)[4]) {
-    if (N == 2) {
-        swap16(x, r[0], r[1]);
-        r[2] = r[3] = 0.;
-    } else {
-        double lo, hi;
-        swap32(x, lo, hi);
-        swap16(lo, r[0], r[1]);
-        swap16(hi, r[2], r[3]);
-    }
+    double lo, hi;
+    swap32(x, lo, hi);
+    swap16(lo, r[0], r[1]);
+    swap16(hi, r[2], r[3]);
 }
 
 // Constants of the lane-per-term path.  They are kept in vector registers (the kernel has
 // plenty and this path uses few): as scalars the compiler spills and reloads some of them in
 // every block step.
 struct TermConsts {
-    double gamma, g_1_inv, c140, c70, c84, c35, half_tree, dt_min, alpha2;
+    double gamma, g_1_inv, c140, c70, c84, c35, cm20, c3, half_tree, dt_min, alpha2;
+    // below the changeover (x < 0, K = 1) at any distance, for the Sun row
+    double sun_r_out_inv;
     __device__ explicit TermConsts(const HP &P)
-        : gamma(P.cut.gamma), g_1_inv(P.cut.g_1_inv), c140(140.), c70(70.), c84(84.), c35(35.),
-          half_tree(0.5 * P.dt_tree), dt_min(P.dt_min), alpha2(P.alpha2) {
-        asm("" : "+v"(gamma), "+v"(g_1_inv), "+v"(c140), "+v"(c70), "+v"(c84));
-        asm("" : "+v"(c35), "+v"(half_tree), "+v"(dt_min), "+v"(alpha2));
+        : gamma(P.cut.gamma), g_1_inv(P.cut.g_1_inv), c140(140.), c70(70.), c84(84.), c35(35.), cm20(-20.), c3(3.),
+          half_tree(0.5 * P.dt_tree), dt_min(P.dt_min), alpha2(P.alpha2),
+          sun_r_out_inv(P.cut.g_1_inv > 0. ? 1e300 : -1e300) {
+        asm("" : "+v"(gamma), "+v"(g_1_inv), "+v"(c140), "+v"(c70), "+v"(c84), "+v"(cm20));
+        asm("" : "+v"(c35), "+v"(c3), "+v"(half_tree), "+v"(dt_min), "+v"(alpha2));
+    }
+};
+// The corrector's and predictor's constants of integrate_pair, likewise.
+struct StepConsts {
+    double third, sixtieth, twelfth, c5, c3a, c6;
+    __device__ StepConsts()
+        : third(THIRDORDER), sixtieth(ONE_SIXTIETH), twelfth(ONE_TWELFTH), c5(5.), c3a(3. * ALPHA_POS), c6(6.) {
+        asm("" : "+v"(third), "+v"(sixtieth), "+v"(twelfth), "+v"(c5), "+v"(c3a), "+v"(c6));
     }
 };
 
-// The lane's term of a hard force evaluation, in one instruction stream for the Sun row
+// The lane's term of a hard force evaluation (dr = xj - x, d2 = |dr|^2, dv = vj - v), in one instruction stream for the Sun row
 // (star_acc_jerk: xj = vj = -0, so that xj - x = -x exactly; mT = m_sun, eps2T =
 // eps2_sun) and the partner rows (pair_term with r_out_inv = min of the two 1/r_out):
 // the Sun's (1/s, then sqrt) and the pair's (sqrt, then 1/r) sequences are both
 // evaluated from one estimate and the row's own one selected.  The Sun row's r_out_inv =
-// SUN_R_OUT_INV puts it below the changeover (x < 0), so K = 1 and dK/dt is a zero of
+// C.sun_r_out_inv puts it below the changeover (x < 0), so K = 1 and dK/dt is a zero of
 // alpha's sign: exact identities (1 K = K, alpha 1 = alpha, 3 alpha + 0 = 3 alpha) that leave
 // star_acc_jerk's acc = mj dr and jerk = mj (dv - 3 alpha dr).  need: the lane's term is used.
-constexpr double SUN_R_OUT_INV = -1e300;
-__device__ inline void term_eval(const TermConsts &C, bool sun, bool pad, bool need, double xi, double vi, double xj,
-                                 double vj, double mT, double eps2T, double r_out_inv, double &ta, double &tj) {
-    const double dr = xj - xi;
-    const double dv = vj - vi;
-    const double s = quad_sq(dr) + eps2T;
+__device__ inline void term_eval(const TermConsts &C, bool sun, bool pad, bool need, double dr, double d2, double dv,
+                                 double mT, double eps2T, double r_out_inv, double &ta, double &tj) {
+    const double s = d2 + eps2T;
     // y1: the Sun's 1/r^2, the pair's r
     double y1, rinv, r2inv;
     {
@@ -1115,13 +1117,13 @@ __device__ inline void term_eval(const TermConsts &C, bool sun, bool pad, bool n
     // cutoff_K_sel and cutoff_dKdt_sel
     const double x = (C.gamma - y1 * r_out_inv) * C.g_1_inv;
     const double x2 = x * x, x_1 = x - 1.;
-    const double poly = (((-20. * x + C.c70) * x - C.c84) * x + C.c35) * x2 * x2;
+    const double poly = (((C.cm20 * x + C.c70) * x - C.c84) * x + C.c35) * x2 * x2;
     const double slope = C.c140 * x * x * x * x_1 * x_1 * x_1 * r_out_inv * C.g_1_inv;
     const bool below = x < 0., above = x >= 1.;
     const double K = 1. - (below ? 0. : (above ? 1. : poly));
     const double dKdt = alpha * y1 * ((below || above) ? 0. : slope);
     const double alpha_c = alpha * K;
-    const double c2 = 3. * alpha_c + dKdt;
+    const double c2 = C.c3 * alpha_c + dKdt;
     ta = mj_r3 * K * dr;
     tj = mj_r3 * (K * dv - c2 * dr);
 }
@@ -1131,8 +1133,8 @@ __device__ inline void term_eval(const TermConsts &C, bool sun, bool pad, bool n
 template <int N>
 __device__ inline void gather_terms(double ta, double tj, double &as, double &js, double &ad, double &jd) {
     double ra[4], rj[4];
-    rows_of<N>(ta, ra);
-    rows_of<N>(tj, rj);
+    rows_of(ta, ra);
+    rows_of(tj, rj);
     as = ra[0];
     js = rj[0];
     ad = 0.;
@@ -1263,26 +1265,63 @@ static bool dyadic_tree(const gplum_params &p) {
     return is_pow2(p.dt_tree) && is_pow2(p.dt_min) && p.dt_min <= 0.5 * p.dt_tree && p.dt_min >= 0x1p-50 * p.dt_tree;
 }
 
-// Block steps of a cluster of N (2 to 4) particles with distinct ids from the start of the
-// soft step (the layout above; one wave; DYADIC: all of them keep to dyadic_steps).  Returns false when a block step
-// may have a collision: the state of the start of that block step is then in H (flags and twins
-// cleared) for integrate_seq.  Else the final calcGravity with potentials is done and
-// written to H.  s_m, s_ri, s_id, s_fr hold the cluster's masses, 1/r_out, ids and
-// f r_planet; s_x, s_v and s_tm are free.
+// The end of integrate_terms and integrate_pair: the final calcGravity with potentials
+// (hermite.h:466-470), one lane per particle.  vec: the lane holds component c of particle p's
+// x and v; lead: its time and dt.
+template <int N>
+__device__ inline void terms_finish(const HP &P, HardView &H, const JData &J, double *s_x, double *s_v, const double *s_ri,
+                                    const int64_t *s_id, double *s_tm, int b, int p, int c, bool vec, bool lead, double x,
+                                    double v, double time, double dt, long long &pairs) {
+    const int L = threadIdx.x;
+    __syncthreads();
+    if (vec) {
+        s_x[3 * p + c] = x;
+        s_v[3 * p + c] = v;
+    }
+    if (lead) {
+        s_tm[2 * p] = time;
+        s_tm[2 * p + 1] = dt;
+    }
+    __syncthreads();
+    if (L < N) {
+        const int gi = b + L;
+        double xi[3], vi[3], fas[3], fjs[3], fad[3], fjd[3], phs = 0., phd = 0.;
+        ld3(s_x, L, xi);
+        ld3(s_v, L, vi);
+        star_acc_jerk(P, xi, vi, fas, fjs, &phs);
+        gravity_loop_lane<false>(P, J, N, L, s_id[L], xi, vi, s_ri[L], fad, fjd, &phd);
+        pairs += N - 1;
+        st3(H.pos, gi, xi); st3(H.vel, gi, vi);
+        st3(H.acc_s, gi, fas); st3(H.jerk_s, gi, fjs);
+        st3(H.acc_d, gi, fad); st3(H.jerk_d, gi, fjd);
+        H.time[gi] = s_tm[2 * L];
+        H.dt[gi] = s_tm[2 * L + 1];
+        H.phi_s[gi] = phs;
+        H.phi_d[gi] = phd;
+        H.flags[gi] &= ~(GPLUM_FLAG_DEAD | GPLUM_FLAG_MERGED);
+        H.twin_of[gi] = -1;
+    }
+    __syncthreads();
+}
+
+// Block steps of a cluster of N (3 or 4) particles with distinct ids from the start of the
+// soft step (the layout above; one wave; DYADIC: all of them keep to dyadic_steps).  Returns
+// false when a block step may have a collision: the state of the start of that block step is
+// then in H (flags and twins cleared) for integrate_seq.  Else the final calcGravity with
+// potentials is done and written to H.  s_m, s_ri, s_id, s_fr hold the cluster's masses, 1/r_out,
+// ids and f r_planet; s_x, s_v and s_tm are free.
 template <int N, bool DYADIC>
 __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double *s_x, double *s_v, double *s_m,
                                 double *s_ri, int64_t *s_id, double *s_fr, double *s_tm, int b, double &sys_time,
                                 long long &loop, long long &pairs) {
     constexpr int m = N - 1;
     const int L = threadIdx.x;
-    const int T = (N == 2) ? ((L >> 4) & 1) : (L >> 4);
-    const int p = (N == 2) ? ((L >> 2) & 1) : ((L >> 2) & 3);
+    const int T = L >> 4, p = (L >> 2) & 3;
     const int c = L & 3;
     // lanes of a particle: every row takes part in the evaluations, so that the cross-row
     // swaps read computed values (rows T >= N, 3 bodies, evaluate a don't-care term)
     const bool own = p < N;
     const bool row = own && T < N;                  // lanes of a term of a particle
-    const bool first = (N == 2) ? L < 32 && ((L >> 2) & 3) < 2 : true;   // not a copy
     const bool sun = T == 0, pad = c == 3;
     const int j = (T >= 1) ? (T - 1) + ((T - 1) >= p ? 1 : 0) : p;   // the row's partner
     const int jc = (j < N) ? j : 0, pc = own ? p : 0;
@@ -1290,7 +1329,7 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
     const TermConsts C(P);
     const double mT = sun ? P.m_sun : s_m[jc];
     const double eps2T = sun ? P.eps2_sun : P.eps2;
-    const double r_out_inv = sun ? SUN_R_OUT_INV : dmin(s_ri[pc], s_ri[jc]);
+    const double r_out_inv = sun ? C.sun_r_out_inv : dmin(s_ri[pc], s_ri[jc]);
     const double etaT = sun ? P.eta_sun : P.eta;
     const double r2c = s_fr[pc] + s_fr[jc];
     const double col_thr = COL_FILTER * r2c * r2c;
@@ -1308,7 +1347,7 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
         acc0 = H.acc0[g];
     }
     const double acc0T = sun ? 0. : acc0;
-    const bool lead = row && sun && c == 0 && first;
+    const bool lead = row && sun && c == 0;
     double as = 0., js = 0., ad = 0., jd = 0., a2s = 0., a3s = 0., a2d = 0., a3d = 0.;
     {
         // initial calcGravity (hermite.h:259-270) at the current state
@@ -1316,14 +1355,15 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
         if (sun) { xj = -0.; vj = -0.; }
         if (own) {
             double ta, tj;
-            term_eval(C, sun, pad, row, x, v, xj, vj, mT, eps2T, r_out_inv, ta, tj);
+            const double dr = xj - x;
+            term_eval(C, sun, pad, row, dr, quad_sq(dr), vj - v, mT, eps2T, r_out_inv, ta, tj);
             gather_terms<N>(ta, tj, as, js, ad, jd);
         }
     }
-    // the smallest value of the particles (quads of a row; 2 bodies: quads 2, 3 are copies)
+    // the smallest value of the particles (quads of a row)
     auto smallest = [](double u) __attribute__((always_inline)) {
         u = __builtin_fmin(u, dpp_f64<DPP_ROW_ROR4>(u));
-        if (N > 2) u = __builtin_fmin(u, dpp_f64<DPP_ROW_ROR8>(u));
+        u = __builtin_fmin(u, dpp_f64<DPP_ROW_ROR8>(u));
         return readlane_f64(u, 0);
     };
     double t_s = smallest(own ? time + dt : 1.e10);
@@ -1333,23 +1373,12 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
         const double a0s = as, j0s = js, a0d = ad, j0d = jd;
         double xp = 0., vp = 0.;
         predict_one(Dt, x, v, as, js, ad, jd, xp, vp);
-        double xj, vj;
-        if (N == 2) {
-            // the partner of quad q is quad q ^ 1, which row_ror:4 brings (quads 2, 3 are
-            // copies of 0, 1)
-            xj = dpp_f64<DPP_ROW_ROR4>(xp);
-            vj = dpp_f64<DPP_ROW_ROR4>(vp);
-        } else {
-            xj = __shfl(xp, src);
-            vj = __shfl(vp, src);
-        }
+        double xj = __shfl(xp, src), vj = __shfl(vp, src);
         if (sun) { xj = -0.; vj = -0.; }
-        if (P.collision) {
-            // collisionDetermination: a pair with R = |dx| / (f_i R_i + f_j R_j) < 1
-            const double dx = xp - xj;
-            const double d2 = quad_sq(dx);
-            if (__ballot(col_row && d2 < col_thr)) { handover = true; break; }   // R itself is left to integrate_seq
-        }
+        // collisionDetermination: a pair with R = |dr| / (f_i R_i + f_j R_j) < 1; R itself is left
+        // to integrate_seq
+        const double drp = xj - xp, d2p = quad_sq(drp);
+        if (__ballot(col_row && d2p < col_thr)) { handover = true; break; }
         if (own && time + dt == t_s) {
             if (lead) pairs += 3 * (long long)m;
             const double Dt2 = Dt * Dt;
@@ -1358,12 +1387,13 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
             const double Dt_inv2 = Dt_inv * Dt_inv;
             const double Dt_inv3 = Dt_inv2 * Dt_inv;
             double ta, tj;
-            term_eval(C, sun, pad, row, xp, vp, xj, vj, mT, eps2T, r_out_inv, ta, tj);
+            term_eval(C, sun, pad, row, drp, d2p, vj - vp, mT, eps2T, r_out_inv, ta, tj);
             gather_terms<N>(ta, tj, as, js, ad, jd);
             for (int ite = 0; ite < 2; ite++) {
                 correct_one(Dt, Dt2, Dt_inv2, Dt_inv3, xp, vp, as, a0s, j0s, js, ad, a0d, j0d, jd, x, v, a2s, a3s,
                             a2d, a3d);
-                term_eval(C, sun, pad, row, x, v, xj, vj, mT, eps2T, r_out_inv, ta, tj);
+                const double dr = xj - x;
+                term_eval(C, sun, pad, row, dr, quad_sq(dr), vj - v, mT, eps2T, r_out_inv, ta, tj);
                 gather_terms<N>(ta, tj, as, js, ad, jd);
             }
             time += Dt;
@@ -1378,7 +1408,7 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
     }
     if (handover) {
         // the state at the start of this block step, for integrate_seq
-        if (row && sun && !pad && first) {
+        if (row && sun && !pad) {
             H.pos[3 * g + c] = x; H.vel[3 * g + c] = v;
             H.acc_s[3 * g + c] = as; H.jerk_s[3 * g + c] = js;
             H.acc_d[3 * g + c] = ad; H.jerk_d[3 * g + c] = jd;
@@ -1391,36 +1421,125 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
         }
         return false;
     }
-    // final calcGravity with potentials (hermite.h:466-470), one lane per particle
-    __syncthreads();
-    if (row && sun && !pad && first) {
-        s_x[3 * p + c] = x;
-        s_v[3 * p + c] = v;
+    terms_finish<N>(P, H, J, s_x, s_v, s_ri, s_id, s_tm, b, p, c, row && sun && !pad, lead, x, v, time, dt, pairs);
+    return true;
+}
+
+// integrate_terms for two bodies, whose chain bounds most soft steps (the cluster with the most
+// block steps is nearly always a pair): row T keeps only its own term's acc and jerk (Sun or
+// partner) and their derivatives, and the rows are added where the predictor and the corrector
+// add them (as + ad, A2_s + A2_d, ...), so the corrector is evaluated once for both.  Bound by
+// instruction issue of its one wave (560 per block step of 4 cycles; 606 when every row kept both
+// terms: 2 bodies 1.06 us per block step in a 100k disk).
+template <bool DYADIC>
+__device__ bool integrate_pair(const HP &P, HardView &H, const JData &J, double *s_x, double *s_v, double *s_m,
+                               double *s_ri, int64_t *s_id, double *s_fr, double *s_tm, int b, double &sys_time,
+                               long long &loop, long long &pairs) {
+    const int L = threadIdx.x;
+    const int T = (L >> 4) & 1, p = (L >> 2) & 1, c = L & 3;
+    const bool sun = T == 0, pad = c == 3;
+    const bool first = L < 32 && ((L >> 2) & 3) < 2;             // not a copy
+    const int g = b + p;
+    const TermConsts C(P);
+    const StepConsts K;
+    const double mT = sun ? P.m_sun : s_m[1 - p];
+    const double eps2T = sun ? P.eps2_sun : P.eps2;
+    const double r_out_inv = sun ? C.sun_r_out_inv : dmin(s_ri[p], s_ri[1 - p]);
+    const double etaT = sun ? P.eta_sun : P.eta;
+    // the partner's term is added to zero (gravity_loop_lane), the Sun's is not: + -0 changes nothing
+    const double zero = sun ? -0. : 0.;
+    const double r2c = s_fr[0] + s_fr[1];
+    const double col_thr = (P.collision && !sun) ? COL_FILTER * r2c * r2c : -1.;
+    const double time_end = P.dt_tree;
+    double x = pad ? 0. : H.pos[3 * g + c], v = pad ? 0. : H.vel[3 * g + c];
+    double time = H.time[g], dt = H.dt[g];
+    const double acc0T = sun ? 0. : H.acc0[g];
+    const bool lead = sun && c == 0 && first;
+    // the partner is the next quad (quads 2, 3 are copies of 0, 1)
+    auto partner = [&](double u) __attribute__((always_inline)) { return sun ? -0. : dpp_f64<DPP_ROW_ROR4>(u); };
+    auto both = [](double u) __attribute__((always_inline)) {
+        double even, odd;
+        swap16(u, even, odd);
+        return even + odd;
+    };
+    auto smallest = [](double u) __attribute__((always_inline)) {
+        return readlane_f64(__builtin_fmin(u, dpp_f64<DPP_ROW_ROR4>(u)), 0);
+    };
+    double a, j, a2 = 0., a3 = 0.;
+    auto force = [&](double dr, double d2, double dv) __attribute__((always_inline)) {
+        double ta, tj;
+        term_eval(C, sun, pad, true, dr, d2, dv, mT, eps2T, r_out_inv, ta, tj);
+        a = ta + zero;
+        j = tj + zero;
+    };
+    {
+        // initial calcGravity (hermite.h:259-270) at the current state
+        const double dr = partner(x) - x;
+        force(dr, quad_sq(dr), partner(v) - v);
     }
-    if (lead) {
-        s_tm[2 * p] = time;
-        s_tm[2 * p + 1] = dt;
+    double t_next = time + dt;
+    double t_s = smallest(t_next);
+    bool handover = false;
+    int n_eval = 0;
+    while (sys_time < time_end && loop < BLOCK_STEP_CAP) {
+        const double Dt = t_s - time;
+        const double acc_sd = both(a), jerk_sd = both(j);
+        const double xp = x + Dt * (v + Dt * (SECONDORDER * acc_sd + K.third * Dt * jerk_sd));
+        const double vp = v + Dt * (acc_sd + Dt * SECONDORDER * jerk_sd);
+        const double xj = partner(xp), vj = partner(vp);
+        // collisionDetermination: R = |dr| / (f_i R_i + f_j R_j) < 1; R itself is left to
+        // integrate_seq
+        const double drp = xj - xp, d2p = quad_sq(drp);
+        if (__ballot(d2p < col_thr)) { handover = true; break; }
+        if (t_next == t_s) {
+            n_eval++;
+            const double Dt2 = Dt * Dt;
+            // DYADIC: Dt = dt, a power of two
+            const double Dt_inv = DYADIC ? hi_word(0x7FE00000 - hi_of(Dt)) : recip_step(Dt);
+            const double Dt_inv2 = Dt_inv * Dt_inv, Dt_inv3 = Dt_inv2 * Dt_inv;
+            const double a0 = a, J0 = Dt * j;
+            force(drp, d2p, vj - vp);
+            for (int ite = 0; ite < 2; ite++) {
+                const double Am = a - a0;
+                const double J1 = Dt * j;
+                const double A2 = C.c3 * Am - (J1 + 2. * J0);
+                const double A3 = -2. * Am + (J1 + J0);
+                a2 = 2. * Dt_inv2 * (A2 + C.c3 * A3);
+                a3 = K.c6 * Dt_inv3 * A3;
+                if (!DYADIC && !sun) a3 = K.c6 * A3 * Dt_inv3;
+                const double A2_sd = both(A2), A3_sd = both(A3);
+                x = xp + K.sixtieth * Dt2 * (K.c5 * A2_sd + K.c3a * A3_sd);
+                v = vp + K.twelfth * Dt * (4. * A2_sd + C.c3 * A3_sd);
+                const double dr = xj - x;
+                force(dr, quad_sq(dr), vj - v);
+            }
+            time += Dt;
+            dt = dt_block_rows<2, DYADIC>(C, time, dt, etaT, acc0T, a, j, a2, a3);
+            t_next = time + dt;
+        }
+        // the system time is asked for once the next block time has reached the end: before
+        // that some particle's time is below it
+        t_s = smallest(t_next);
+        if (!(t_s < time_end)) sys_time = smallest(time);
+        loop++;
     }
-    __syncthreads();
-    if (L < N) {
-        const int gi = b + L;
-        double xi[3], vi[3], fas[3], fjs[3], fad[3], fjd[3], phs = 0., phd = 0.;
-        ld3(s_x, L, xi);
-        ld3(s_v, L, vi);
-        star_acc_jerk(P, xi, vi, fas, fjs, &phs);
-        gravity_loop_lane<false>(P, J, N, L, s_id[L], xi, vi, s_ri[L], fad, fjd, &phd);
-        pairs += m;
-        st3(H.pos, gi, xi); st3(H.vel, gi, vi);
-        st3(H.acc_s, gi, fas); st3(H.jerk_s, gi, fjs);
-        st3(H.acc_d, gi, fad); st3(H.jerk_d, gi, fjd);
-        H.time[gi] = s_tm[2 * L];
-        H.dt[gi] = s_tm[2 * L + 1];
-        H.phi_s[gi] = phs;
-        H.phi_d[gi] = phd;
-        H.flags[gi] &= ~(GPLUM_FLAG_DEAD | GPLUM_FLAG_MERGED);
-        H.twin_of[gi] = -1;
+    if (lead) pairs += 3 * (long long)n_eval;
+    if (handover) {
+        // the state at the start of this block step, for integrate_seq
+        if (!pad && first) {
+            if (sun) { H.pos[3 * g + c] = x; H.vel[3 * g + c] = v; }
+            (sun ? H.acc_s : H.acc_d)[3 * g + c] = a;
+            (sun ? H.jerk_s : H.jerk_d)[3 * g + c] = j;
+        }
+        if (lead) {
+            H.time[g] = time;
+            H.dt[g] = dt;
+            H.flags[g] &= ~(GPLUM_FLAG_DEAD | GPLUM_FLAG_MERGED);
+            H.twin_of[g] = -1;
+        }
+        return false;
     }
-    __syncthreads();
+    terms_finish<2>(P, H, J, s_x, s_v, s_ri, s_id, s_tm, b, p, c, sun && !pad && first, lead, x, v, time, dt, pairs);
     return true;
 }
 
@@ -1517,7 +1636,8 @@ __global__ __launch_bounds__(HERMITE_BLOCK) void k_hermite_small(HP P_arg, HardV
                     return integrate_terms<N.value, DYADIC>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b, sys_time,
                                                             loop, pairs);
                 };
-                const bool done = (n == 2)   ? terms(std::integral_constant<int, 2>())
+                const bool done = (n == 2) ? integrate_pair<DYADIC>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b,
+                                                                    sys_time, loop, pairs)
                                   : (n == 3) ? terms(std::integral_constant<int, 3>())
                                              : terms(std::integral_constant<int, 4>());
                 if (done) return;
