@@ -574,6 +574,145 @@ __global__ void k_flag01(int n, const int32_t *__restrict__ flag, int32_t *__res
     if (a < n) out[a] = flag[a] ? 1 : 0;
 }
 
+// ------------------------------------------------- the whole tree in one workgroup
+//
+// Up to TREE_SMALL particles the level, moment and group kernels above are launch latency: 4
+// dependent launches per level of a few hundred nodes.  Here one workgroup builds all of it, the
+// keys in LDS, with a barrier between the levels: bound by the latency of the levels' few
+// dependent loads.  The same nodes in the same order, and node_moments in the same order of
+// operations, so the results are the same bits.  A step's whole tree part (sort to walk), level
+// kernels -> here, us: 300 particles 190 -> 112, 1000 222 -> 130, 3000 251 -> 164, 5000 271 -> 200,
+// 8192 289 -> 240 (linear in the particles: beyond, the level kernels' 256 workgroups win).
+constexpr int TREE_SMALL = 8192;
+constexpr int SMALL_BLOCK = 1024;
+
+struct SmallTree {
+    const uint64_t *key;
+    const double *pos, *mass, *rsearch;
+    int32_t *lvl, *start, *count, *level, *parent, *child, *nchild;
+    double *nm, *ncom, *nq, *bmin, *bmax, *nrs;
+    int32_t *gnode, *gstart, *gcount, *ng;
+};
+
+// exclusive prefix of v over the workgroup's threads; *total: the sum
+__device__ inline int small_scan(int v, int *s_w, int *total) {
+    int tot;
+    int ex = wave_excl_scan(v, &tot);
+    if (__lane_id() == 0) s_w[threadIdx.x >> 6] = tot;
+    __syncthreads();
+    int all = 0;
+    for (int w = 0; w < SMALL_BLOCK / 64; w++) {
+        if (w < (int)(threadIdx.x >> 6)) ex += s_w[w];
+        all += s_w[w];
+    }
+    __syncthreads();
+    *total = all;
+    return ex;
+}
+
+__global__ __launch_bounds__(SMALL_BLOCK) void k_tree_small(int n, int n_leaf, int cap, int G, SmallTree t) {
+    __shared__ uint64_t s_key[TREE_SMALL];
+    __shared__ int s_flag[TREE_SMALL];
+    __shared__ int s_lvl[MAXLEVEL + 3], s_w[SMALL_BLOCK / 64];
+    const int tid = (int)threadIdx.x;
+    for (int a = tid; a < n; a += SMALL_BLOCK) {
+        s_key[a] = t.key[a];
+        s_flag[a] = 0;
+    }
+    if (tid == 0) {
+        t.start[0] = 0; t.count[0] = n; t.level[0] = 0; t.parent[0] = -1;
+        s_lvl[0] = 0;
+        s_lvl[1] = 1;
+    }
+    __syncthreads();
+    // levels: eight lanes per node, lane d the child of digit d; the children of a level in
+    // node and digit order
+    int L = 0, err = 0;
+    for (; L <= MAXLEVEL; L++) {
+        const int lb = s_lvl[L], le = s_lvl[L + 1];
+        if (le <= lb) break;
+        int next = le;
+        for (int r0 = lb; r0 < le; r0 += SMALL_BLOCK / 8) {
+            const int c = r0 + (tid >> 3), d = tid & 7;
+            int s = 0, bnd = 0;
+            bool split = false;
+            if (c < le) {
+                const int cnt = t.count[c];
+                s = t.start[c];
+                split = cnt > n_leaf && L < MAXLEVEL;
+                if (split) {                 // the end of digit d: the first key of a larger one
+                    int lo = s, hi = s + cnt;
+                    if (d == 7) lo = hi;
+                    while (lo < hi) {
+                        const int mid = (lo + hi) >> 1;
+                        if (digit_at(s_key[mid], L) <= d) lo = mid + 1; else hi = mid;
+                    }
+                    bnd = lo;
+                }
+            }
+            int prev = __shfl_up(bnd, 1, 8);
+            if (d == 0) prev = s;
+            const bool has = split && bnd > prev;
+            const int nc = __popcll((__ballot(has) >> (__lane_id() & 56)) & 0xFFull);
+            int total;
+            const int w = next + small_scan(has ? 1 : 0, s_w, &total);
+            if (has && w < cap) {
+                t.start[w] = prev; t.count[w] = bnd - prev; t.level[w] = L + 1; t.parent[w] = c;
+            }
+            if (c < le && d == 0) {
+                t.nchild[c] = nc;
+                t.child[c] = nc ? w : -1;
+            }
+            next += total;
+        }
+        if (next > cap) { err = 1; next = le; }
+        if (tid == 0) s_lvl[L + 2] = next;
+        __syncthreads();
+        if (err) break;
+    }
+    // the levels past the last one are empty
+    const int filled = err ? L + 2 : L + 1;
+    if (tid == 0)
+        for (int k = filled + 1; k <= MAXLEVEL + 2; k++) s_lvl[k] = s_lvl[filled];
+    __syncthreads();
+    if (tid <= LVL_ERR) t.lvl[tid] = tid <= MAXLEVEL + 2 ? s_lvl[tid] : tid == LVL_ERR ? err : 0;
+    if (err) {
+        if (tid == 0) *t.ng = 0;
+        return;
+    }
+    for (int l = L - 1; l >= 0; l--) {
+        const int le = s_lvl[l + 1];
+        for (int c = s_lvl[l] + tid; c < le; c += SMALL_BLOCK)
+            node_moments(c, t.pos, t.mass, t.rsearch, t.start, t.count, t.child, t.nchild, t.nm, t.ncom, t.nq, t.bmin, t.bmax,
+                         t.nrs);
+        __syncthreads();
+    }
+    // i-groups (k_group_flags, k_group_write)
+    for (int c = tid; c < s_lvl[L]; c += SMALL_BLOCK) {
+        const int cnt = t.count[c];
+        const bool cand = (cnt <= G) || (t.nchild[c] == 0);
+        const bool top = (t.parent[c] < 0) || (t.count[t.parent[c]] > G);
+        if (!(cand && top)) continue;
+        for (int off = 0; off < cnt; off += G) s_flag[t.start[c] + off] = c + 1;
+    }
+    __syncthreads();
+    int base = 0;
+    for (int a0 = 0; a0 < n; a0 += SMALL_BLOCK) {
+        const int a = a0 + tid;
+        const int f = a < n ? s_flag[a] : 0;
+        int total;
+        const int g = base + small_scan(f ? 1 : 0, s_w, &total);
+        if (f) {
+            const int c = f - 1, rem = t.start[c] + t.count[c] - a;
+            t.gnode[g] = c;
+            t.gstart[g] = a;
+            t.gcount[g] = rem < G ? rem : G;
+        }
+        base += total;
+    }
+    if (tid == 0) *t.ng = base;
+}
+
 // ------------------------------------------------------------------- walk
 
 // One pass: workgroup b owns the list regions [b*cap_q, (b+1)*cap_q) of the three
@@ -842,9 +981,21 @@ int tree_build_nodes(Tree &t, const gplum_params &p, const double *d_pos, const 
     GPLUM_ENSURE(t.group_node, std::max(n, 1));
     GPLUM_ENSURE(t.group_start, std::max(n, 1));
     GPLUM_ENSURE(t.group_count, std::max(n, 1));
+    GPLUM_ENSURE(t.lvl, LVL_ERR + 5);
+    t.n_part = n;
+    t.n_group = -1;
+    if (n > 0 && n <= TREE_SMALL && n < t.coop_min) {   // a coop_min below n asks for the level kernels
+        t.L_end = MAXLEVEL + 1;              // whole: nothing is left for the walk to finish
+        const SmallTree q{t.key.p, d_pos, d_mass, d_rsearch, t.lvl.p, t.node_start.p, t.node_count.p, t.node_level.p,
+                          t.node_parent.p, t.node_child.p, t.node_nchild.p, t.node_mass.p, t.node_com.p, t.node_quad.p,
+                          t.node_bmin.p, t.node_bmax.p, t.node_rs.p, t.group_node.p, t.group_start.p, t.group_count.p,
+                          t.ng_dev.p};
+        hipLaunchKernelGGL(k_tree_small, dim3(1), dim3(SMALL_BLOCK), 0, st, n, p.n_leaf_limit, cap, p.n_group_limit, q);
+        GPLUM_HIP(hipGetLastError());
+        return GPLUM_OK;
+    }
     hipLaunchKernelGGL(k_root, dim3(1), dim3(1), 0, st, n, t.node_start.p, t.node_count.p,
                        t.node_level.p, t.node_parent.p);
-    GPLUM_ENSURE(t.lvl, LVL_ERR + 5);
     hipLaunchKernelGGL(k_lvl_init, dim3(1), dim3(64), 0, st, t.lvl.p);
     GPLUM_ENSURE(t.lvl_part, LEVEL_GRID);
     GPLUM_ENSURE(t.lvl_bnd, 8 * ((size_t)n + 64));   // a level holds at most n nodes
@@ -857,8 +1008,6 @@ int tree_build_nodes(Tree &t, const gplum_params &p, const double *d_pos, const 
     t.cap = cap;
     t.L_end = t.n_level > 0 ? std::min(MAXLEVEL + 1, t.n_level + 2) : MAXLEVEL + 1;
     launch_levels(t, p, 0, t.L_end, cap, st);
-    t.n_part = n;
-    t.n_group = -1;
     return launch_moments_groups(t, p, t.L_end, st);
 }
 
