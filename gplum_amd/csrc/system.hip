@@ -708,6 +708,7 @@ __global__ __launch_bounds__(HSTAT_BLOCK) void k_hard_stats(int ncl, const int *
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
+            if (c00 + u * HSTAT_BLOCK >= ncl) break;
             const int c = c00 + u * HSTAT_BLOCK + t;
             if (c < ncl) {
                 if (b[u] < 0) s_cap = 1;
@@ -733,10 +734,22 @@ __global__ __launch_bounds__(HSTAT_BLOCK) void k_hard_stats(int ncl, const int *
             __syncthreads();
         }
     }
-    atomicAdd(&s_sum[0], bs);
-    atomicAdd(&s_sum[1], pr);
-    atomicAdd(&s_sum[2], nc);
-    atomicMax(&s_max, mx);
+    // over the wave first: 1024 lanes adding to one LDS word take their turns (20 us for 88 clusters,
+    // with the empty rounds; now 5 us)
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        bs += __shfl_xor(bs, d);
+        pr += __shfl_xor(pr, d);
+        nc += __shfl_xor(nc, d);
+        const unsigned long long o = __shfl_xor(mx, d);
+        mx = o > mx ? o : mx;
+    }
+    if (lane == 0) {
+        atomicAdd(&s_sum[0], bs);
+        atomicAdd(&s_sum[1], pr);
+        atomicAdd(&s_sum[2], nc);
+        atomicMax(&s_max, mx);
+    }
     __syncthreads();
     // the dissipated energies of the collided clusters, gathered by all threads and
     // summed by one in ascending cluster order
