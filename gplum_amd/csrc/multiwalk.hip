@@ -116,7 +116,9 @@ std::vector<SoftGroup> walk_groups(TagCtx *c, int n_walk, const int *n_epi, cons
         for (int w = 0; w < n_walk; w++) n += ((long long)n_epi[w] + per_wg - 1) / per_wg;
         return n;
     };
-    direct_lanes(count, [&](auto LI) { c->i_lanes = LI.value; });
+    long long entries = 0;
+    for (int w = 0; w < n_walk; w++) entries += (long long)n_epj[w] + n_spj[w];
+    direct_lanes(entries / std::max(1, n_walk), count, [&](auto LI) { c->i_lanes = LI.value; });
     const int per_wg = DIRECT_IPL * c->i_lanes;
     c->i_off.assign(n_walk + 1, 0);
     long long io = 0, jo = 0, so = 0;

@@ -228,7 +228,7 @@ __global__ __launch_bounds__(DIRECT_BLOCK) void k_direct_f32(const SoftGroup *__
     }
 }
 
-// LI: the most i-lanes that still leave enough workgroups.  More i-lanes mean fewer workgroups
+// LI: the most i-lanes that still leave enough workgroups (or enough for a short list, below).  More i-lanes mean fewer workgroups
 // that each stage the j list, fewer workgroups mean idle CUs: up to 8 i-lanes about one per
 // CU is enough, above, where staging is under a tenth of the work, two (both resident).
 // EP-EP, us, LI = 2 / 4 / 8 / 16 / 32 / 64 (the chosen one starred; in brackets a workgroup of
@@ -240,12 +240,19 @@ __global__ __launch_bounds__(DIRECT_BLOCK) void k_direct_f32(const SoftGroup *__
 //   20000 x 20000    669 / 477 / 380 / *407 / 508 / 608         (3075)
 //   65536 x 65536    6647 / 4686 / 3711 / 3301 / 3179 / *3251   (10050; now 1.3 T pairs/s)
 constexpr int direct_min_wg(int li) { return li <= 8 ? 240 : 500; }
+// A short list takes as many i-lanes as leave its quads a j-lane each: more j-lanes only make the
+// sum over them longer.  us: 8 x 32 6.6 / 6.2 / 5.4 / 5.0 / 4.7 / *4.6, 64 x 64 6.8 / 6.4 / 6.0 / 5.6 /
+// *5.5 / 5.8, 120 x 120 6.9 / 6.5 / 6.2 / *5.8 / 6.7 / 8.5, 64 x 256 6.9 / 6.7 / *6.4 / 6.7 / 8.4 / 11.4,
+// 60 x 500 7.2 / *7.2 / 7.5 / 8.9 / 12.4 / 18.8, 2000 x 200 10.1 / 6.9 / *6.6 / 7.1 / 7.8 / 10.6.
+constexpr int DIRECT_SHORT = DIRECT_WAVES * 64 * 4;
 
-// calls f(LI) with the rule's LI; count(i-particles per workgroup): the workgroups of the call
+// calls f(LI) with the rule's LI; entries: of a list (the average of several); count(i-particles
+// per workgroup): the workgroups of the call
 template <class COUNT, class F>
-void direct_lanes(COUNT count, F f) {
+void direct_lanes(long long entries, COUNT count, F f) {
     auto fits = [&](auto LI) {
-        if (LI.value > 2 && count(DIRECT_IPL * LI.value) < direct_min_wg(LI.value)) return false;
+        if (LI.value > 2 && LI.value * entries > DIRECT_SHORT && count(DIRECT_IPL * LI.value) < direct_min_wg(LI.value))
+            return false;
         f(LI);
         return true;
     };
@@ -276,7 +283,7 @@ void launch_direct_f32(const gplum_epi *epi, int ni, typename J::Src js, int nj,
     one.ni = ni;
     one.nj = one.ns = nj;
     auto count = [&](int per_wg) { return ceil_div(ni, per_wg); };
-    direct_lanes(count, [&](auto LI) {
+    direct_lanes(nj, count, [&](auto LI) {
         hipLaunchKernelGGL((k_direct_f32<MODE, LI.value, J, J>), dim3(count(DIRECT_IPL * LI.value)), dim3(DIRECT_BLOCK), 0, st,
                            nullptr, one, SrcEPI{epi}, js, js, SinkForce{force}, eps2);
     });

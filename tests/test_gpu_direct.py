@@ -1,6 +1,7 @@
 """The FP32 functors at the edges of their kernel: the i-counts where the number of i-lanes per
-wave changes (1912/1913 ... 63872/63873) and the smallest, j-counts around a tile (512) and
-its remainders, an i-array that is accumulated into, against the FP64 sums.
+wave changes (1912/1913 ... 63872/63873) and the smallest, the j-counts where it does (32/33 ...
+512/513), j-counts around a tile (512) and its remainders, an i-array that is accumulated into,
+against the FP64 sums.
 
 Tolerance: a pair term carries at most 16 roundings of 2^-24 (relative coordinates, 1/r and
 its cube, products), an FP32 run of at most 33 additions 33 more, and the sum over the runs is
@@ -36,9 +37,10 @@ def check(force, start, a64, p64, sa, sp):
     assert np.all(err_p <= TOL * (sp + np.abs(start["phi"])))
 
 
-@pytest.mark.parametrize("ni,nj", [(1, 0), (1, 513), (3, 1), (4, 255), (5, 511), (9, 512), (130, 1025), (1912, 40), (1913, 1029),
-                                   (3824, 33), (3825, 33), (15968, 17), (15969, 600), (31936, 9), (31937, 9), (63872, 65),
-                                   (63873, 65)])
+@pytest.mark.parametrize("ni,nj", [(1, 0), (1, 513), (3, 1), (4, 255), (5, 511), (9, 512), (130, 1025), (1912, 1029),
+                                   (1913, 1029), (3824, 300), (3825, 300), (15968, 130), (15969, 600), (31936, 70),
+                                   (31937, 70), (63872, 65), (63873, 65), (41, 4), (129, 32), (129, 33), (65, 64), (65, 65),
+                                   (33, 128), (33, 129), (17, 256), (17, 257), (9, 513)])
 def test_functors_at_kernel_edges(oracle_lib, ni, nj):
     rng = np.random.default_rng(ni + nj)
     n = max(ni, nj)
