@@ -7,7 +7,7 @@
 // the active particles with two P(EC) iterations and updates their block steps.
 // The active particles of one block step are independent (each reads only the
 // predicted positions of the others), so they are corrected in parallel.  Clusters of 2 to
-// 4 bodies hold their state in registers (integrate_terms), those of up to HERMITE_LDS in
+// 4 bodies hold their state in registers (integrate_pair, integrate_terms), those of up to HERMITE_LDS in
 // LDS (hermite_lds.hpp), larger ones in global memory.
 // The kernels are persistent: workgroups pull clusters (costliest first: estimated block
 // steps times size) from an atomic queue until it is empty.
@@ -31,7 +31,7 @@ struct HP {                                  // physics constants for the kernel
     double m_sun, eps2, eps2_sun, dt_tree, dt_min, eta, eta_0, eta_sun, eta_sun0, alpha2;
     Cutoff cut;
     int collision;
-    int terms_max;     // clusters of 2 .. terms_max (<= 4) bodies run integrate_terms
+    int terms_max;     // clusters of 2 .. terms_max (<= 4) bodies run integrate_pair, integrate_terms
 };
 
 __device__ inline double dmin(double a, double b) { return (b < a) ? b : a; }
