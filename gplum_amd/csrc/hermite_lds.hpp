@@ -16,7 +16,7 @@
 // (hermite.h:224-479), so the results are those of the other paths bit for bit.
 //
 // What bounds it: the latency of three pair terms (each a correctly rounded FP64 square
-// root and division in sequence), the sums over j and seven barriers per block step; the
+// root and reciprocal), the sums over j and seven barriers per block step; the
 // chip's FP64 rate is far away (a cluster occupies one CU).  Measured on one cluster, us per
 // block step, against one lane per particle in registers and, from the first merger on, one
 // lane per particle in global memory (up to 64 members), or lane groups of 8 to 64 lanes (above):
