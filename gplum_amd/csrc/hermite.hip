@@ -738,7 +738,7 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// The active-particle correction of integrate_from for clusters above HARD_SEQ_MAX
+// The active-particle correction of the global-memory path for clusters above HARD_SEQ_MAX
 // particles (H.act marks the active ones): the k-th active particle (ascending index)
 // goes to wave k mod (waves per workgroup), and the wave's 64 lanes evaluate its hard
 // force together (coop_pair_sum); every lane carries the same particle state in
