@@ -6,6 +6,7 @@
 // (mode 1) or with one launch per cluster (mode 0, the plain comparator).
 // gplum_hard_integrate_graph captures the persistent launch into a hipGraph and
 // replays it.
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -59,12 +60,14 @@ int download(std::vector<T> &h, const DArray<T> &d, hipStream_t st) {
 }
 
 
-// Host-side layout of one call: cluster sizes, processing order (largest first) and the
-// callers' times (the device integrates in local time from 0).
+// Host-side layout of one call: cluster sizes, processing order (largest first; the small clusters
+// with given steps off the grid last) and the callers' times (the device integrates in local time
+// from 0).
 struct HardPlan {
     std::vector<int32_t> sizes, order;
+    std::vector<char> off_grid;
     std::vector<double> tc;
-    int n = 0, n_cluster = 0;
+    int n = 0, n_cluster = 0, n_off_grid = 0;
 };
 
 int check_args(const gplum_params *p, const gplum_particle *pp, int n, const int32_t *offsets, int n_cluster) {
@@ -110,6 +113,18 @@ int hard_upload(HardCtx &c, const gplum_params *p, const gplum_particle *pp, int
         pl.order[k] = k;
     }
     std::stable_sort(pl.order.begin(), pl.order.end(), [&](int a, int b) { return pl.sizes[a] > pl.sizes[b]; });
+    // (prepared steps are the device's own and on the grid)
+    pl.off_grid.assign(n_cluster, 0);
+    pl.n_off_grid = 0;
+    if (!prepare) {
+        for (int k = 0; k < n_cluster; k++) {
+            if (pl.sizes[k] > TERMS_MAX) continue;
+            for (int i = offsets[k]; i < offsets[k + 1]; i++) pl.off_grid[k] |= hard_off_grid(*p, pp[i].dt);
+            pl.n_off_grid += pl.off_grid[k];
+        }
+        if (pl.n_off_grid > 0)
+            std::stable_partition(pl.order.begin(), pl.order.end(), [&](int k) { return !pl.off_grid[k]; });
+    }
     hb.max_size = max_size;
     GPLUM_ENSURE(c.aos, n);
     GPLUM_HIP(hipMemcpyAsync(c.aos.p, pp, sizeof(gplum_particle) * (size_t)n, hipMemcpyHostToDevice, c.st));
@@ -126,7 +141,7 @@ int hard_upload(HardCtx &c, const gplum_params *p, const gplum_particle *pp, int
     GPLUM_ENSURE(c.order, n_cluster);
     if ((rc = upload(c.off, offs, c.st))) return rc;
     if ((rc = upload(c.order, pl.order, c.st))) return rc;
-    GPLUM_ENSURE(hb.next, HERMITE_CLASSES);
+    GPLUM_ENSURE(hb.next, HERMITE_QUEUES);
     GPLUM_ENSURE(hb.edisp, n_cluster);
     GPLUM_ENSURE(hb.ncol, n_cluster);
     GPLUM_ENSURE(hb.nblock, n_cluster);
@@ -216,11 +231,11 @@ extern "C" int gplum_hard_integrate(const gplum_params *p, gplum_particle *pp, i
         const int giant_min = (mode & 4) ? HARD_SEQ_MAX : GIANT_MIN_DEFAULT;
         const int terms_max = (mode & 8) ? 0 : TERMS_MAX;
         if ((rc = hard_launch(*p, c.hb, n_cluster, c.off.p, c.order.p, true, c.n_cu, c.st, c.hs, 8,
-                              HERMITE_LDS, giant_min, terms_max)))
+                              HERMITE_LDS, giant_min, terms_max, pl.n_off_grid)))
             return rc;
     } else {
         for (int k = 0; k < n_cluster; k++)
-            if ((rc = hard_launch_single(*p, c.hb, k, pl.sizes[k], c.off.p, c.st))) return rc;
+            if ((rc = hard_launch_single(*p, c.hb, k, pl.sizes[k], c.off.p, c.st, pl.off_grid[k] != 0))) return rc;
     }
     GPLUM_HIP(hipEventRecord(c.e1, c.st));
     GPLUM_HIP(hipStreamSynchronize(c.st));
@@ -271,7 +286,7 @@ extern "C" int gplum_hard_integrate_graph(const gplum_params *p, gplum_particle 
     // (the whole-GPU path for giant clusters is host-driven and cannot be captured)
     if (!rc)
         rc = hard_launch(*p, hb, n_cluster, c.off.p, c.order.p, true, c.n_cu, c.st, c.hs, 8,
-                         HERMITE_LDS, GIANT_OFF);
+                         HERMITE_LDS, GIANT_OFF, TERMS_MAX, pl.n_off_grid);
     const hipError_t ec = hipStreamEndCapture(c.st, &graph);
     if (rc) { if (graph) (void)hipGraphDestroy(graph); return rc; }
     GPLUM_HIP(ec);

@@ -1264,6 +1264,7 @@ __device__ inline bool dyadic_steps(const HP &P, double time, double dt) {
 static bool dyadic_tree(const gplum_params &p) {
     return is_pow2(p.dt_tree) && is_pow2(p.dt_min) && p.dt_min <= 0.5 * p.dt_tree && p.dt_min >= 0x1p-50 * p.dt_tree;
 }
+bool hard_off_grid(const gplum_params &p, double dt) { return dyadic_tree(p) && !(is_pow2(dt) && dt >= p.dt_min); }
 
 // The end of integrate_terms and integrate_pair: the final calcGravity with potentials
 // (hermite.h:466-470), one lane per particle.  vec: the lane holds component c of particle p's
@@ -1594,7 +1595,8 @@ __device__ __forceinline__ void cluster_queue(const HP &P, const ClusterArgs &A,
 // per term (a collision hands over to the LDS path in the middle of the soft step), the
 // others on the LDS path.  The arguments are read from LDS: in scalar registers they would
 // be spilled and reloaded in the block-step loop.  DYADIC: dyadic_tree's parameters, as in
-// every ordinary run; a cluster whose own steps are not powers of two then takes the LDS path.
+// every ordinary run; a cluster whose own steps are not powers of two then takes the LDS path
+// (hard_launch gives those that its caller lists to the other instantiation).
 template <bool DYADIC>
 __global__ __launch_bounds__(HERMITE_BLOCK) void k_hermite_small(HP P_arg, HardView H_arg, ClusterArgs A_arg, int lo,
                                                                  int hi) {
@@ -2297,18 +2299,18 @@ static void launch_class(int cls, bool dyadic, const HP &P, const HardView &H, c
 // zeroes the cluster-queue counters (a kernel, not a memset, so that the launch
 // sequence can be captured into a graph and replayed)
 __global__ void k_reset_queue(int *next) {
-    if (threadIdx.x < HERMITE_CLASSES) next[threadIdx.x] = 0;
+    if (threadIdx.x < HERMITE_QUEUES) next[threadIdx.x] = 0;
 }
 
 int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *d_off,
                 const int32_t *d_order, bool persistent, int n_cu, hipStream_t st, HardStreams &hs,
-                int wg_per_cu, int lds_max, int giant_min, int terms_max) {
+                int wg_per_cu, int lds_max, int giant_min, int terms_max, int n_off_grid) {
     if (ncl <= 0) return GPLUM_OK;
     HP P = make_hp(p);
     P.terms_max = std::max(0, std::min(TERMS_MAX, terms_max));
-    const bool dyadic = dyadic_tree(p);
+    const bool dyadic = dyadic_tree(p) && n_off_grid < ncl;   // every cluster off the grid: on st itself
     HardView H = hard_view(hb);
-    GPLUM_ENSURE(hb.next, HERMITE_CLASSES);
+    GPLUM_ENSURE(hb.next, HERMITE_QUEUES);
     GPLUM_ENSURE(hb.edisp, ncl);
     GPLUM_ENSURE(hb.ncol, ncl);
     GPLUM_ENSURE(hb.nblock, ncl);
@@ -2317,7 +2319,8 @@ int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *
     lds_max = std::min(HERMITE_LDS, std::max(HARD_SEQ_MAX, lds_max));
     const int grid = persistent ? std::min(ncl, std::max(1, n_cu) * std::max(1, wg_per_cu)) : ncl;
     const bool big = hb.max_size > HERMITE_SMALL;
-    if (big) {
+    if (!dyadic) n_off_grid = 0;
+    if (big || n_off_grid > 0) {
         int rc = hs.ensure();
         if (rc) return rc;
         GPLUM_HIP(hipEventRecord(hs.fork, st));
@@ -2337,10 +2340,23 @@ int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *
         const int lo = class_lo(cls, lds_max), hi = std::min(class_hi(cls, lds_max), giant_min);
         if (cls > 0 && (hb.max_size <= lo || hi <= lo)) continue;
         A.next = hb.next.p + cls;
+        A.ncl = (cls == 0) ? ncl - n_off_grid : ncl;
+        if (A.ncl <= 0) continue;
         if (cls > 0) GPLUM_HIP(hipStreamWaitEvent(hs.s[cls - 1], hs.fork, 0));
         launch_class(cls, dyadic, P, H, A, grid, lo, hi, cls > 0 ? hs.s[cls - 1] : st);
         if (cls > 0) GPLUM_HIP(hipEventRecord(hs.join[cls - 1], hs.s[cls - 1]));
         launched[cls] = true;
+    }
+    if (n_off_grid > 0) {
+        // on a stream and a queue of their own, beside the other clusters
+        hipStream_t so = hs.s[HERMITE_CLASSES - 1];
+        ClusterArgs O = A;
+        O.order = d_order + (ncl - n_off_grid);
+        O.ncl = n_off_grid;
+        O.next = hb.next.p + HERMITE_CLASSES;
+        GPLUM_HIP(hipStreamWaitEvent(so, hs.fork, 0));
+        launch_class(0, false, P, H, O, std::min(grid, n_off_grid), 0, HERMITE_SMALL, so);
+        GPLUM_HIP(hipEventRecord(hs.join[HERMITE_CLASSES - 1], so));
     }
     if (hb.max_size > giant_min) {
         // giant clusters: several at a time over the whole GPU on a stream pool (the
@@ -2359,6 +2375,7 @@ int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *
     }
     for (int cls = 1; cls < HERMITE_CLASSES; cls++)
         if (launched[cls]) GPLUM_HIP(hipStreamWaitEvent(st, hs.join[cls - 1], 0));
+    if (n_off_grid > 0) GPLUM_HIP(hipStreamWaitEvent(st, hs.join[HERMITE_CLASSES - 1], 0));
     GPLUM_HIP(hipGetLastError());
     return GPLUM_OK;
 }
@@ -2393,14 +2410,14 @@ int hard_prepare(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t 
 }
 
 int hard_launch_single(const gplum_params &p, HardBuffers &hb, int c, int n_c, const int32_t *d_off,
-                       hipStream_t st) {
+                       hipStream_t st, bool off_grid) {
     // one launch integrating cluster c (n_c particles) only: the per-cluster-launch comparator
     HP P = make_hp(p);
     HardView H = hard_view(hb);
     const ClusterArgs A{d_off + c, nullptr, 1, 0, hb.next.p, hb.edisp.p + c, hb.ncol.p + c, hb.nblock.p + c, hb.npair.p + c};
     int cls = 0;
     while (n_c > class_hi(cls, HERMITE_LDS)) cls++;
-    launch_class(cls, dyadic_tree(p), P, H, A, 1, 0, 0x7fffffff, st);
+    launch_class(cls, dyadic_tree(p) && !off_grid, P, H, A, 1, 0, 0x7fffffff, st);
     GPLUM_HIP(hipGetLastError());
     return GPLUM_OK;
 }

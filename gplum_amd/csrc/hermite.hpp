@@ -12,6 +12,7 @@ constexpr int HERMITE_MID = 32;        // members of the largest cluster of the 
 constexpr int HERMITE_BIG_BLOCK = 512;
 constexpr int HERMITE_GLOBAL_BLOCK = 512;
 constexpr int HERMITE_CLASSES = 5;     // size classes of a batched launch
+constexpr int HERMITE_QUEUES = HERMITE_CLASSES + 1;   // and the small clusters off the step grid
 constexpr int HERMITE_LDS = 256;       // clusters up to this size are integrated in LDS
 // Clusters up to HARD_SEQ_MAX particles sum each particle's hard force sequentially in
 // j (one lane per particle); larger ones with 64 lane-strided partial sums and a
@@ -57,11 +58,11 @@ struct HardBuffers {
     }
 };
 
-// Streams of the size classes above the one-wave kernel, so that the classes' longest chains
-// run side by side: fork after the gather on the caller's stream, which waits for the joins.
+// Streams of the size classes above the one-wave kernel and (the last) of the small clusters off
+// the step grid, so that the longest chains of all run side by side: fork after the gather on the caller's stream, which waits for the joins.
 struct HardStreams {
-    hipStream_t s[HERMITE_CLASSES - 1] = {};
-    hipEvent_t fork = nullptr, join[HERMITE_CLASSES - 1] = {};
+    hipStream_t s[HERMITE_QUEUES - 1] = {};
+    hipEvent_t fork = nullptr, join[HERMITE_QUEUES - 1] = {};
     HardStreams() = default;
     HardStreams(const HardStreams &) = delete;
     HardStreams &operator=(const HardStreams &) = delete;
@@ -97,18 +98,27 @@ struct IsoArgs {
 // integrated in LDS (larger ones on the global-memory state); clusters above giant_min run
 // over the whole GPU, several at a time on a stream pool, host-driven (not capturable in
 // a graph).  terms_max: clusters of 2 .. terms_max bodies take the lane-per-term path
-// (0: every cluster up to HERMITE_SMALL takes the LDS path).  None of these changes results.
+// (0: every cluster up to HERMITE_SMALL takes the LDS path).  n_off_grid: the last n_off_grid
+// clusters of d_order have at most TERMS_MAX members, some of them hard_off_grid: they take the
+// instantiation for any step (one cluster of 2 to 4 bodies 2.8 to 3.2 us per block step, launch
+// included; in the other one such a cluster takes the LDS path, 5.9 to 6.2 us).  None of these
+// changes results.
 constexpr int GIANT_MIN_DEFAULT = 1024;
 constexpr int GIANT_OFF = 0x7fffffff;
 int hard_launch(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *d_off,
                 const int32_t *d_order, bool persistent, int n_cu, hipStream_t st, HardStreams &hs, int wg_per_cu = 8,
-                int lds_max = HERMITE_LDS, int giant_min = GIANT_MIN_DEFAULT, int terms_max = TERMS_MAX);
+                int lds_max = HERMITE_LDS, int giant_min = GIANT_MIN_DEFAULT, int terms_max = TERMS_MAX,
+                int n_off_grid = 0);
+// Whether a member's given step is off the grid that dt_tree and dt_min make (powers of two; false
+// where these are none).  The library's own steps are never off it.
+bool hard_off_grid(const gplum_params &p, double dt);
 // Sun + hard acc/jerk and the initial block step of every cluster particle (as the
 // initial force correction leaves them), for callers that bring bare clusters.
 int hard_prepare(const gplum_params &p, HardBuffers &hb, int ncl, const int32_t *d_off, hipStream_t st);
-// One launch for cluster c (n_c particles) only (the per-cluster-launch comparator).
+// One launch for cluster c (n_c particles) only (the per-cluster-launch comparator); off_grid: it
+// has a member that is hard_off_grid.
 int hard_launch_single(const gplum_params &p, HardBuffers &hb, int c, int n_c, const int32_t *d_off,
-                       hipStream_t st);
+                       hipStream_t st, bool off_grid = false);
 // Isolated particles (number == 0): Kepler drift or Sun-only Hermite.
 int isolated_launch(const gplum_params &p, const IsoArgs &a, int n, double t0, double t1,
                     hipStream_t st);
