@@ -582,8 +582,12 @@ __global__ void k_flag01(int n, const int32_t *__restrict__ flag, int32_t *__res
 // dependent loads.  The same nodes in the same order, and node_moments in the same order of
 // operations, so the results are the same bits.  A step's whole tree part (sort to walk), level
 // kernels -> here, us: 300 particles 190 -> 112, 1000 222 -> 130, 3000 251 -> 164, 5000 271 -> 200,
-// 8192 289 -> 240 (linear in the particles: beyond, the level kernels' 256 workgroups win).
+// 8192 289 -> 240 (linear in the particles: beyond, the level kernels' 256 workgroups win).  Small
+// leaves make more nodes, and the line lies lower (small_tree_max): leaves of 1, us, 4096 particles
+// 336 -> 319, 5000 351 -> 365, 8192 358 -> 501; of 2, 5000 305 -> 290, 6144 309 -> 321; of 3, 7000 309 -> 303,
+// 8192 313 -> 337; of 4, 8192 295 -> 291.
 constexpr int TREE_SMALL = 8192;
+static int small_tree_max(int n_leaf) { return (int)std::min<long long>(TREE_SMALL, 3584 + 1024ll * std::max(1, n_leaf)); }
 constexpr int SMALL_BLOCK = 1024;
 
 struct SmallTree {
@@ -984,7 +988,7 @@ int tree_build_nodes(Tree &t, const gplum_params &p, const double *d_pos, const 
     GPLUM_ENSURE(t.lvl, LVL_ERR + 5);
     t.n_part = n;
     t.n_group = -1;
-    if (n > 0 && n <= TREE_SMALL && n < t.coop_min) {   // a coop_min below n asks for the level kernels
+    if (n > 0 && n <= small_tree_max(p.n_leaf_limit) && n < t.coop_min) {   // a coop_min below n asks for the level kernels
         t.L_end = MAXLEVEL + 1;              // whole: nothing is left for the walk to finish
         const SmallTree q{t.key.p, d_pos, d_mass, d_rsearch, t.lvl.p, t.node_start.p, t.node_count.p, t.node_level.p,
                           t.node_parent.p, t.node_child.p, t.node_nchild.p, t.node_mass.p, t.node_com.p, t.node_quad.p,

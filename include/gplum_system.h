@@ -156,7 +156,8 @@ typedef struct gplum_tuning {
     int32_t tree_coop_min;   /* tree nodes of at least this many particles split with a
                                 workgroup-wide search (not tuned; 0 = 65536); a value
                                 up to the particle number also keeps trees of up to 8192
-                                particles on the level kernels (same results)         */
+                                particles (fewer with n_leaf_limit below 5) on the
+                                level kernels (same results)                          */
     int32_t hard_terms_max;  /* clusters of 2 .. this many (<= 4) bodies spread a block
                                 step over one lane per particle, term and component;
                                 0: the larger clusters' path (not tuned; same results) */
