@@ -324,3 +324,12 @@ extern "C" int gplum_hermite_dt_selfcheck(const gplum_params *p, int64_t n, uint
     if (fallbacks) *fallbacks = f;
     return rc;
 }
+
+extern "C" int gplum_hermite_path_selfcheck(const gplum_params *p, int64_t n, uint64_t seed, gplum_path_selfcheck *out) {
+    if (!p || !out) return gplum::fail(GPLUM_E_ARG, "null argument");
+    int64_t c[9] = {};
+    const int rc = gplum::hermite_path_selfcheck(*p, (long long)n, seed, c);
+    if (rc) return rc;
+    *out = gplum_path_selfcheck{c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], c[8]};
+    return GPLUM_OK;
+}

@@ -13,6 +13,7 @@
 // steps times size) from an atomic queue until it is empty.
 #include <algorithm>
 #include <cfloat>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -51,7 +52,7 @@ constexpr double COL_FILTER = 1.0 + 1e-10;
 // Newton steps the correctly rounded reciprocal (Markstein, IBM J. Res. Dev. 34, 1990).  The
 // library's sqrt takes the same corrections after scaling, its division starts over from the
 // estimate of 1 / b; in range there is nothing to scale, and a wave with a value out of range
-// calls the library.  gplum_hermite_dt_selfcheck compares the results with sqrt and 1 / x bit for
+// calls the library.  gplum_hermite_path_selfcheck compares the results with sqrt and 1 / x bit for
 // bit.  sqrt and division in sequence took 92 + 70 cycles of latency (dependent FP64
 // operations 7 cycles, the estimate 18); here 18 + 14 operations.
 
@@ -2449,53 +2450,161 @@ __device__ inline double rnd_mag(uint64_t &st, int e0, int e1) {
     return ((r >> 10) & 1) ? -ldexp(m, e) : ldexp(m, e);
 }
 
-// dt_block with the fast criterion against dt_block with calc_dt4 on random states:
-// accelerations and their derivatives over many decades, steps dt_tree 2^-k and times on
-// the step's grid.  One sample in four widens every magnitude by 2^+-540, so that the
-// products of squares in the fast criterion underflow below DBL_MIN or overflow past
-// DBL_MAX.  Counts results that differ in any bit and fast values sent to the exact
-// evaluation; the pairs of roots and reciprocals are compared as well.
+// A random state: accelerations and their derivatives over many decades (wide: every magnitude
+// spread by another 2^+-wide), a step dt_tree 2^-kk, kk <= k_max, and a time on the step's grid.
+struct DtSample {
+    double v[8][3], acc0, dt, time;      // v: acc, jerk, snap, crackle of the planets, of the Sun
+};
+__device__ inline void dt_sample(const HP &P, uint64_t &st, int wide, int k_max, DtSample &s) {
+    const int e_lo[8] = {-20, -24, -28, -32, -12, -16, -20, -24};
+    const int e_hi[8] = {8, 14, 20, 26, 4, 8, 12, 16};
+    for (int q = 0; q < 8; q++)
+        for (int k = 0; k < 3; k++) s.v[q][k] = rnd_mag(st, e_lo[q] - wide, e_hi[q] + wide);
+    s.acc0 = fabs(rnd_mag(st, -12, 4));
+    st += 0x9E3779B97F4A7C15ULL;
+    const uint64_t r = mix64(st);
+    const int kk = 1 + (int)(r % (uint64_t)k_max);
+    s.dt = ldexp(P.dt_tree, -kk);
+    s.time = s.dt * (double)((r >> 8) % (1ULL << kk));
+}
+template <bool FAST>
+__device__ inline double dt_of(const HP &P, const DtSample &s, int *fell = nullptr) {
+    return dt_block<FAST>(P, s.time + s.dt, s.dt, s.acc0, s.v[0], s.v[1], s.v[2], s.v[3], s.v[4], s.v[5], s.v[6], s.v[7], fell);
+}
+
+// dt_block with the fast criterion against dt_block with calc_dt4 on random states.  One sample
+// in four is spread by 2^+-540, so that the products of squares in the fast criterion underflow
+// below DBL_MIN or overflow past DBL_MAX.  Counts results that differ in any bit and fast values
+// sent to the exact evaluation.
 __global__ void k_dt_selfcheck(HP P, long long n, uint64_t seed, unsigned long long *out) {
     unsigned long long mism = 0, fb = 0;
     for (long long s = blockIdx.x * (long long)blockDim.x + threadIdx.x; s < n; s += (long long)gridDim.x * blockDim.x) {
         uint64_t st = seed ^ mix64((uint64_t)s * 0x2545F4914F6CDD1DULL);
-        double v[8][3];
-        const int e_lo[8] = {-20, -24, -28, -32, -12, -16, -20, -24};
-        const int e_hi[8] = {8, 14, 20, 26, 4, 8, 12, 16};
-        const int wide = ((s & 3) == 3) ? 540 : 0;
-        for (int q = 0; q < 8; q++)
-            for (int k = 0; k < 3; k++) v[q][k] = rnd_mag(st, e_lo[q] - wide, e_hi[q] + wide);
-        const double acc0 = fabs(rnd_mag(st, -12, 4));
-        st += 0x9E3779B97F4A7C15ULL;
-        const uint64_t r = mix64(st);
-        const int kk = 1 + (int)(r % 30);                       // dt = dt_tree 2^-kk
-        const double dt = ldexp(P.dt_tree, -kk);
-        const double time = dt * (double)((r >> 8) % (1ULL << kk));   // on the grid of dt
+        DtSample d;
+        dt_sample(P, st, ((s & 3) == 3) ? 540 : 0, 30, d);
         int fell = 0;
-        const double a = dt_block<true>(P, time + dt, dt, acc0, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], &fell);
-        const double b = dt_block<false>(P, time + dt, dt, acc0, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]);
+        const double a = dt_of<true>(P, d, &fell), b = dt_of<false>(P, d);
         mism += (__double_as_longlong(a) != __double_as_longlong(b)) ? 1 : 0;
         fb += fell;
-        // the roots and reciprocals of the force terms: random mantissas, and those next to a
-        // power of two or to a square, where a rounding is closest
-        st += 0x9E3779B97F4A7C15ULL;
-        const uint64_t u = mix64(st);
-        double x = fabs(rnd_mag(st, -420, 420));
-        const uint64_t ulps = u >> 58;
-        if ((u & 3) == 1) x = ldexp(1.0, (int)(u >> 8 & 511) - 256) * (1.0 + ((u & 4) ? 1. : -0.5) * 0x1p-52 * (double)ulps);
-        if ((u & 3) == 2) {
-            const double q = fabs(rnd_mag(st, -200, 200));
-            x = __longlong_as_double(__double_as_longlong(q * q) + (long long)ulps - 32);
-        }
-        double rt, rtinv, sinv, root;
-        root_and_inverse(x, true, rt, rtinv);
-        inverse_and_root(x, sinv, root);
-        const double r0 = sqrt(x), s0 = 1. / x;
-        mism += (__double_as_longlong(rt) != __double_as_longlong(r0)) + (__double_as_longlong(rtinv) != __double_as_longlong(1. / r0)) +
-                (__double_as_longlong(sinv) != __double_as_longlong(s0)) + (__double_as_longlong(root) != __double_as_longlong(sqrt(s0)));
     }
     atomicAdd(&out[0], mism);
     atomicAdd(&out[1], fb);
+}
+
+// The helpers of the lane-per-term and LDS paths, which act on a whole wave, one wave per sample:
+//   roots      8 values per lane through root_and_inverse and inverse_and_root against sqrt and 1 / x.
+//              One lane that a helper has to send to the library takes its whole wave there, so such
+//              values (out of range; a low word of ones) come in one wave of eight each and the others
+//              hold none: random mantissas, those next to a power of two or to a square, where a
+//              rounding is closest.  Counts the values whose wave kept to the estimate.
+//   steps      dt_block_rows of 2, 3 and 4 bodies (the sample number picks) on both kinds of grid and
+//              dt_block_quad, a state per particle in the lanes of its quads, against dt_block with
+//              calc_dt4.  Of eight samples one is wide (see dt_sample), three have derivatives scaled to
+//              dt_1 = dt 2^k (1 + d), |d| from 2^-8 to 2^-51 or 0, around the 2^-10 margin and the grid
+//              itself, and one has dt 3/4 of a power of two (not through the dyadic rule).
+enum { CHK_ROOTS, CHK_ROOTS_FAST, CHK_ROOTS_BAD, CHK_STEPS, CHK_STEPS_NEAR, CHK_ROWS_BAD, CHK_DYADIC, CHK_DYADIC_BAD, CHK_QUAD_BAD,
+       CHK_N };
+__device__ inline bool bits_differ(double a, double b) { return __double_as_longlong(a) != __double_as_longlong(b); }
+
+template <int N>
+__device__ inline void check_rows(const HP &P, bool dyadic_p, int k_max, long long q, uint64_t seed, int mode,
+                                  unsigned long long cnt[CHK_N]) {
+    const int L = (int)threadIdx.x;
+    const int T = (N == 2) ? ((L >> 4) & 1) : (L >> 4), p = (N == 2) ? ((L >> 2) & 1) : ((L >> 2) & 3), c = L & 3;
+    const bool sun = T == 0, pad = c == 3;
+    uint64_t st = seed ^ mix64((uint64_t)(q * 4 + p) * 0x2545F4914F6CDD1DULL);
+    DtSample d;
+    dt_sample(P, st, mode == 3 ? 540 : 0, k_max, d);
+    const bool off_grid = mode == 2, near = mode >= 5;
+    if (off_grid) {
+        d.dt *= 0.75;
+        d.time = 0.75 * d.time;
+    }
+    if (near) {
+        const double dt_1 = dmin(calc_dt4(P.eta, P.alpha2, d.acc0, d.v[0], d.v[1], d.v[2], d.v[3]),
+                                 calc_dt4(P.eta_sun, P.alpha2, 0., d.v[4], d.v[5], d.v[6], d.v[7]));
+        st += 0x9E3779B97F4A7C15ULL;
+        const uint64_t r = mix64(st);
+        const int e = 8 + (int)((r >> 4) % 45);
+        const double delta = (e == 52) ? 0. : ((r & 1) ? 1. : -1.) * ldexp(1., -e);
+        const double lam = dt_1 / (ldexp(d.dt, (int)((r >> 1) & 3) - 2) * (1. + delta));
+        for (int k = 0; k < 3; k++)
+            for (int b = 0; b < 8; b += 4) {
+                d.v[b + 1][k] *= lam;
+                d.v[b + 2][k] *= lam * lam;
+                d.v[b + 3][k] *= lam * lam * lam;
+            }
+    }
+    const double want = dt_of<false>(P, d);
+    double z[8];
+    for (int b = 0; b < 8; b++) z[b] = pad ? 0. : (c == 0 ? d.v[b][0] : c == 1 ? d.v[b][1] : d.v[b][2]);
+    const TermConsts C(P);
+    const double za = sun ? z[4] : z[0], zj = sun ? z[5] : z[1], zs = sun ? z[6] : z[2], zc = sun ? z[7] : z[3];
+    const double eta = sun ? P.eta_sun : P.eta, acc0 = sun ? 0. : d.acc0;
+    cnt[CHK_STEPS]++;
+    cnt[CHK_STEPS_NEAR] += near;
+    cnt[CHK_ROWS_BAD] += bits_differ(dt_block_rows<N, false>(C, d.time + d.dt, d.dt, eta, acc0, za, zj, zs, zc), want);
+    if (dyadic_p && !off_grid) {
+        cnt[CHK_DYADIC]++;
+        cnt[CHK_DYADIC_BAD] += bits_differ(dt_block_rows<N, true>(C, d.time + d.dt, d.dt, eta, acc0, za, zj, zs, zc), want);
+    }
+    cnt[CHK_QUAD_BAD] += bits_differ(dt_block_quad(P, d.time + d.dt, d.dt, d.acc0, z[0], z[1], z[2], z[3], z[4], z[5], z[6], z[7]),
+                                     want);
+}
+
+__global__ __launch_bounds__(64) void k_path_selfcheck(HP P, bool dyadic_p, int k_max, long long n, uint64_t seed,
+                                                       unsigned long long *out) {
+    unsigned long long cnt[CHK_N] = {};
+    for (long long q = blockIdx.x; q < n; q += gridDim.x) {
+        const int mode = (int)(q & 7);
+        uint64_t st = ~seed ^ mix64((uint64_t)(q * 64 + (int)threadIdx.x) * 0x2545F4914F6CDD1DULL);
+        for (int v = 0; v < 8; v++) {
+            double x = fabs(rnd_mag(st, -398, 398));
+            st += 0x9E3779B97F4A7C15ULL;
+            // (just below a power of two, value or root have a low word of ones)
+            const uint64_t u = mix64(st), ulps = (u >> 58) + ((mode < 6 && !(u & 4)) ? 4 : 0);
+            if ((u & 3) == 1) x = ldexp(1.0, (int)(u >> 8 & 511) - 256) * (1.0 + ((u & 4) ? 1. : -0.5) * 0x1p-52 * (double)ulps);
+            if ((u & 3) == 2) {
+                const double w = fabs(rnd_mag(st, -198, 198));
+                x = __longlong_as_double(__double_as_longlong(w * w) + (long long)ulps - 32);
+            }
+            if (mode == 6 && (u & 48) == 0) x = __longlong_as_double(__double_as_longlong(x) | 0xFFFFFFFFll);
+            if (mode == 7 && (u & 48) == 0) x = fabs(rnd_mag(st, -1000, 1000));
+            double rt, rtinv, sinv, root;
+            root_and_inverse(x, true, rt, rtinv);
+            inverse_and_root(x, sinv, root);
+            const double r0 = sqrt(x), s0 = 1. / x;
+            const bool library = __ballot(!root_range(x) || rcp_exception(x) || rcp_exception(r0)) != 0;
+            cnt[CHK_ROOTS]++;
+            cnt[CHK_ROOTS_FAST] += !library;
+            cnt[CHK_ROOTS_BAD] += bits_differ(rt, r0) || bits_differ(rtinv, 1. / r0) || bits_differ(sinv, s0) ||
+                                  bits_differ(root, sqrt(s0));
+        }
+        const int bodies = 2 + (int)((q >> 3) % 3);
+        if (bodies == 2) check_rows<2>(P, dyadic_p, k_max, q, seed, mode, cnt);
+        else if (bodies == 3) check_rows<3>(P, dyadic_p, k_max, q, seed, mode, cnt);
+        else check_rows<4>(P, dyadic_p, k_max, q, seed, mode, cnt);
+    }
+    for (int k = 0; k < CHK_N; k++)
+        if (cnt[k]) atomicAdd(&out[k], cnt[k]);
+}
+
+int hermite_path_selfcheck(const gplum_params &p, long long n, uint64_t seed, int64_t counts[CHK_N]) {
+    if (n < 0) return fail(GPLUM_E_ARG, "negative sample count");
+    if (!(p.dt_tree > 0.) || !(p.dt_min > 0.) || p.dt_min > 0.25 * p.dt_tree)
+        return fail(GPLUM_E_ARG, "dt_min must lie in (0, dt_tree / 4]");
+    DArray<unsigned long long> cnt;
+    GPLUM_ENSURE(cnt, CHK_N);
+    GPLUM_HIP(hipMemset(cnt.p, 0, CHK_N * sizeof(unsigned long long)));
+    // no sample's step lies below dt_min, as the dyadic rule asks
+    int k_max = 1;
+    while (k_max < 30 && std::ldexp(p.dt_tree, -(k_max + 1)) >= p.dt_min) k_max++;
+    hipLaunchKernelGGL(k_path_selfcheck, dim3(1024), dim3(64), 0, 0, make_hp(p), dyadic_tree(p), k_max, n, seed, cnt.p);
+    GPLUM_HIP(hipGetLastError());
+    unsigned long long h[CHK_N] = {};
+    GPLUM_HIP(hipMemcpy(h, cnt.p, sizeof(h), hipMemcpyDeviceToHost));
+    for (int k = 0; k < CHK_N; k++) counts[k] = (int64_t)h[k];
+    return GPLUM_OK;
 }
 
 int hermite_dt_selfcheck(const gplum_params &p, long long n, uint64_t seed, long long *mismatches,

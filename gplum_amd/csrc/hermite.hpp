@@ -126,5 +126,8 @@ int isolated_launch(const gplum_params &p, const IsoArgs &a, int n, double t0, d
 // dt_block's fast criterion against the correctly rounded one on n random states.
 int hermite_dt_selfcheck(const gplum_params &p, long long n, uint64_t seed, long long *mismatches,
                          long long *fallbacks);
+// The roots, reciprocals and step rules of the clusters' kernels on n random wave samples (counts:
+// the fields of gplum_path_selfcheck in order).
+int hermite_path_selfcheck(const gplum_params &p, long long n, uint64_t seed, int64_t counts[9]);
 
 }  // namespace gplum

@@ -134,6 +134,19 @@ def hermite_dt_selfcheck(p, n, seed=1):
     return m.value, f.value
 
 
+class PathSelfcheck(ctypes.Structure):
+    """gplum_path_selfcheck (include/gplum_system.h)."""
+    _fields_ = [(n, ctypes.c_int64) for n in ("roots", "roots_fast", "roots_bad", "steps", "steps_near", "steps_rows_bad",
+                                              "steps_dyadic", "steps_dyadic_bad", "steps_quad_bad")]
+
+
+def hermite_path_selfcheck(p, n, seed=1):
+    """gplum_hermite_path_selfcheck: the counts as a dict."""
+    out = PathSelfcheck()
+    check(lib().gplum_hermite_path_selfcheck(ctypes.byref(p), ctypes.c_int64(n), ctypes.c_uint64(seed), ctypes.byref(out)))
+    return {k: getattr(out, k) for k, _ in out._fields_}
+
+
 class SnapshotHeader(ctypes.Structure):
     """gplum_snapshot_header (include/gplum_system.h)."""
     _fields_ = [("time", ctypes.c_double), ("n_body", ctypes.c_int32), ("id_next", ctypes.c_int32),

@@ -290,6 +290,22 @@ int gplum_hard_integrate_graph(const gplum_params *p, gplum_particle *pp, int n,
 int gplum_hermite_dt_selfcheck(const gplum_params *p, int64_t n, uint64_t seed, int64_t *mismatches,
                                int64_t *fallbacks);
 
+/* The same for the clusters of up to 256 members, whose kernels act on a wave at a time: n wave
+ * samples of 512 values through the square roots and reciprocals of a force term, compared
+ * with the correctly rounded ones, and of 2 to 4 particles through the step rules, compared
+ * with FPHard::calcDeltat; random, next to the roundings and step grids where the fast forms
+ * could err, and beyond their range.  Counts per lane; every *_bad is 0.  dt_min <=
+ * dt_tree / 4.  steps_dyadic is 0 unless dt_tree and dt_min are powers of two. */
+typedef struct gplum_path_selfcheck {
+    int64_t roots, roots_fast;      /* values; those whose wave did not need the library's functions */
+    int64_t roots_bad;              /* values with a result that differs in any bit                  */
+    int64_t steps, steps_near;      /* steps; those with a criterion within 2^-8 of the step grid    */
+    int64_t steps_rows_bad;         /* 2 to 4 bodies, steps of any kind                              */
+    int64_t steps_dyadic, steps_dyadic_bad;   /* 2 to 4 bodies, steps that are powers of two         */
+    int64_t steps_quad_bad;         /* larger clusters                                               */
+} gplum_path_selfcheck;
+int gplum_hermite_path_selfcheck(const gplum_params *p, int64_t n, uint64_t seed, gplum_path_selfcheck *out);
+
 #ifdef __cplusplus
 }
 #endif
