@@ -364,7 +364,6 @@ __device__ inline void st3(double *a, int i, const double v[3]) {
 struct JData {
     const double *x, *v, *m, *ri;
     const int64_t *id;
-    int stride;            // 3 for interleaved global arrays
 };
 
 // pairs evaluated side by side per lane (independent dependency chains; the one wave
@@ -417,48 +416,38 @@ __device__ inline void gravity_loop(const HP &P, const JData &J, int n, int64_t 
     pair_sum_strided(P, J, 0, 1, n, idi, xi, vi, rinv_i, acc, jerk, phi);
 }
 
-// gravity_loop for the one-particle-per-lane path of lane i: the lane's partners are
-// j = k + (k >= i) for k = 0 .. n-2, ascending j as in gravity_loop, so every lane runs
-// the same n-1 iterations (the loop over all j with a self test would run n iterations
-// with one lane masked off in each).  A partner with the same id (never, before any
-// merger) is evaluated and not added, as gravity_loop skips it; CHECK = false leaves
-// the test out, for clusters whose ids are known to be distinct.
-template <bool CHECK = true>
-__device__ inline void gravity_loop_lane(const HP &P, const JData &J, int n, int i, int64_t idi,
-                                         const double xi[3], const double vi[3], double rinv_i,
-                                         double acc[3], double jerk[3], double *phi) {
+// gravity_loop with one lane per particle, for clusters whose ids are known to be distinct: lane
+// i's partners are j = k + (k >= i) for k = 0 .. n-2, ascending j as in gravity_loop, so every
+// lane runs the same n-1 iterations (the loop over all j with a self test would run n iterations
+// with one lane masked off in each).
+__device__ inline void gravity_loop_lane(const HP &P, const JData &J, int n, int i, const double xi[3], const double vi[3],
+                                         double rinv_i, double acc[3], double jerk[3], double *phi) {
     acc[0] = acc[1] = acc[2] = 0.;
     jerk[0] = jerk[1] = jerk[2] = 0.;
     const int m = n - 1;
     int k = 0;
     for (; k + HARD_ILP <= m; k += HARD_ILP) {
         double ta[HARD_ILP][3], tj[HARD_ILP][3], tp[HARD_ILP];
-        int jj[HARD_ILP];
+#pragma unroll
+        for (int u = 0; u < HARD_ILP; u++)
+            pair_term_j(P, J, k + u + ((k + u) >= i ? 1 : 0), xi, vi, rinv_i, ta[u], tj[u], phi ? &tp[u] : nullptr);
 #pragma unroll
         for (int u = 0; u < HARD_ILP; u++) {
-            jj[u] = k + u + ((k + u) >= i ? 1 : 0);
-            pair_term_j(P, J, jj[u], xi, vi, rinv_i, ta[u], tj[u], phi ? &tp[u] : nullptr);
-        }
-#pragma unroll
-        for (int u = 0; u < HARD_ILP; u++) {
-            const bool use = !CHECK || J.id[jj[u]] != idi;
             for (int d = 0; d < 3; d++) {
-                acc[d] = use ? acc[d] + ta[u][d] : acc[d];
-                jerk[d] = use ? jerk[d] + tj[u][d] : jerk[d];
+                acc[d] += ta[u][d];
+                jerk[d] += tj[u][d];
             }
-            if (phi) *phi = use ? *phi - tp[u] : *phi;
+            if (phi) *phi -= tp[u];
         }
     }
     for (; k < m; k++) {
-        const int j = k + (k >= i ? 1 : 0);
         double ta[3], tj[3], tp;
-        pair_term_j(P, J, j, xi, vi, rinv_i, ta, tj, phi ? &tp : nullptr);
-        const bool use = !CHECK || J.id[j] != idi;
+        pair_term_j(P, J, k + (k >= i ? 1 : 0), xi, vi, rinv_i, ta, tj, phi ? &tp : nullptr);
         for (int d = 0; d < 3; d++) {
-            acc[d] = use ? acc[d] + ta[d] : acc[d];
-            jerk[d] = use ? jerk[d] + tj[d] : jerk[d];
+            acc[d] += ta[d];
+            jerk[d] += tj[d];
         }
-        if (phi) *phi = use ? *phi - tp : *phi;
+        if (phi) *phi -= tp;
     }
 }
 
@@ -468,7 +457,7 @@ __device__ void gravity_full(const HP &P, HardView &H, int b, int n, int i) {
     ld3(H.pos, b + i, x);
     ld3(H.vel, b + i, v);
     star_acc_jerk(P, x, v, as, js, &phs);
-    const JData Jc{H.pos + 3 * b, H.vel + 3 * b, H.mass + b, H.rinv + b, H.id + b, 3};
+    const JData Jc{H.pos + 3 * b, H.vel + 3 * b, H.mass + b, H.rinv + b, H.id + b};
     gravity_loop(P, Jc, n, H.id[b + i], x, v, H.rinv[b + i], ad, jd, &phd);
     st3(H.acc_s, b + i, as);
     st3(H.jerk_s, b + i, js);
@@ -554,7 +543,7 @@ __device__ inline double readlane_f64(double v, int lane) {
 __device__ inline void coop_pair_sum(const HP &P, const JData &J, int n, int64_t idi, const double xi[3],
                                      const double vi[3], double rinv_i, double acc[3], double jerk[3]) {
     double a[3] = {0., 0., 0.}, jk[3] = {0., 0., 0.};
-    // two pairs at a time: the multi-wave kernels hold more state per lane
+    // two pairs at a time: the callers hold much state per lane
     pair_sum_strided<2>(P, J, (int)(threadIdx.x & 63), 64, n, idi, xi, vi, rinv_i, a, jk, nullptr);
     // butterfly x += x[lane ^ d] for d = 32, 16, 8, 4, 2, 1 (every lane active): the two
     // levels across rows of 16 lanes by shuffles, the four inside a row by DPP moves
@@ -745,10 +734,10 @@ __device__ inline void wave_sync() {
 // force together (coop_pair_sum); every lane carries the same particle state in
 // registers and lane 0 writes it back.  Active particles only read the predicted
 // j-data, so the waves need not wait for each other.  Twins of a merged target are
-// integrated alongside with their own cut-off radius, as in the per-lane path.  tw: the
-// cluster's twin_of (cluster-local indices; an LDS copy where the kernel keeps one).
+// integrated alongside with their own cut-off radius.
 __device__ void coop_correct_active(const HP &P, HardView &H, const JData &J, int b, int n, double t_s,
-                                    int flag_col, long long &pairs, int wave, int n_wave, const int32_t *tw) {
+                                    int flag_col, long long &pairs, int wave, int n_wave) {
+    const int32_t *tw = H.twin_of + b;     // cluster-local indices
     const int lane = (int)(threadIdx.x & 63);
     const bool lead = lane == 0;
     int rank = 0;                          // active particles seen so far (wave-uniform)
@@ -848,7 +837,7 @@ __device__ void coop_correct_active(const HP &P, HardView &H, const JData &J, in
     }
 }
 
-// ------------------------------------- multi-wave kernel: workgroup-level reductions
+// ------------------------------------- global-memory path: workgroup-level reductions
 
 // One slot per wave for each reduction (separate slots, so that a reduction needs no
 // barrier before its writes).
@@ -976,7 +965,7 @@ __device__ void integrate_global(const HP &P, HardView &H, const JData &J, int b
                            (flag_col || H.time[b + i] + H.dt[b + i] == t_s);
         __threadfence_block();
         __syncthreads();
-        coop_correct_active(P, H, J, b, n, t_s, flag_col, pairs, (int)(threadIdx.x >> 6), B >> 6, H.twin_of + b);
+        coop_correct_active(P, H, J, b, n, t_s, flag_col, pairs, (int)(threadIdx.x >> 6), B >> 6);
         __threadfence_block();
         __syncthreads();
         if (flag_col) {
@@ -1014,7 +1003,7 @@ __device__ void integrate_global(const HP &P, HardView &H, const JData &J, int b
 // cross-row lane swaps (v_permlane16/32_swap, no LDS) and adds them as star_acc_jerk
 // and gravity_loop_lane do (the Sun row; the partner rows in ascending j from zero), and
 // the Sun and planet time-step criteria likewise.  Same operations in the same order
-// as the one-lane-per-particle path.
+// as the reference's loops.
 
 constexpr int DPP_ROW_ROR4 = 0x124;
 
@@ -1272,7 +1261,7 @@ bool hard_off_grid(const gplum_params &p, double dt) { return dyadic_tree(p) && 
 // x and v; lead: its time and dt.
 template <int N>
 __device__ inline void terms_finish(const HP &P, HardView &H, const JData &J, double *s_x, double *s_v, const double *s_ri,
-                                    const int64_t *s_id, double *s_tm, int b, int p, int c, bool vec, bool lead, double x,
+                                    double *s_tm, int b, int p, int c, bool vec, bool lead, double x,
                                     double v, double time, double dt, long long &pairs) {
     const int L = threadIdx.x;
     __syncthreads();
@@ -1291,7 +1280,7 @@ __device__ inline void terms_finish(const HP &P, HardView &H, const JData &J, do
         ld3(s_x, L, xi);
         ld3(s_v, L, vi);
         star_acc_jerk(P, xi, vi, fas, fjs, &phs);
-        gravity_loop_lane<false>(P, J, N, L, s_id[L], xi, vi, s_ri[L], fad, fjd, &phd);
+        gravity_loop_lane(P, J, N, L, xi, vi, s_ri[L], fad, fjd, &phd);
         pairs += N - 1;
         st3(H.pos, gi, xi); st3(H.vel, gi, vi);
         st3(H.acc_s, gi, fas); st3(H.jerk_s, gi, fjs);
@@ -1310,11 +1299,11 @@ __device__ inline void terms_finish(const HP &P, HardView &H, const JData &J, do
 // soft step (the layout above; one wave; DYADIC: all of them keep to dyadic_steps).  Returns
 // false when a block step may have a collision: the state of the start of that block step is
 // then in H (flags and twins cleared) for integrate_seq.  Else the final calcGravity with
-// potentials is done and written to H.  s_m, s_ri, s_id, s_fr hold the cluster's masses, 1/r_out,
-// ids and f r_planet; s_x, s_v and s_tm are free.
+// potentials is done and written to H.  s_m, s_ri, s_fr hold the cluster's masses, 1/r_out
+// and f r_planet; s_x, s_v and s_tm are free.
 template <int N, bool DYADIC>
 __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double *s_x, double *s_v, double *s_m,
-                                double *s_ri, int64_t *s_id, double *s_fr, double *s_tm, int b, double &sys_time,
+                                double *s_ri, double *s_fr, double *s_tm, int b, double &sys_time,
                                 long long &loop, long long &pairs) {
     constexpr int m = N - 1;
     const int L = threadIdx.x;
@@ -1423,7 +1412,7 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
         }
         return false;
     }
-    terms_finish<N>(P, H, J, s_x, s_v, s_ri, s_id, s_tm, b, p, c, row && sun && !pad, lead, x, v, time, dt, pairs);
+    terms_finish<N>(P, H, J, s_x, s_v, s_ri, s_tm, b, p, c, row && sun && !pad, lead, x, v, time, dt, pairs);
     return true;
 }
 
@@ -1435,7 +1424,7 @@ __device__ bool integrate_terms(const HP &P, HardView &H, const JData &J, double
 // terms: 2 bodies 1.06 us per block step in a 100k disk).
 template <bool DYADIC>
 __device__ bool integrate_pair(const HP &P, HardView &H, const JData &J, double *s_x, double *s_v, double *s_m,
-                               double *s_ri, int64_t *s_id, double *s_fr, double *s_tm, int b, double &sys_time,
+                               double *s_ri, double *s_fr, double *s_tm, int b, double &sys_time,
                                long long &loop, long long &pairs) {
     const int L = threadIdx.x;
     const int T = (L >> 4) & 1, p = (L >> 2) & 1, c = L & 3;
@@ -1541,7 +1530,7 @@ __device__ bool integrate_pair(const HP &P, HardView &H, const JData &J, double 
         }
         return false;
     }
-    terms_finish<2>(P, H, J, s_x, s_v, s_ri, s_id, s_tm, b, p, c, sun && !pad && first, lead, x, v, time, dt, pairs);
+    terms_finish<2>(P, H, J, s_x, s_v, s_ri, s_tm, b, p, c, sun && !pad && first, lead, x, v, time, dt, pairs);
     return true;
 }
 
@@ -1633,13 +1622,13 @@ __global__ __launch_bounds__(HERMITE_BLOCK) void k_hermite_small(HP P_arg, HardV
                 for (int j = 0; j < n; j++) other = other || (j != t && C.id[j] == C.id[t]);
             }
             if (__ballot(other) == 0) {
-                const JData J{C.xp, C.vp, C.mass, C.rinv, C.id, 3};
+                const JData J{C.xp, C.vp, C.mass, C.rinv, C.id};
                 double *tm = reinterpret_cast<double *>(s_term);
                 auto terms = [&](auto N) {
-                    return integrate_terms<N.value, DYADIC>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b, sys_time,
+                    return integrate_terms<N.value, DYADIC>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.fr, tm, b, sys_time,
                                                             loop, pairs);
                 };
-                const bool done = (n == 2) ? integrate_pair<DYADIC>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.id, C.fr, tm, b,
+                const bool done = (n == 2) ? integrate_pair<DYADIC>(P, H, J, C.xp, C.vp, C.mass, C.rinv, C.fr, tm, b,
                                                                     sys_time, loop, pairs)
                                   : (n == 3) ? terms(std::integral_constant<int, 3>())
                                              : terms(std::integral_constant<int, 4>());
@@ -1705,7 +1694,7 @@ __global__ __launch_bounds__(HERMITE_GLOBAL_BLOCK) __attribute__((amdgpu_waves_p
     const int t = threadIdx.x;
     cluster_queue(P, A, lo, hi, [&](int b, int n, double &sys_time, long long &loop, double &ed, int &n_col,
                                     long long &pairs) {
-        const JData J{H.xp + 3 * b, H.vp + 3 * b, H.mass + b, H.rinv + b, H.id + b, 3};
+        const JData J{H.xp + 3 * b, H.vp + 3 * b, H.mass + b, H.rinv + b, H.id + b};
         // initial calcGravity for all, flags cleared (hermite.h:259-270)
         for (int i = t; i < n; i += HERMITE_GLOBAL_BLOCK) {
             gravity_full(P, H, b, n, i);
@@ -1891,7 +1880,7 @@ static HardView hard_view(HardBuffers &hb) {
 // with OpenMP inside the cluster, hard.h:583-658) are spread over the whole GPU: each
 // block step is a short sequence of kernels (predict all; collision test over all pairs
 // with per-workgroup minima; decision and active flags; the active particles, one wave
-// each, as in the multi-wave kernels; the collision aftermath phase by phase; next
+// each, as on the global-memory path; the collision aftermath phase by phase; next
 // block time and system time), launched in batches by the host, which checks a done
 // flag between batches.  Same functions, same summation orders: results identical to the size-class
 // kernels.
@@ -2058,11 +2047,11 @@ __global__ __launch_bounds__(GIANT_RED) void k_g_decide(HP P, HardView H, int b,
 // the active members, one wave each (coop_correct_active over the whole grid)
 __global__ __launch_bounds__(GIANT_T) void k_g_correct(HP P, HardView H, int b, int n, GiantState *G) {
     if (G->done) return;
-    const JData J{H.xp + 3 * b, H.vp + 3 * b, H.mass + b, H.rinv + b, H.id + b, 3};
+    const JData J{H.xp + 3 * b, H.vp + 3 * b, H.mass + b, H.rinv + b, H.id + b};
     long long pairs = 0;
     const int waves = (int)(blockDim.x >> 6);
     coop_correct_active(P, H, J, b, n, G->t_s, G->flag_col, pairs, (int)blockIdx.x * waves + (int)(threadIdx.x >> 6),
-                        (int)gridDim.x * waves, H.twin_of + b);
+                        (int)gridDim.x * waves);
     if ((threadIdx.x & 63) == 0 && pairs) atomicAdd((unsigned long long *)&G->pairs, (unsigned long long)pairs);
 }
 

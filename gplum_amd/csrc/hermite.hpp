@@ -14,9 +14,9 @@ constexpr int HERMITE_GLOBAL_BLOCK = 512;
 constexpr int HERMITE_CLASSES = 5;     // size classes of a batched launch
 constexpr int HERMITE_QUEUES = HERMITE_CLASSES + 1;   // and the small clusters off the step grid
 constexpr int HERMITE_LDS = 256;       // clusters up to this size are integrated in LDS
-// Clusters up to HARD_SEQ_MAX particles sum each particle's hard force sequentially in
-// j (one lane per particle); larger ones with 64 lane-strided partial sums and a
-// butterfly (all lanes on one particle), an order the oracle reproduces.
+// Clusters up to HARD_SEQ_MAX particles sum each particle's hard force sequentially in j; larger
+// ones with 64 lane-strided partial sums and a butterfly (a wave on one particle), an order the
+// oracle reproduces.
 constexpr int HARD_SEQ_MAX = 64;
 // Clusters of 2 .. TERMS_MAX bodies spread each block step over one lane per particle,
 // term (Sun or partner) and component (4 n^2 <= 64 lanes).

@@ -166,7 +166,7 @@ __device__ inline void lds_relations(ClusterLds<NMAX> &C, int n) {
 // Sun and hard acc/jerk of every member at its current state, one thread each
 template <int NMAX, int T>
 __device__ inline void lds_gravity_all(const HP &P, ClusterLds<NMAX> &C, int n, long long &pairs) {
-    const JData J{C.pos, C.vel, C.mass, C.rinv, C.id, 3};
+    const JData J{C.pos, C.vel, C.mass, C.rinv, C.id};
     for (int i = (int)threadIdx.x; i < n; i += T) {
         double x[3], v[3], as[3], js[3], ad[3], jd[3];
         ld3(C.pos, i, x);
@@ -606,7 +606,7 @@ __device__ void integrate_tree(const HP &P, ClusterLds<NMAX> &C, TreeLds<NMAX> &
             if (first && !flag_col && P.collision) {
                 if (lds_any_close(C, n, my_j, my_r, cb, rounds)) C.hit = 1;
             }
-            const JData J{C.xp, C.vp, C.mass, C.rinv, C.id, 3};
+            const JData J{C.xp, C.vp, C.mass, C.rinv, C.id};
             for (int s = w; s < nb; s += W) {
                 const int bd = C.body[s];
                 const double *px = first ? C.xp + 3 * bd : C.bx + 3 * s;
@@ -761,7 +761,7 @@ __device__ __forceinline__ void run_cluster_lds(const HP &P, HardView &H, Cluste
     V.f = C.f; V.id = C.id; V.flags = C.flags; V.twin_of = C.twin_of;
     V.base = b;
     integrate(V);
-    const JData J{C.pos, C.vel, C.mass, C.rinv, C.id, 3};
+    const JData J{C.pos, C.vel, C.mass, C.rinv, C.id};
     for (int i = t; i < n; i += T) {
         double x[3], v[3], as[3], js[3], ad[3], jd[3], phs = 0., phd = 0.;
         ld3(C.pos, i, x);

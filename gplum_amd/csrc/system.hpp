@@ -85,7 +85,7 @@ struct System {
     // launch shapes picked by autotune() (defaults until it runs)
     int soft_tile = SOFT_TILE;          // j-particles staged per LDS pass of the soft kernel
     int hard_wg_per_cu = 8;             // persistent Hermite workgroups per CU
-    int hard_lds_max = HERMITE_LDS;     // largest cluster whose j-data is staged in LDS
+    int hard_lds_max = HERMITE_LDS;     // largest cluster integrated in LDS
     int hard_giant_min = GIANT_MIN_DEFAULT;   // larger clusters run over the whole GPU
     int hard_terms_max = TERMS_MAX;     // clusters of 2 .. this many bodies: lane per term
     bool tuning = false;                // inside autotune(): no training, no statistics

@@ -92,8 +92,8 @@ def hard_integrate(p, pp, offsets, persistent=True, prepare=False, counts=False,
     """Integrate clusters pp[offsets[c]:offsets[c+1]] over one soft step (in place).
     prepare: compute acc/jerk and the first block step on the device first.
     giant: every cluster above 64 particles on the whole-GPU path (same results).
-    lane_per_particle: clusters of 2 to 4 bodies on the one-lane-per-particle path instead
-    of the lane-per-term path (same results).
+    lane_per_particle: clusters of 2 to 4 bodies on the larger clusters' path in LDS instead
+    of one lane per particle, term and component (same results).
     Returns (edisp, block_steps, kernel_ms), plus pair evaluations when counts."""
     off = np.ascontiguousarray(offsets, dtype=np.int32)
     ed = ctypes.c_double(0.0)

@@ -101,8 +101,8 @@ def test_hermite_perfect_merging_matches_oracle(oracle_lib):
 
 def test_repeated_ids_match_oracle(oracle_lib):
     """A cluster member that repeats another member's id is skipped as a partner (the
-    oracle's same-id test); such clusters leave the register path for the global-memory
-    path, which keeps the test."""
+    oracle's same-id test); such clusters of 2 to 4 bodies leave the lane-per-term path for the
+    path in LDS, which keeps the test."""
     po, pg, pp, off = make_clusters(oracle_lib, 30, seed=17, size_max=40, collision=0)
     rep = 0
     for c in range(len(off) - 1):
@@ -138,7 +138,7 @@ def _same_state(a, b, fields=("pos", "vel", "acc_d", "jerk_d", "acc_s", "jerk_s"
 
 def test_graph_replay_matches_eager(no_collision_case):
     """The persistent launch captured into a hipGraph (state restore, queue reset by a
-    kernel, size-class kernels on two streams): every replay reproduces the first bit
+    kernel, each size class on a stream of its own): every replay reproduces the first bit
     for bit (checked inside the call with synchronisations between replays), and the
     first equals the eager launch."""
     pg, pp, off, ref, nb_ref = no_collision_case
@@ -168,7 +168,7 @@ def test_graph_replay_with_merging(oracle_lib):
 @pytest.mark.parametrize("planar", [False, True])
 def test_small_clusters_lane_per_term(oracle_lib, planar):
     """Clusters of 2 to 4 bodies (one lane per particle, term and component): bit-identical
-    to the oracle and to the one-lane-per-particle path; in the planar case z and v_z stay
+    to the oracle and to the larger clusters' path in LDS; in the planar case z and v_z stay
     exactly zero and the Sun's z-terms are -0, so the sign handling of the quad dot
     products shows in the compared bits."""
     po, pg, pp, off = make_clusters(oracle_lib, 300, seed=23, size_max=4, collision=0, planar=planar)
@@ -179,7 +179,7 @@ def test_small_clusters_lane_per_term(oracle_lib, planar):
     ed_g, nb_g, ms = gpu.hard_integrate(pg, got, off, persistent=True)
     lpp = pp.copy()
     ed_l, nb_l, ms_l = gpu.hard_integrate(pg, lpp, off, persistent=True, lane_per_particle=True)
-    print("planar %s: %d clusters, block steps %d (oracle %d), kernel %.2f ms (one lane per particle %.2f ms)"
+    print("planar %s: %d clusters, block steps %d (oracle %d), kernel %.2f ms (path in LDS %.2f ms)"
           % (planar, len(off) - 1, nb_g, nb_ref, ms, ms_l))
     assert nb_g == nb_ref == nb_l
     assert _same_state(got, ref, fields=("pos", "vel", "acc_d", "jerk_d", "acc_s", "jerk_s", "phi_s", "dt",
@@ -192,7 +192,7 @@ def test_small_clusters_lane_per_term(oracle_lib, planar):
 
 def test_small_clusters_lane_per_term_collisions(oracle_lib):
     """Clusters of 2 to 4 bodies with inflated radii: the block step of a collision hands
-    the cluster to the global-memory path; the same merges as the oracle."""
+    the cluster to the path in LDS; the same merges as the oracle."""
     po, pg, pp, off = make_clusters(oracle_lib, 200, seed=29, size_max=4, collision=1, f=300.0, m_hi=1e-8)
     ref = pp.copy()
     nc, ed, nb_ref = oracle_lib.hermite_clusters(po, ref, off)
