@@ -15,8 +15,11 @@
 // active particles.  Same operations in the same order as the reference's loops
 // (hermite.h:224-479), so the results are those of the other paths bit for bit.
 //
-// What bounds it: the latency of three pair terms (each a correctly rounded FP64 square
-// root and reciprocal), the sums over j and seven barriers per block step; the
+// What bounds it: the latency of three evaluations, one after the other: waves wait 56 to 72 % of
+// their cycles.  64 members, 3.4 bodies corrected, 18,000 cycles per block step: pair terms (each a
+// correctly rounded FP64 square root and reciprocal, and the loads before it) 2,600, 1,800 and 1,800,
+// sums over j with corrections, step choice and stores 3,100, 2,400 and 3,900, prediction, lists and
+// next time 2,300; 128 members, 22,000: evaluations 4,600, 4,300 and 4,300 with their sums.  The
 // chip's FP64 rate is far away (a cluster occupies one CU).  Measured on one cluster, us per
 // block step, against one lane per particle in registers and, from the first merger on, one
 // lane per particle in global memory (up to 64 members), or lane groups of 8 to 64 lanes (above):
