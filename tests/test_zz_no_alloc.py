@@ -1,8 +1,8 @@
 """The allocation-free EP-EP entry point (gplum_calc_force_epep_noalloc) against the
 allocating one (gplum_calc_force_epep) on the same inputs: bit-identical Force arrays on
-two calls in a row, the second with fewer i- and j-particles (the per-device chunk table
-keeps the first call's entries beyond the second's and must not be read), accumulation
-into a non-cleared Force array, and the size limit reported as an argument error.
+two calls in a row, the second with fewer i- and j-particles (nothing of the first call may
+be left for it), accumulation into a non-cleared Force array, and the size limit reported as an
+argument error.
 
 Device buffers for the calls come from the HIP runtime the library itself links
 (hipMalloc through ctypes in the test, not in the entry point)."""
